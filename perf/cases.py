@@ -28,6 +28,9 @@ _abi = grmp._abi
 # relative residual of the solves: the single-instance configurations' 1e-10,
 # the served stream's 1e-9, the Newton loop's inner 1e-12
 RTOL, RTOL_SERVED, RTOL_NEWTON = 1e-10, 1e-9, 1e-12
+# the Newton loop's own target: the residual's rounding floor is below 1e-9 over
+# these sizes and data, and the sixth step reaches it
+RESIDUAL_NEWTON = 5e-9
 
 
 def listed():
@@ -322,7 +325,7 @@ def run(st):
         return _fetch(st["X"].vec, st["out"])
     if kind == "newton":
         sol = grmp.FEVector(st["fes"])
-        grmp.solve(sol, st["pde"], target_residual=1e-10, nonlinear_maxiterations=12, rtol=RTOL_NEWTON)
+        grmp.solve(sol, st["pde"], target_residual=RESIDUAL_NEWTON, nonlinear_maxiterations=12, rtol=RTOL_NEWTON)
         return sol.entries()
     srv = st["server"]
     tickets = [srv.submit(k, fe, n, s, rtol=RTOL_SERVED, out=v) for (k, fe, n, s), v in zip(st["reqs"], st["views"])]
