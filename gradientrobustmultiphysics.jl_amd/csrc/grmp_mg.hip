@@ -151,8 +151,21 @@ struct MgRows {
     double *part;        // block partials (OP_PCG_Q: p.q; OP_CHEB_POST2 at level 0: r.z)
 };
 
+// d0 = D^-1 b / theta, the first step of the pre-smoothing from x0 = 0.  The
+// kernel that produces a level's right-hand side (the restriction, the CG
+// update, the true residual, the preconditioner's input) writes d0 beside it,
+// 16 bytes a row, so that the pre-smoothing product gathers one array per
+// nonzero.  Forming d0 inside the product gathered b, D^-1 and the mask per
+// nonzero: 59 us on 4.2M P1 rows against 45 us with d0 stored (the
+// producers take 16 bytes a row more).
+__device__ __forceinline__ double cheb_first(bool fx, double dinv, double b, double lam)
+{
+    return fx ? 0.0 : dinv * b * CHEB_ITHETA(lam);
+}
+
 // 256 rows per block through the LDS-staged row product, then the epilogue:
 //   RESID   o1 = b - A v
+//   TRUE_RESID  the same, and o2 = d0 of the residual
 //   PRE     v = d0:  o1 = (1 + C1) d0 + C2 D^-1 (b - A d0)
 //   POST1   v = x:   d = D^-1 (b - A x) / theta -> o1,  x + d -> o2
 //   POST2   v = x1:  o1 = x1 + C1 d + C2 D^-1 (b - A x1)   [+ partials of b . o1]
@@ -164,8 +177,12 @@ __device__ __forceinline__ double mg_epilogue(int64_t i, double s, bool fx, cons
                                               const double *__restrict__ d, const double *__restrict__ lam,
                                               double *__restrict__ o1, double *__restrict__ o2)
 {
-    if (OP == OP_RESID || OP == OP_TRUE_RESID) {
+    if (OP == OP_RESID) {
         o1[i] = fx ? 0.0 : b[i] - s;
+    } else if (OP == OP_TRUE_RESID) {
+        const double r = fx ? 0.0 : b[i] - s;
+        o1[i] = r;
+        o2[i] = cheb_first(fx, dinv[i], r, *lam);
     } else if (OP == OP_CHEB_PRE) {
         const double l = *lam;
         o1[i] = fx ? 0.0 : (1.0 + CHEB_C1) * v[i] + CHEB_C2(l) * dinv[i] * (b[i] - s);
@@ -207,47 +224,6 @@ __device__ __forceinline__ void mg_rows_body(const MgRows &a, int64_t r0, int pi
         block_sum2(pa, pb);
         if (threadIdx.x == 0) a.part[pidx] = pa;
     }
-}
-
-// Chebyshev pre-smoothing from x0 = 0 in one pass: d0 = D^-1 b / theta is
-// formed on the fly in the staged row product (the same products as a stored
-// d0), then o1 = (1 + C1) d0 + C2 D^-1 (b - A d0).
-__device__ __forceinline__ void mg_pre_body(const MgRows &a, int64_t r0)
-{
-    __shared__ double lds[MG_ROWS_CAP];
-    const double l = *a.lam, ith = CHEB_ITHETA(l);
-    const int64_t r1 = r0 + KB < a.n ? r0 + KB : a.n;
-    const int t = threadIdx.x;
-    const int64_t r = r0 + t;
-    const int32_t base = a.rp[r0], end = a.rp[r1];
-    int32_t my0 = 0, my1 = 0;
-    if (r < r1) {
-        my0 = a.rp[r];
-        my1 = a.rp[r + 1];
-    }
-    double s = 0.0;
-    for (int32_t c0 = base; c0 < end; c0 += MG_ROWS_CAP) {
-        const int32_t c1 = c0 + MG_ROWS_CAP < end ? c0 + MG_ROWS_CAP : end;
-        __syncthreads();
-        for (int32_t k = c0 + t; k < c1; k += KB) {
-            const int32_t c = a.ci[k];
-            lds[k - c0] = (double)a.val32[k] * (a.fixed[c] ? 0.0 : a.dinv[c] * a.b[c] * ith);
-        }
-        __syncthreads();
-        const int32_t lo = my0 > c0 ? my0 : c0, hi = my1 < c1 ? my1 : c1;
-        for (int32_t k = lo; k < hi; ++k) s += lds[k - c0];
-    }
-    if (r < r1) {
-        const bool fx = a.fixed[r] != 0;
-        const double d0 = fx ? 0.0 : a.dinv[r] * a.b[r] * ith;
-        a.o1[r] = fx ? 0.0 : (1.0 + CHEB_C1) * d0 + CHEB_C2(l) * a.dinv[r] * (a.b[r] - s);
-    }
-}
-
-__global__ __launch_bounds__(KB) void k_mg_pre(MgRows a)
-{
-    if (a.sc->done) return;
-    mg_pre_body(a, (int64_t)blockIdx.x * KB);
 }
 
 template <int OP>
@@ -353,7 +329,7 @@ __device__ __forceinline__ void prolong_p1_one(int64_t Nf64, int64_t Nc64, int n
     xf[t] += s;
 }
 
-// bc = P^T rf on free coarse dofs, 0 on fixed ones; t < nnc * ncomp.  Fine
+// the value of P^T rf at coarse dof t < nnc * ncomp, 0 on fixed ones.  Fine
 // node (i, j) has weight Nf - max(|a|, |b|) for a b >= 0 and
 // max(Nf - |a| - |b|, 0) otherwise, a = i Nc - I Nf and b = j Nc - J Nf being
 // its offsets from coarse node (I, J) in units of 1 / (Nf Nc): p1_weight's
@@ -362,16 +338,12 @@ __device__ __forceinline__ void prolong_p1_one(int64_t Nf64, int64_t Nc64, int n
 // once.  Walking the index box node by node instead (a division and a
 // dependent load per step) made this a serial chain of memory latencies:
 // 10.2 us per launch whatever the size, against 3.4 us.
-__device__ __forceinline__ void restrict_p1_one(int64_t Nf64, int64_t Nc64, int ncomp, const double *__restrict__ rf,
-                                                const uint8_t *__restrict__ fixed_c, double *__restrict__ bc,
-                                                int64_t t)
+__device__ __forceinline__ double restrict_p1_one(int64_t Nf64, int64_t Nc64, const double *__restrict__ rf,
+                                                  const uint8_t *__restrict__ fixed_c, int64_t t)
 {
     const int Nf = (int)Nf64, Nc = (int)Nc64;
     const int64_t nnf = (int64_t)(Nf + 1) * (Nf + 1), nnc = (int64_t)(Nc + 1) * (Nc + 1);
-    if (fixed_c[t]) {
-        bc[t] = 0.0;
-        return;
-    }
+    if (fixed_c[t]) return 0.0;
     int64_t node64 = t;
     const int k = p1_split(nnc, node64);
     const uint32_t node = (uint32_t)node64;
@@ -401,7 +373,7 @@ __device__ __forceinline__ void restrict_p1_one(int64_t Nf64, int64_t Nc64, int 
 #pragma unroll
         for (int p = 0; p < 4; ++p)
             if (w[q][p] != 0) s += (double)w[q][p] * inv * v[q][p];
-    bc[t] = s;
+    return s;
 }
 
 // P1 -> P2 on the same N-square, added into x2: node dofs copy (t < nn),
@@ -428,14 +400,11 @@ __device__ __forceinline__ void prolong_p2_one(int64_t N, const int32_t *__restr
 // its transpose (v < nn): node v gathers r2[v] and half of each incident
 // face's entry (left / right horizontal, lower / upper vertical, lower-left /
 // upper-right diagonal)
-__device__ __forceinline__ void restrict_p2_one(int64_t N, const double *__restrict__ r2,
-                                                const uint8_t *__restrict__ fixed1, double *__restrict__ b1, int64_t v)
+__device__ __forceinline__ double restrict_p2_one(int64_t N, const double *__restrict__ r2,
+                                                  const uint8_t *__restrict__ fixed1, int64_t v)
 {
     const int64_t nn = (N + 1) * (N + 1);
-    if (fixed1[v]) {
-        b1[v] = 0.0;
-        return;
-    }
+    if (fixed1[v]) return 0.0;
     const int64_t i = v % (N + 1), j = v / (N + 1);
     const double *rf = r2 + nn;
     double s = 0.0;
@@ -445,7 +414,7 @@ __device__ __forceinline__ void restrict_p2_one(int64_t N, const double *__restr
     if (j < N) s += rf[sq_V(N, i, j)];
     if (i > 0 && j > 0) s += rf[sq_D(N, i - 1, j - 1)];
     if (i < N && j < N) s += rf[sq_D(N, i, j)];
-    b1[v] = r2[v] + 0.5 * s;
+    return r2[v] + 0.5 * s;
 }
 
 __global__ void k_mg_prolong_p1(int64_t Nf, int64_t Nc, int ncomp, const double *__restrict__ xc,
@@ -456,12 +425,18 @@ __global__ void k_mg_prolong_p1(int64_t Nf, int64_t Nc, int ncomp, const double 
     if (t < (Nf + 1) * (Nf + 1) * ncomp) prolong_p1_one(Nf, Nc, ncomp, xc, fixed_f, xf, t);
 }
 
+// b_c = P^T r_f and, for the coarse level's smoothing, d_c = d0 of b_c
 __global__ void k_mg_restrict_p1(int64_t Nf, int64_t Nc, int ncomp, const double *__restrict__ rf,
-                                 const uint8_t *__restrict__ fixed_c, double *__restrict__ bc, const MgScal *sc)
+                                 const uint8_t *__restrict__ fixed_c, const double *__restrict__ dinv_c,
+                                 const double *__restrict__ lam_c, double *__restrict__ bc, double *__restrict__ dc,
+                                 const MgScal *sc)
 {
     if (sc->done) return;
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < (Nc + 1) * (Nc + 1) * ncomp) restrict_p1_one(Nf, Nc, ncomp, rf, fixed_c, bc, t);
+    if (t >= (Nc + 1) * (Nc + 1) * ncomp) return;
+    const double b = restrict_p1_one(Nf, Nc, rf, fixed_c, t);
+    bc[t] = b;
+    dc[t] = cheb_first(fixed_c[t] != 0, dinv_c[t], b, *lam_c);
 }
 
 __global__ void k_mg_prolong_p2(int64_t N, const int32_t *__restrict__ cells, const int8_t *__restrict__ fsign,
@@ -474,11 +449,15 @@ __global__ void k_mg_prolong_p2(int64_t N, const int32_t *__restrict__ cells, co
 }
 
 __global__ void k_mg_restrict_p2(int64_t N, const double *__restrict__ r2, const uint8_t *__restrict__ fixed1,
-                                 double *__restrict__ b1, const MgScal *sc)
+                                 const double *__restrict__ dinv1, const double *__restrict__ lam1,
+                                 double *__restrict__ b1, double *__restrict__ d1, const MgScal *sc)
 {
     if (sc->done) return;
     const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (v < (N + 1) * (N + 1)) restrict_p2_one(N, r2, fixed1, b1, v);
+    if (v >= (N + 1) * (N + 1)) return;
+    const double b = restrict_p2_one(N, r2, fixed1, v);
+    b1[v] = b;
+    d1[v] = cheb_first(fixed1[v] != 0, dinv1[v], b, *lam1);
 }
 
 // coarse coefficient: geometric mean of the fine cells whose centroid lies in
@@ -585,22 +564,38 @@ __global__ void k_mg_dot(const double *__restrict__ a, const double *__restrict_
     if (threadIdx.x == 0) part[blockIdx.x] = pa;
 }
 
-// x += alpha p, r -= alpha q; partials of r.r
+// x += alpha p, r -= alpha q; partials of r.r; d = d0 of the new r
 __global__ void k_mg_axpy(double *__restrict__ x, double *__restrict__ r, const double *__restrict__ p,
-                          const double *__restrict__ q, int64_t n, double *part, const MgScal *sc)
+                          const double *__restrict__ q, const uint8_t *__restrict__ fixed,
+                          const double *__restrict__ dinv, const double *__restrict__ lam, double *__restrict__ d,
+                          int64_t n, double *part, const MgScal *sc)
 {
     if (sc->done) return;
-    const double al = sc->alpha;
+    const double al = sc->alpha, l = *lam;
     const int64_t i = (int64_t)blockIdx.x * KB + threadIdx.x;
     double pa = 0.0, pb = 0.0;
     if (i < n) {
         x[i] += al * p[i];
         const double ri = r[i] - al * q[i];
         r[i] = ri;
+        d[i] = cheb_first(fixed[i] != 0, dinv[i], ri, l);
         pa = ri * ri;
     }
     block_sum2(pa, pb);
     if (threadIdx.x == 0) part[blockIdx.x] = pa;
+}
+
+// r = rhs on the free rows, 0 on the fixed ones; d = d0 of it
+__global__ void k_mg_start(const double *__restrict__ rhs, const uint8_t *__restrict__ fixed,
+                           const double *__restrict__ dinv, const double *__restrict__ lam, double *__restrict__ r,
+                           double *__restrict__ d, int64_t n)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const bool fx = fixed[i] != 0;
+    const double ri = fx ? 0.0 : rhs[i];
+    r[i] = ri;
+    d[i] = cheb_first(fx, dinv[i], ri, *lam);
 }
 
 __global__ void k_mg_update_p(double *__restrict__ p, const double *__restrict__ z, int64_t n, const MgScal *sc)
@@ -702,15 +697,15 @@ __device__ double blk_vcycle(const MgBDesc &D)
     for (int l = D.first; l < L1; ++l) {
         const MgBLevel &L = D.lv[l], &C = D.lv[l + 1];
         for (int64_t i = threadIdx.x; i < L.n; i += MG_BT)
-            L.d[i] = L.fixed[i] ? 0.0 : L.dinv[i] * L.b[i] * CHEB_ITHETA(*L.lam);
+            L.d[i] = cheb_first(L.fixed[i] != 0, L.dinv[i], L.b[i], *L.lam);
         __syncthreads();
         blk_rows<OP_CHEB_PRE>(L, L.d, L.b, nullptr, L.x, nullptr);
         __syncthreads();
         blk_rows<OP_RESID>(L, L.x, L.b, nullptr, L.r, nullptr);
         __syncthreads();
         for (int64_t t = threadIdx.x; t < C.n; t += MG_BT) {
-            if (L.fe == GRMP_FE_H1P2) restrict_p2_one(L.N, L.r, C.fixed, C.b, t);
-            else restrict_p1_one(L.N, C.N, L.ncomp, L.r, C.fixed, C.b, t);
+            C.b[t] = L.fe == GRMP_FE_H1P2 ? restrict_p2_one(L.N, L.r, C.fixed, t)
+                                          : restrict_p1_one(L.N, C.N, L.r, C.fixed, t);
         }
         __syncthreads();
     }
@@ -773,7 +768,7 @@ __device__ void mg_pcg_block_body(const MgBDesc &D, MgScal *sc, int iters)
         __syncthreads();
         if (st == 1) return;
         if (st == 2) {  // the updated residual met rtol: check b - A x
-            blk_rows<OP_TRUE_RESID>(L0, D.x, D.rhs, nullptr, D.r, nullptr);
+            blk_rows<OP_TRUE_RESID>(L0, D.x, D.rhs, nullptr, D.r, L0.d);
             __syncthreads();
             double p = 0.0;
             for (int64_t i = threadIdx.x; i < n; i += MG_BT) p += D.r[i] * D.r[i];
@@ -902,23 +897,6 @@ __global__ __launch_bounds__(KB) void k_mgb_rows(const MgTile *__restrict__ T, c
     }
 }
 
-// d0 = D^-1 b / theta on the level's rows, the first step of the
-// pre-smoothing, stored for k_mgb_rows<OP_CHEB_PRE>.  Batched launches cost
-// little, so the separate pass (about a sixth of the product's bytes) beats
-// forming d0 inside the product, which gathers three arrays per nonzero.
-__global__ __launch_bounds__(KB) void k_mgb_first(const MgTile *__restrict__ T, const MgBDesc *const *__restrict__ Dp)
-{
-    const MgTile t = T[blockIdx.x];
-    const MgBDesc &D = *Dp[t.req];
-    if (D.sc->done) return;
-    const MgBLevel &L = D.lv[t.level];
-    const double ith = CHEB_ITHETA(*L.lam);
-    for (int c = 0; c < MG_TILE_CHUNKS; ++c) {
-        const int64_t i = t.row0 + (int64_t)c * KB + threadIdx.x;
-        if (i < L.n) L.d[i] = L.fixed[i] ? 0.0 : L.dinv[i] * L.b[i] * ith;
-    }
-}
-
 // tiles over the rows of coarse level t.level (> 0)
 __global__ __launch_bounds__(KB) void k_mgb_restrict(const MgTile *__restrict__ T,
                                                      const MgBDesc *const *__restrict__ Dp)
@@ -930,8 +908,10 @@ __global__ __launch_bounds__(KB) void k_mgb_restrict(const MgTile *__restrict__ 
     for (int c = 0; c < MG_TILE_CHUNKS; ++c) {
         const int64_t i = t.row0 + (int64_t)c * KB + threadIdx.x;
         if (i >= C.n) break;
-        if (F.fe == GRMP_FE_H1P2) restrict_p2_one(F.N, F.r, C.fixed, C.b, i);
-        else restrict_p1_one(F.N, C.N, F.ncomp, F.r, C.fixed, C.b, i);
+        const double b = F.fe == GRMP_FE_H1P2 ? restrict_p2_one(F.N, F.r, C.fixed, i)
+                                              : restrict_p1_one(F.N, C.N, F.r, C.fixed, i);
+        C.b[i] = b;
+        C.d[i] = cheb_first(C.fixed[i] != 0, C.dinv[i], b, *C.lam);
     }
 }
 
@@ -954,14 +934,15 @@ __global__ __launch_bounds__(KB) void k_mgb_prolong(const MgTile *__restrict__ T
     }
 }
 
-// level-0 tiles: x += alpha p, r -= alpha q, partials of r.r
+// level-0 tiles: x += alpha p, r -= alpha q, partials of r.r, d0 of the new r
 __global__ __launch_bounds__(KB) void k_mgb_axpy(const MgTile *__restrict__ T, const MgBDesc *const *__restrict__ Dp)
 {
     const MgTile t = T[blockIdx.x];
     const MgBDesc &D = *Dp[t.req];
     if (D.sc->done) return;
-    const double al = D.sc->alpha;
-    const int64_t n = D.lv[0].n;
+    const MgBLevel &L = D.lv[0];
+    const double al = D.sc->alpha, l = *L.lam;
+    const int64_t n = L.n;
     for (int c = 0; c < MG_TILE_CHUNKS; ++c) {
         const int64_t r0 = t.row0 + (int64_t)c * KB;
         if (r0 >= n) break;
@@ -971,6 +952,7 @@ __global__ __launch_bounds__(KB) void k_mgb_axpy(const MgTile *__restrict__ T, c
             D.x[i] += al * D.p[i];
             const double ri = D.r[i] - al * D.q[i];
             D.r[i] = ri;
+            L.d[i] = cheb_first(L.fixed[i] != 0, L.dinv[i], ri, l);
             pa = ri * ri;
         }
         block_sum2(pa, pb);
@@ -1287,10 +1269,10 @@ static void mg_restrict(MgJob *j, int l)
     const MgLevel &F = j->lv[l], &C = j->lv[l + 1];
     if (F.in.fe == GRMP_FE_H1P2)
         hipLaunchKernelGGL(k_mg_restrict_p2, dim3(nblk(C.n, 256)), dim3(256), 0, j->st, (int64_t)F.in.N, F.r,
-                           C.in.A->fixed, C.b, j->sc);
+                           C.in.A->fixed, C.dinv, C.lam, C.b, C.d, j->sc);
     else
         hipLaunchKernelGGL(k_mg_restrict_p1, dim3(nblk(C.n, 256)), dim3(256), 0, j->st, (int64_t)F.in.N,
-                           (int64_t)C.in.N, F.in.ncomp, F.r, C.in.A->fixed, C.b, j->sc);
+                           (int64_t)C.in.N, F.in.ncomp, F.r, C.in.A->fixed, C.dinv, C.lam, C.b, C.d, j->sc);
 }
 
 static void mg_prolong(MgJob *j, int l)
@@ -1307,7 +1289,7 @@ static void mg_prolong(MgJob *j, int l)
     }
 }
 
-// x_0 (= z) = V(b_0 (= r)); the level-0 block partials of r.z land in part.
+// x_0 (= z) = V(b_0 (= r)), d_0 holding d0 of r; the level-0 block partials of r.z land in part.
 // Levels below first_small run as grid kernels, the rest in one workgroup.
 static void mg_vcycle(MgJob *j)
 {
@@ -1316,9 +1298,10 @@ static void mg_vcycle(MgJob *j)
         MgLevel &L = j->lv[l];
         MgRows a;
         rows_args(a, L, j);
+        a.v = L.d;
         a.b = L.b;
         a.o1 = L.x;
-        hipLaunchKernelGGL(k_mg_pre, dim3(nblk(L.n, KB)), dim3(KB), 0, j->st, a);
+        launch_rows<OP_CHEB_PRE>(j, a);
         rows_args(a, L, j);
         a.v = L.x;
         a.b = L.b;
@@ -1385,8 +1368,8 @@ static int mg_job_start(MgJob *j, double rtol, int maxit)
     const int64_t n = j->lv[0].n;
     GRMP_HIP(ctx, hipMemsetAsync(j->x, 0, n * 8, st));
     GRMP_HIP(ctx, hipMemsetAsync(j->p, 0, n * 8, st));
-    GRMP_HIP(ctx, hipMemcpyAsync(j->r, j->rhs, n * 8, hipMemcpyDeviceToDevice, st));
-    GRMP_TRY(zero_fixed_launch(j->lv[0].in.A, j->r, st));
+    hipLaunchKernelGGL(k_mg_start, dim3(nblk(n, 256)), dim3(256), 0, st, j->rhs, j->lv[0].in.A->fixed, j->lv[0].dinv,
+                       j->lv[0].lam, j->r, j->lv[0].d, n);
     mg_vcycle(j);
     hipLaunchKernelGGL(k_mg_dot, dim3(j->nb0), dim3(KB), 0, st, j->r, j->r, n, j->part2, j->sc);
     hipLaunchKernelGGL(k_mg_red<RED_INIT>, dim3(1), dim3(KB), 0, st, j->part, j->nb0, j->part2, j->sc);
@@ -1490,7 +1473,8 @@ static int mg_iterate_grid(MgJob *j, int iters)
         a.part = j->part;
         launch_rows<OP_PCG_Q>(j, a);
         hipLaunchKernelGGL(k_mg_red<RED_ALPHA>, dim3(1), dim3(KB), 0, j->st, j->part, j->nb0, nullptr, j->sc);
-        hipLaunchKernelGGL(k_mg_axpy, dim3(j->nb0), dim3(KB), 0, j->st, j->x, j->r, j->p, j->q, n, j->part, j->sc);
+        hipLaunchKernelGGL(k_mg_axpy, dim3(j->nb0), dim3(KB), 0, j->st, j->x, j->r, j->p, j->q, L0.in.A->fixed,
+                           L0.dinv, L0.lam, L0.d, n, j->part, j->sc);
         hipLaunchKernelGGL(k_mg_red<RED_CONV>, dim3(1), dim3(KB), 0, j->st, j->part, j->nb0, nullptr, j->sc);
         mg_vcycle(j);
         hipLaunchKernelGGL(k_mg_red<RED_BETA>, dim3(1), dim3(KB), 0, j->st, j->part, j->nb0, nullptr, j->sc);
@@ -1528,6 +1512,7 @@ int mg_job_verify(MgJob *j)
     a.v = j->x;
     a.b = j->rhs;
     a.o1 = j->r;
+    a.o2 = L0.d;
     launch_rows<OP_TRUE_RESID>(j, a, L0.nnz);
     hipLaunchKernelGGL(k_mg_dot, dim3(j->nb0), dim3(KB), 0, j->st, j->r, j->r, n, j->part, j->sc);
     hipLaunchKernelGGL(k_mg_red<RED_VERIFY>, dim3(1), dim3(KB), 0, j->st, j->part, j->nb0, nullptr, j->sc);
@@ -1732,7 +1717,6 @@ int mg_batch_run(MgBatch *b, MgJob *const *jobs, int n, int iters)
         hipLaunchKernelGGL(k_mgb_red<RED_CONV>, dim3(ng), dim3(KB), 0, st, D, G);
         for (int l = 0; l < Fmax; ++l) {
             if (lev[l].cnt == 0) continue;
-            hipLaunchKernelGGL(k_mgb_first, dim3(ublk(lev[l].cnt)), dim3(KB), 0, st, tiles(lev[l]), D);
             hipLaunchKernelGGL(k_mgb_rows<OP_CHEB_PRE>, dim3(ublk(lev[l].cnt)), dim3(KB), 0, st, tiles(lev[l]), D);
             hipEvent_t e0, e1;
             if (b->profile && ev_take(b->pool, e0, e1)) {
@@ -1961,17 +1945,22 @@ extern "C" int grmp_mg_apply(grmp_mg *m, const grmp_vector *b, grmp_vector *x, d
 }
 
 // ------------------------------------------- one V-cycle as a preconditioner
-// r_0 = v with the fixed rows zeroed; the device scalars are reset so the
-// V-cycle kernels run (a finished CG leaves done set)
-__global__ void k_mg_pc_in(const double *__restrict__ v, const uint8_t *__restrict__ fixed, double *__restrict__ r,
-                           MgScal *__restrict__ sc, int64_t n)
+// r_0 = v with the fixed rows zeroed and d0 of it; the device scalars are
+// reset so the V-cycle kernels run (a finished CG leaves done set)
+__global__ void k_mg_pc_in(const double *__restrict__ v, const uint8_t *__restrict__ fixed,
+                           const double *__restrict__ dinv, const double *__restrict__ lam, double *__restrict__ r,
+                           double *__restrict__ d, MgScal *__restrict__ sc, int64_t n)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) {
         sc->done = 0;
         sc->status = 0;
     }
-    if (i < n) r[i] = fixed[i] ? 0.0 : v[i];
+    if (i >= n) return;
+    const bool fx = fixed[i] != 0;
+    const double ri = fx ? 0.0 : v[i];
+    r[i] = ri;
+    d[i] = cheb_first(fx, dinv[i], ri, *lam);
 }
 
 int64_t mg_level0_rows(const grmp_mg *m) { return m->n; }
@@ -2021,10 +2010,12 @@ int mg_precond_apply_pair(grmp_mg *m, const double *v0, double *z0, const double
     GRMP_CHECK(m->ctx, st == j->st && j2, GRMP_ERR_ARG, "multigrid preconditioner pair: not prepared");
     GRMP_HIP(m->ctx, hipEventRecord(m->fork, st));
     GRMP_HIP(m->ctx, hipStreamWaitEvent(m->st2, m->fork, 0));
-    hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, m->st2, v1, m->A0->fixed, j2->r, j2->sc, n);
+    hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, m->st2, v1, m->A0->fixed, j2->lv[0].dinv,
+                       j2->lv[0].lam, j2->r, j2->lv[0].d, j2->sc, n);
     mg_vcycle(j2);
     GRMP_HIP(m->ctx, hipMemcpyAsync(z1, j2->z, sizeof(double) * n, hipMemcpyDeviceToDevice, m->st2));
-    hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, st, v0, m->A0->fixed, j->r, j->sc, n);
+    hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, st, v0, m->A0->fixed, j->lv[0].dinv,
+                       j->lv[0].lam, j->r, j->lv[0].d, j->sc, n);
     mg_vcycle(j);
     GRMP_HIP(m->ctx, hipMemcpyAsync(z0, j->z, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
     GRMP_HIP(m->ctx, hipEventRecord(m->join, m->st2));
@@ -2038,7 +2029,8 @@ int mg_precond_apply(grmp_mg *m, const double *v, double *z, hipStream_t st)
     MgJob *j = m->job;
     const int64_t n = m->n;
     GRMP_CHECK(m->ctx, st == j->st, GRMP_ERR_ARG, "multigrid preconditioner: not the hierarchy's stream");
-    hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, st, v, m->A0->fixed, j->r, j->sc, n);
+    hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, st, v, m->A0->fixed, j->lv[0].dinv, j->lv[0].lam,
+                       j->r, j->lv[0].d, j->sc, n);
     mg_vcycle(j);
     GRMP_HIP(m->ctx, hipMemcpyAsync(z, j->z, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
     GRMP_HIP(m->ctx, hipGetLastError());
@@ -2329,9 +2321,11 @@ __global__ void k_amg_dinv(const double *__restrict__ diag, const uint8_t *__res
     dinv[i] = (fixed[i] || !(diag[i] > 0.0)) ? 0.0 : 1.0 / diag[i];
 }
 
-// restriction b_c[I] = sum of r over the members of I, in row order
+// restriction b_c[I] = sum of r over the members of I, in row order; d_c = d0 of b_c
 __global__ void k_amg_restrict(const int32_t *__restrict__ mptr, const int32_t *__restrict__ midx,
-                               const double *__restrict__ r, double *__restrict__ bc, int64_t nc, const MgScal *sc)
+                               const double *__restrict__ r, const uint8_t *__restrict__ fixed_c,
+                               const double *__restrict__ dinv_c, const double *__restrict__ lam_c,
+                               double *__restrict__ bc, double *__restrict__ dc, int64_t nc, const MgScal *sc)
 {
     if (sc->done) return;
     const int64_t I = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2339,6 +2333,7 @@ __global__ void k_amg_restrict(const int32_t *__restrict__ mptr, const int32_t *
     double s = 0.0;
     for (int32_t k = mptr[I]; k < mptr[I + 1]; ++k) s += r[midx[k]];
     bc[I] = s;
+    dc[I] = cheb_first(fixed_c[I] != 0, dinv_c[I], s, *lam_c);
 }
 
 // prolongation x_i += scale x_c[agg i] on the free rows
@@ -2637,7 +2632,7 @@ static void amg_rows(MgRows &a, const AmgLevel &L, const grmp_amg *m)
     a.sc = m->sc;
 }
 
-// z (= x_0) = V(r (= b_0)); level-0 partials of r.z land in part
+// z (= x_0) = V(r (= b_0)), d_0 holding d0 of r; level-0 partials of r.z land in part
 static void amg_vcycle(grmp_amg *m)
 {
     hipStream_t st = m->ctx->stream;
@@ -2646,16 +2641,17 @@ static void amg_vcycle(grmp_amg *m)
         const AmgLevel &L = m->lv[l], &C = m->lv[l + 1];
         MgRows a;
         amg_rows(a, L, m);
+        a.v = L.d;
         a.b = L.b;
         a.o1 = L.x;
-        hipLaunchKernelGGL(k_mg_pre, dim3(nblk(L.n, KB)), dim3(KB), 0, st, a);
+        hipLaunchKernelGGL(k_mg_rows<OP_CHEB_PRE>, dim3(nblk(L.n, KB)), dim3(KB), 0, st, a);
         amg_rows(a, L, m);
         a.v = L.x;
         a.b = L.b;
         a.o1 = L.r;
         hipLaunchKernelGGL(k_mg_rows<OP_RESID>, dim3(nblk(L.n, KB)), dim3(KB), 0, st, a);
-        hipLaunchKernelGGL(k_amg_restrict, dim3(nblk(C.n, 256)), dim3(256), 0, st, C.mptr, C.midx, L.r, C.b, C.n,
-                           m->sc);
+        hipLaunchKernelGGL(k_amg_restrict, dim3(nblk(C.n, 256)), dim3(256), 0, st, C.mptr, C.midx, L.r, C.fixed,
+                           C.dinv, C.lam, C.b, C.d, C.n, m->sc);
     }
     const AmgLevel &C = m->lv[L1];
     hipLaunchKernelGGL(k_mg_dense_apply, dim3(1), dim3(MG_DENSE_MAX), 0, st, m->inv, C.b, (int)C.n, C.x, m->sc);
@@ -2696,7 +2692,8 @@ static void amg_iterate(grmp_amg *m, int iters)
         a.part = m->part;
         hipLaunchKernelGGL(k_mg_rows<OP_PCG_Q>, dim3(nblk(n, KB)), dim3(KB), 0, st, a);
         hipLaunchKernelGGL(k_mg_red<RED_ALPHA>, dim3(1), dim3(KB), 0, st, m->part, m->nb0, nullptr, m->sc);
-        hipLaunchKernelGGL(k_mg_axpy, dim3(m->nb0), dim3(KB), 0, st, m->x, m->r, m->p, m->q, n, m->part, m->sc);
+        hipLaunchKernelGGL(k_mg_axpy, dim3(m->nb0), dim3(KB), 0, st, m->x, m->r, m->p, m->q, L0.fixed, L0.dinv, L0.lam,
+                           L0.d, n, m->part, m->sc);
         hipLaunchKernelGGL(k_mg_red<RED_CONV>, dim3(1), dim3(KB), 0, st, m->part, m->nb0, nullptr, m->sc);
         amg_vcycle(m);
         hipLaunchKernelGGL(k_mg_red<RED_BETA>, dim3(1), dim3(KB), 0, st, m->part, m->nb0, nullptr, m->sc);
@@ -2716,6 +2713,7 @@ static void amg_verify(grmp_amg *m)
     a.v = m->x;
     a.b = m->rhs;
     a.o1 = m->r;
+    a.o2 = L0.d;
     hipLaunchKernelGGL(k_mg_rows<OP_TRUE_RESID>, dim3(nblk(n, KB)), dim3(KB), 0, st, a);
     hipLaunchKernelGGL(k_mg_dot, dim3(m->nb0), dim3(KB), 0, st, m->r, m->r, n, m->part, m->sc);
     hipLaunchKernelGGL(k_mg_red<RED_VERIFY>, dim3(1), dim3(KB), 0, st, m->part, m->nb0, nullptr, m->sc);
@@ -2752,7 +2750,8 @@ int amg_precond_apply(grmp_amg *m, const double *v, double *z, hipStream_t st)
     GRMP_CHECK(m->ctx, st == m->ctx->stream, GRMP_ERR_ARG,
                "algebraic multigrid preconditioner: not the hierarchy's stream");
     const AmgLevel &L0 = m->lv[0];
-    hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(L0.n, 256)), dim3(256), 0, st, v, L0.fixed, m->r, m->sc, L0.n);
+    hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(L0.n, 256)), dim3(256), 0, st, v, L0.fixed, L0.dinv, L0.lam, m->r, L0.d, m->sc,
+                       L0.n);
     amg_vcycle(m);
     GRMP_HIP(m->ctx, hipMemcpyAsync(z, m->z, sizeof(double) * L0.n, hipMemcpyDeviceToDevice, st));
     GRMP_HIP(m->ctx, hipGetLastError());
@@ -2832,6 +2831,7 @@ extern "C" int grmp_amg_apply(grmp_amg *m, const grmp_vector *b, grmp_vector *x,
         a.v = m->x;
         a.b = m->rhs;
         a.o1 = m->r;
+        a.o2 = m->lv[0].d;
         hipLaunchKernelGGL(k_mg_rows<OP_TRUE_RESID>, dim3(nblk(n, KB)), dim3(KB), 0, st, a);
         amg_vcycle(m);
         hipLaunchKernelGGL(k_mg_dot, dim3(m->nb0), dim3(KB), 0, st, m->r, m->r, n, m->part2, m->sc);
