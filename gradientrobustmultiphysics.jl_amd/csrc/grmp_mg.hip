@@ -648,6 +648,33 @@ struct MgBLevel {
     const int8_t *fsign;
 };
 
+// The levels of a one-workgroup coarse end packed into LDS: an image of their
+// matrices (FP32 values, 16-bit columns and row pointers, D^-1, masks, lambda,
+// aggregates) laid out once per hierarchy in device memory and copied in at
+// the kernel's start, and behind it the level vectors, which never leave LDS.
+// Offsets are in bytes from the start of LDS.
+#define MG_PACK_LEVELS 12
+#define MG_LDS_MAX (155 * 1024)  // of a CU's 160 KB; the reductions' static arrays need the rest
+enum MgTransfer { TR_P1 = 0, TR_P2 = 1, TR_AGG = 2 };
+struct MgPackLevel {
+    int32_t n, N, fe, ncomp;
+    int32_t tr;                   // transfer to the next level
+    int32_t val, ci, rp, dinv, fix, lam;
+    int32_t agg, mptr, midx;      // TR_AGG: row -> coarse row, and the coarse rows' members
+    int32_t x, b, r, d;
+};
+struct MgPack {
+    int32_t nlev;                 // 0: does not fit, the levels stay in device memory
+    int32_t image, lds;           // bytes of the image (a multiple of 16) and in all
+    int32_t ninv;
+    const char *img;
+    const double *inv;            // dense inverse of the last level
+    const int32_t *cells;         // TR_P2: the fine level's mesh
+    const int8_t *fsign;
+    double scale;                 // TR_AGG: of the coarse correction
+    MgPackLevel lv[MG_PACK_LEVELS];
+};
+
 struct MgBDesc {
     int first, nlev, nb0, pad;  // levels first .. nlev-1 run in the workgroup
     MgBLevel lv[MG_MAX_LEVELS];
@@ -656,6 +683,7 @@ struct MgBDesc {
     const double *rhs;
     double *part;               // level-0 block partials (nb0 entries)
     MgScal *sc;
+    MgPack pack;                // the same levels in LDS, where they fit
 };
 
 // sum over the workgroup, returned to every thread
@@ -745,23 +773,244 @@ __device__ double blk_vcycle(const MgBDesc &D)
     return rz;
 }
 
+// ---- the same V-cycle with everything in LDS
+// Latency-bound: about seven short phases a level with a workgroup barrier
+// after each.  With matrices and vectors in device memory every phase waited
+// for a chain of three or four L2 reads (row pointer, column and value, x,
+// epilogue operands): 59-104 us per V-cycle of 25 ... 1,089 rows a level.  One
+// coalesced copy of the image (about 100 KB) and LDS latencies after it take
+// 30-35 us.
+__device__ __forceinline__ void pk_stage(const MgPack &P, char *lds)
+{
+    const uint4 *src = reinterpret_cast<const uint4 *>(P.img);
+    uint4 *dst = reinterpret_cast<uint4 *>(lds);
+    for (int k = threadIdx.x; k < P.image / 16; k += MG_BT) dst[k] = src[k];
+}
+
+// this thread's share of the dense inverse: row t / 16, columns t % 16 + 16 m
+__device__ __forceinline__ void pk_load_inv(const MgPack &P, double inv[4])
+{
+    const int i = threadIdx.x >> 4, n = P.ninv;
+#pragma unroll
+    for (int m = 0; m < 4; ++m) {
+        const int j = (threadIdx.x & 15) + 16 * m;
+        inv[m] = i < n && j < n ? P.inv[i * n + j] : 0.0;
+    }
+}
+
+// rows of level L through the epilogue OP (as blk_rows); returns this thread's partial
+template <int OP>
+__device__ __forceinline__ double pk_rows(const MgPackLevel &L, char *lds, int ov, int oo1, int oo2)
+{
+    const float *val = reinterpret_cast<const float *>(lds + L.val);
+    const uint16_t *ci = reinterpret_cast<const uint16_t *>(lds + L.ci);
+    const uint16_t *rp = reinterpret_cast<const uint16_t *>(lds + L.rp);
+    const double *v = reinterpret_cast<const double *>(lds + ov);
+    const double *b = reinterpret_cast<const double *>(lds + L.b), *d = reinterpret_cast<const double *>(lds + L.d);
+    const double *dinv = reinterpret_cast<const double *>(lds + L.dinv);
+    const double *lam = reinterpret_cast<const double *>(lds + L.lam);
+    const uint8_t *fix = reinterpret_cast<const uint8_t *>(lds + L.fix);
+    double *o1 = reinterpret_cast<double *>(lds + oo1), *o2 = reinterpret_cast<double *>(lds + oo2);
+    double part = 0.0;
+    for (int i = threadIdx.x; i < L.n; i += MG_BT) {
+        const int k0 = rp[i], k1 = rp[i + 1];
+        double s = 0.0;
+        for (int k = k0; k < k1; k += 4) {  // four products in flight; past the row's end its last entry again, unused
+            float w[4];
+            int c[4];
+            double xv[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int e = k + u < k1 ? k + u : k1 - 1;
+                w[u] = val[e];
+                c[u] = ci[e];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) xv[u] = v[c[u]];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (k + u < k1) s += (double)w[u] * xv[u];
+        }
+        // b and d are read before o1 / o2 of the same row are written
+        part += mg_epilogue<OP>(i, s, fix[i] != 0, v, b, dinv, d, lam, o1, o2);
+    }
+    return part;
+}
+
+// x_0 = V(b_0) on the packed levels; b_0 is set, row by row by the thread that
+// owns it.  Returns this thread's partial of b_0 . x_0; x_0 likewise is
+// complete for a thread's own rows.
+__device__ double pk_vcycle(const MgPack &P, char *lds, const double inv[4])
+{
+    const int L1 = P.nlev - 1;
+    {
+        const MgPackLevel &L = P.lv[0];
+        const double *b = reinterpret_cast<const double *>(lds + L.b);
+        const double *dinv = reinterpret_cast<const double *>(lds + L.dinv);
+        const uint8_t *fix = reinterpret_cast<const uint8_t *>(lds + L.fix);
+        double *d = reinterpret_cast<double *>(lds + L.d);
+        const double lam = *reinterpret_cast<const double *>(lds + L.lam);
+        for (int i = threadIdx.x; i < L.n; i += MG_BT) d[i] = cheb_first(fix[i] != 0, dinv[i], b[i], lam);
+    }
+    __syncthreads();
+    for (int l = 0; l < L1; ++l) {
+        const MgPackLevel &L = P.lv[l], &C = P.lv[l + 1];
+        pk_rows<OP_CHEB_PRE>(L, lds, L.d, L.x, L.x);
+        __syncthreads();
+        pk_rows<OP_RESID>(L, lds, L.x, L.r, L.r);
+        __syncthreads();
+        const double *r = reinterpret_cast<const double *>(lds + L.r);
+        const double *dinv = reinterpret_cast<const double *>(lds + C.dinv);
+        const uint8_t *fix = reinterpret_cast<const uint8_t *>(lds + C.fix);
+        double *bc = reinterpret_cast<double *>(lds + C.b), *dc = reinterpret_cast<double *>(lds + C.d);
+        const double lam = *reinterpret_cast<const double *>(lds + C.lam);
+        for (int t = threadIdx.x; t < C.n; t += MG_BT) {
+            double s;
+            if (L.tr == TR_P1) {
+                s = restrict_p1_one(L.N, C.N, r, fix, t);
+            } else if (L.tr == TR_P2) {
+                s = restrict_p2_one(L.N, r, fix, t);
+            } else {
+                const uint16_t *mp = reinterpret_cast<const uint16_t *>(lds + L.mptr);
+                const uint16_t *mi = reinterpret_cast<const uint16_t *>(lds + L.midx);
+                s = 0.0;
+                for (int k = mp[t]; k < mp[t + 1]; ++k) s += r[mi[k]];
+            }
+            bc[t] = s;
+            dc[t] = cheb_first(fix[t] != 0, dinv[t], s, lam);
+        }
+        __syncthreads();
+    }
+    {  // dense solve: sixteen lanes a row
+        const MgPackLevel &C = P.lv[L1];
+        const double *b = reinterpret_cast<const double *>(lds + C.b);
+        double s = 0.0;
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            const int j = (threadIdx.x & 15) + 16 * m;
+            if (j < C.n) s += inv[m] * b[j];
+        }
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 16);
+        const int i = threadIdx.x >> 4;
+        if ((threadIdx.x & 15) == 0 && i < C.n) reinterpret_cast<double *>(lds + C.x)[i] = s;
+        __syncthreads();
+    }
+    double part = 0.0;
+    for (int l = L1 - 1; l >= 0; --l) {
+        const MgPackLevel &L = P.lv[l], &C = P.lv[l + 1];
+        const double *xc = reinterpret_cast<const double *>(lds + C.x);
+        double *x = reinterpret_cast<double *>(lds + L.x);
+        const uint8_t *fix = reinterpret_cast<const uint8_t *>(lds + L.fix);
+        if (L.tr == TR_P1) {
+            for (int t = threadIdx.x; t < L.n; t += MG_BT) prolong_p1_one(L.N, C.N, L.ncomp, xc, fix, x, t);
+        } else if (L.tr == TR_P2) {
+            const int nn = (L.N + 1) * (L.N + 1), nc = 2 * L.N * L.N;
+            for (int t = threadIdx.x; t < (nn > nc ? nn : nc); t += MG_BT)
+                prolong_p2_one(L.N, P.cells, P.fsign, xc, fix, x, t);
+        } else {
+            const uint16_t *agg = reinterpret_cast<const uint16_t *>(lds + L.agg);
+            for (int t = threadIdx.x; t < L.n; t += MG_BT)
+                if (agg[t] != 0xffff) x[t] += P.scale * xc[agg[t]];
+        }
+        __syncthreads();
+        pk_rows<OP_CHEB_POST1>(L, lds, L.x, L.d, L.r);
+        __syncthreads();
+        part = pk_rows<OP_CHEB_POST2>(L, lds, L.r, L.x, L.x);
+        __syncthreads();
+    }
+    if (L1 == 0) {  // a single level: x is the exact solve
+        const double *b = reinterpret_cast<const double *>(lds + P.lv[0].b);
+        const double *x = reinterpret_cast<const double *>(lds + P.lv[0].x);
+        for (int i = threadIdx.x; i < P.lv[0].n; i += MG_BT) part += b[i] * x[i];
+    }
+    return part;
+}
+
+// packed V-cycle from b to x in device memory
+__device__ __forceinline__ double pk_apply(const MgPack &P, char *lds, const double inv[4],
+                                           const double *__restrict__ b, double *__restrict__ x)
+{
+    double *lb = reinterpret_cast<double *>(lds + P.lv[0].b);
+    const double *lx = reinterpret_cast<const double *>(lds + P.lv[0].x);
+    const int n = P.lv[0].n;
+    for (int i = threadIdx.x; i < n; i += MG_BT) lb[i] = b[i];
+    const double part = pk_vcycle(P, lds, inv);
+    for (int i = threadIdx.x; i < n; i += MG_BT) x[i] = lx[i];
+    return part;
+}
+
+// the levels D.first .. D.nlev-1 of a V-cycle in one workgroup; returns the
+// workgroup total of b_0 . x_0 when D.first == 0
+__device__ double blk_coarse(const MgBDesc &D, char *lds)
+{
+    if (D.pack.nlev == 0) return blk_vcycle(D);
+    double inv[4];
+    pk_load_inv(D.pack, inv);
+    pk_stage(D.pack, lds);
+    __syncthreads();
+    const MgBLevel &L = D.lv[D.first];
+    const double part = pk_apply(D.pack, lds, inv, L.b, L.x);
+    return D.first == 0 ? blk_sum(part) : 0.0;
+}
+
+// one level's part of the image
+struct MgPackSrc {
+    const int32_t *rp, *ci;
+    const float *val32;
+    const double *dinv, *lam;
+    const uint8_t *fixed;
+    const int32_t *agg, *mptr, *midx;  // aggregates (TR_AGG), or nullptr
+    int32_t nnz, nc;                   // nonzeros; rows of the next level
+};
+__global__ void k_mg_pack(MgPackLevel L, MgPackSrc S, char *__restrict__ img)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < S.nnz) {
+        reinterpret_cast<float *>(img + L.val)[t] = S.val32[t];
+        reinterpret_cast<uint16_t *>(img + L.ci)[t] = (uint16_t)S.ci[t];
+    }
+    if (t <= L.n) reinterpret_cast<uint16_t *>(img + L.rp)[t] = (uint16_t)S.rp[t];
+    if (t < L.n) {
+        reinterpret_cast<double *>(img + L.dinv)[t] = S.dinv[t];
+        reinterpret_cast<uint8_t *>(img + L.fix)[t] = S.fixed[t];
+        if (S.agg) {
+            reinterpret_cast<uint16_t *>(img + L.agg)[t] = S.agg[t] < 0 ? (uint16_t)0xffff : (uint16_t)S.agg[t];
+            reinterpret_cast<uint16_t *>(img + L.midx)[t] = (uint16_t)S.midx[t];
+        }
+    }
+    if (S.agg && t <= S.nc) reinterpret_cast<uint16_t *>(img + L.mptr)[t] = (uint16_t)S.mptr[t];
+    if (t == 0) *reinterpret_cast<double *>(img + L.lam) = *S.lam;
+}
+
 // coarse end of a V-cycle (levels D.first ..); at D.first == 0 also the
 // level-0 partials of r.z (total in part[0], zeros after it)
 __global__ __launch_bounds__(MG_BT) void k_mg_vcycle_block(const MgBDesc *__restrict__ Dp, const MgScal *sc)
 {
+    extern __shared__ __align__(16) char pk_lds[];
     if (sc->done) return;
     const MgBDesc &D = *Dp;
-    const double rz = blk_vcycle(D);
+    const double rz = blk_coarse(D, pk_lds);
     if (D.first == 0)
         for (int k = threadIdx.x; k < D.nb0; k += MG_BT) D.part[k] = k == 0 ? rz : 0.0;
 }
 
 // up to iters CG iterations of a request whose levels all fit the workgroup,
 // with the true-residual check and restart of mg_job_verify done in place
-__device__ void mg_pcg_block_body(const MgBDesc &D, MgScal *sc, int iters)
+__device__ void mg_pcg_block_body(const MgBDesc &D, MgScal *sc, int iters, char *lds)
 {
     const MgBLevel &L0 = D.lv[0];
     const int64_t n = L0.n;
+    const bool packed = D.pack.nlev > 0;
+    double inv[4] = {0.0, 0.0, 0.0, 0.0};
+    if (packed) {  // staged once for all the iterations
+        if (sc->done == 1) return;
+        pk_load_inv(D.pack, inv);
+        pk_stage(D.pack, lds);
+    }
+    auto vcycle = [&]() -> double {
+        return packed ? blk_sum(pk_apply(D.pack, lds, inv, D.r, D.z)) : blk_vcycle(D);
+    };
     for (int k = 0; k < iters; ++k) {
         __syncthreads();
         const int st = sc->done;
@@ -779,7 +1028,7 @@ __device__ void mg_pcg_block_body(const MgBDesc &D, MgScal *sc, int iters)
             }
             __syncthreads();
             if (sc->done) continue;
-            const double rz = blk_vcycle(D);
+            const double rz = vcycle();
             if (threadIdx.x == 0) mg_scalar<RED_RESTART>(sc, rz, 0.0);
             __syncthreads();
             if (sc->done) continue;
@@ -802,7 +1051,7 @@ __device__ void mg_pcg_block_body(const MgBDesc &D, MgScal *sc, int iters)
         if (threadIdx.x == 0) mg_scalar<RED_CONV>(sc, rr, 0.0);
         __syncthreads();
         if (sc->done) continue;
-        const double rz = blk_vcycle(D);
+        const double rz = vcycle();
         if (threadIdx.x == 0) mg_scalar<RED_BETA>(sc, rz, 0.0);
         __syncthreads();
         if (sc->done) continue;
@@ -813,7 +1062,8 @@ __device__ void mg_pcg_block_body(const MgBDesc &D, MgScal *sc, int iters)
 
 __global__ __launch_bounds__(MG_BT) void k_mg_pcg_block(const MgBDesc *__restrict__ Dp, MgScal *sc, int iters)
 {
-    mg_pcg_block_body(*Dp, sc, iters);
+    extern __shared__ __align__(16) char pk_lds[];
+    mg_pcg_block_body(*Dp, sc, iters, pk_lds);
 }
 
 // ------------------------------------------------------ lockstep batches
@@ -988,16 +1238,18 @@ __global__ __launch_bounds__(KB) void k_mgb_red(const MgBDesc *const *__restrict
 __global__ __launch_bounds__(MG_BT) void k_mgb_vcycle_block(const MgBDesc *const *__restrict__ Dp,
                                                             const int32_t *__restrict__ reqs)
 {
+    extern __shared__ __align__(16) char pk_lds[];
     const MgBDesc &D = *Dp[reqs[blockIdx.x]];
     if (D.sc->done) return;
-    blk_vcycle(D);
+    blk_coarse(D, pk_lds);
 }
 
 __global__ __launch_bounds__(MG_BT) void k_mgb_pcg_block(const MgBDesc *const *__restrict__ Dp,
                                                          const int32_t *__restrict__ reqs, int iters)
 {
+    extern __shared__ __align__(16) char pk_lds[];
     const MgBDesc &D = *Dp[reqs[blockIdx.x]];
-    mg_pcg_block_body(D, D.sc, iters);
+    mg_pcg_block_body(D, D.sc, iters, pk_lds);
 }
 
 __global__ void k_mgb_status(const MgBDesc *const *__restrict__ Dp, int n, MgStatus *__restrict__ out)
@@ -1010,6 +1262,78 @@ __global__ void k_mgb_status(const MgBDesc *const *__restrict__ Dp, int n, MgSta
     out[i].done = sc->done;
     out[i].status = sc->status;
     out[i].pad = 0;
+}
+
+// ------------------------------------------------------ packing (host)
+static size_t mg_lds_limit()
+{
+    int dev = 0, v = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess)
+        return 0;
+    return std::min<size_t>((size_t)std::max(v - 1024, 0), MG_LDS_MAX);
+}
+
+struct MgPackShape {
+    int64_t n, nnz;
+    int N, fe, ncomp, tr;
+};
+// Offsets of the levels (the last one solved by its dense inverse); false, and
+// P.nlev = 0, if they do not fit: 16-bit indices and the LDS of one workgroup.
+static bool mg_pack_layout(MgPack &P, const MgPackShape *sh, int nlev)
+{
+    memset(&P, 0, sizeof(P));
+    if (nlev < 1 || nlev > MG_PACK_LEVELS || sh[nlev - 1].n > MG_DENSE_MAX) return false;
+    const size_t limit = mg_lds_limit();
+    size_t off = 0;
+    auto take = [&](size_t bytes, size_t align) {
+        off = (off + align - 1) / align * align;
+        const size_t o = off;
+        off += bytes;
+        return (int32_t)o;
+    };
+    for (int l = 0; l < nlev; ++l) {
+        const MgPackShape &S = sh[l];
+        if (S.n >= 0xffff || S.nnz >= 0xffff || off > limit) return false;
+        MgPackLevel &L = P.lv[l];
+        L.n = (int32_t)S.n;
+        L.N = S.N;
+        L.fe = S.fe;
+        L.ncomp = S.ncomp;
+        L.tr = S.tr;
+        L.dinv = take(8 * S.n, 8);
+        L.lam = take(8, 8);
+        L.val = take(4 * S.nnz, 4);
+        L.ci = take(2 * S.nnz, 2);
+        L.rp = take(2 * (S.n + 1), 2);
+        if (S.tr == TR_AGG && l + 1 < nlev) {
+            L.agg = take(2 * S.n, 2);
+            L.midx = take(2 * S.n, 2);
+            L.mptr = take(2 * (sh[l + 1].n + 1), 2);
+        }
+        L.fix = take(S.n, 1);
+    }
+    off = (off + 15) / 16 * 16;
+    P.image = (int32_t)off;
+    for (int l = 0; l < nlev; ++l) {
+        MgPackLevel &L = P.lv[l];
+        L.x = take(8 * sh[l].n, 8);
+        L.b = take(8 * sh[l].n, 8);
+        L.r = take(8 * sh[l].n, 8);
+        L.d = take(8 * sh[l].n, 8);
+    }
+    if (off > limit) return false;
+    P.lds = (int32_t)off;
+    P.ninv = (int32_t)sh[nlev - 1].n;
+    P.nlev = nlev;
+    return true;
+}
+
+// the kernels with a packed coarse end take more than 64 KB of dynamic LDS
+static int mg_allow_lds(grmp_ctx *ctx, const void *kernel)
+{
+    GRMP_HIP(ctx, hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, MG_LDS_MAX));
+    return GRMP_OK;
 }
 
 // ------------------------------------------------------------- the job
@@ -1036,6 +1360,7 @@ struct MgJob {
     MgScal *sc = nullptr;
     int nb0 = 0;
     int first_small = 0;      // first level that runs inside one workgroup
+    char *img = nullptr;      // LDS image of those levels
     MgBDesc hdesc;
     MgBDesc *ddesc = nullptr;
     hipEvent_t ev = nullptr;
@@ -1064,7 +1389,7 @@ static size_t mg_layout(MgJob *j, bool assign)
            o_q = take(n0 * 8), o_part = take(nb0 * 8), o_part2 = take(nb0 * 8), o_sc = take(sizeof(MgScal)),
            o_desc = take(sizeof(MgBDesc));
     const MgLevel &c = j->lv[j->nlev - 1];
-    size_t o_inv = take(c.n * c.n * 8);
+    size_t o_inv = take(c.n * c.n * 8), o_img = take(MG_LDS_MAX);
     std::vector<size_t> o(MG_MAX_LEVELS * 10);
     for (int l = 0; l < j->nlev; ++l) {
         const MgLevel &L = j->lv[l];
@@ -1093,6 +1418,7 @@ static size_t mg_layout(MgJob *j, bool assign)
     j->sc = (MgScal *)(B + o_sc);
     j->ddesc = (MgBDesc *)(B + o_desc);
     j->inv = (double *)(B + o_inv);
+    j->img = B + o_img;
     j->nb0 = nb0;
     for (int l = 0; l < j->nlev; ++l) {
         MgLevel &L = j->lv[l];
@@ -1123,6 +1449,18 @@ int64_t mg_job_bytes(const MgLevelIn *in, int nlev)
         j.lv[l].nc = in[l].sp->mesh->ncells;
     }
     return (int64_t)mg_layout(&j, false);
+}
+
+// the packed form of the levels from first_small on
+static bool mg_job_pack_layout(const MgJob *j, MgPack &P)
+{
+    MgPackShape sh[MG_MAX_LEVELS];
+    for (int l = j->first_small; l < j->nlev; ++l) {
+        const MgLevel &L = j->lv[l];
+        sh[l - j->first_small] = MgPackShape{L.n, L.nnz, L.in.N, L.in.fe, L.in.ncomp,
+                                             L.in.fe == GRMP_FE_H1P2 ? TR_P2 : TR_P1};
+    }
+    return mg_pack_layout(P, sh, j->nlev - j->first_small);
 }
 
 static void fill_desc(MgJob *j)
@@ -1162,6 +1500,25 @@ static void fill_desc(MgJob *j)
     D.rhs = j->rhs;
     D.part = j->part;
     D.sc = j->sc;
+    if (mg_job_pack_layout(j, D.pack)) {
+        D.pack.img = j->img;
+        D.pack.inv = j->inv;
+        D.pack.cells = D.lv[j->first_small].cells;
+        D.pack.fsign = D.lv[j->first_small].fsign;
+    }
+}
+
+// the LDS image, once the levels' values, bounds and inverse are enqueued
+static void mg_job_pack(MgJob *j)
+{
+    const MgPack &P = j->hdesc.pack;
+    for (int k = 0; k < P.nlev; ++k) {
+        const MgLevel &L = j->lv[j->first_small + k];
+        const MgPackSrc S{L.in.A->rowptr, L.in.A->cols, L.val32, L.dinv, L.lam, L.in.A->fixed,
+                          nullptr, nullptr, nullptr, (int32_t)L.nnz, 0};
+        hipLaunchKernelGGL(k_mg_pack, dim3(nblk(std::max(L.nnz, L.n + 1), 256)), dim3(256), 0, j->st, P.lv[k], S,
+                           j->img);
+    }
 }
 
 int mg_job_create(grmp_ctx *ctx, hipStream_t st, const MgLevelIn *in, int nlev, bool profile, int block_rows,
@@ -1208,7 +1565,18 @@ int mg_job_create(grmp_ctx *ctx, hipStream_t st, const MgLevelIn *in, int nlev, 
     if (j->lv[0].n <= block_rows) j->first_small = 0;
     else
         while (j->first_small > 1 && j->lv[j->first_small - 1].n <= coarse_rows) --j->first_small;
+    // a coarse end that does not fit LDS gives its finest levels to grid
+    // kernels: six launches of about 4.5 us against the 104 us that elasticity's
+    // 1,250 ... 32 rows took in device memory
+    MgPack P;
+    while (j->first_small > 0 && j->first_small < nlev - 1 && !mg_job_pack_layout(j, P)) ++j->first_small;
     fill_desc(j);
+    if (mg_allow_lds(ctx, (const void *)k_mg_vcycle_block) || mg_allow_lds(ctx, (const void *)k_mg_pcg_block) ||
+        mg_allow_lds(ctx, (const void *)k_mgb_vcycle_block) || mg_allow_lds(ctx, (const void *)k_mgb_pcg_block)) {
+        (void)hipFreeAsync(j->buf, st);
+        delete j;
+        return GRMP_ERR_HIP;
+    }
     if (hipEventCreateWithFlags(&j->ev, hipEventDisableTiming) != hipSuccess) {
         (void)hipFreeAsync(j->buf, st);
         delete j;
@@ -1309,7 +1677,7 @@ static void mg_vcycle(MgJob *j)
         launch_rows<OP_RESID>(j, a, L.nnz);
         mg_restrict(j, l);
     }
-    hipLaunchKernelGGL(k_mg_vcycle_block, dim3(1), dim3(MG_BT), 0, j->st, j->ddesc, j->sc);
+    hipLaunchKernelGGL(k_mg_vcycle_block, dim3(1), dim3(MG_BT), j->hdesc.pack.lds, j->st, j->ddesc, j->sc);
     for (int l = F - 1; l >= 0; --l) {
         MgLevel &L = j->lv[l];
         mg_prolong(j, l);
@@ -1350,6 +1718,7 @@ static int mg_job_assemble(MgJob *j)
     const MgLevel &C = j->lv[j->nlev - 1];
     hipLaunchKernelGGL(k_mg_dense_inv, dim3(1), dim3(256), 0, st, C.in.A->rowptr, C.in.A->cols, C.val, C.in.A->fixed,
                        (int)C.n, j->inv);
+    mg_job_pack(j);
     GRMP_HIP(ctx, hipMemcpyAsync(j->ddesc, &j->hdesc, sizeof(MgBDesc), hipMemcpyHostToDevice, st));
     return GRMP_OK;
 }
@@ -1420,6 +1789,7 @@ int mg_jobs_setup_batched(MgJob *const *jobs, int n, hipStream_t st, double *con
         const MgLevel &C = j->lv[j->nlev - 1];
         hipLaunchKernelGGL(k_mg_dense_inv, dim3(1), dim3(256), 0, st, C.in.A->rowptr, C.in.A->cols, C.val,
                            C.in.A->fixed, (int)C.n, j->inv);
+        mg_job_pack(j);
         GRMP_HIP(ctx, hipMemcpyAsync(j->ddesc, &j->hdesc, sizeof(MgBDesc), hipMemcpyHostToDevice, st));
         GRMP_TRY(mg_job_start(j, rtol[k], maxit));
     }
@@ -1431,7 +1801,7 @@ static int mg_iterate_grid(MgJob *j, int iters);
 int mg_job_iterate(MgJob *j, int iters)
 {
     if (j->first_small == 0) {  // every level fits one workgroup: whole iterations in one launch
-        hipLaunchKernelGGL(k_mg_pcg_block, dim3(1), dim3(MG_BT), 0, j->st, j->ddesc, j->sc, iters);
+        hipLaunchKernelGGL(k_mg_pcg_block, dim3(1), dim3(MG_BT), j->hdesc.pack.lds, j->st, j->ddesc, j->sc, iters);
         GRMP_HIP(j->ctx, hipGetLastError());
         return GRMP_OK;
     }
@@ -1663,12 +2033,16 @@ int mg_batch_run(MgBatch *b, MgJob *const *jobs, int n, int iters)
     grmp_ctx *ctx = b->ctx;
     hipStream_t st = b->st;
     std::vector<int> grid, blk;
-    int Fmax = 0;
+    int Fmax = 0, lds_grid = 0, lds_blk = 0;  // LDS of the one-workgroup kernels: the largest of their jobs
     for (int i = 0; i < n; ++i) {
-        if (jobs[i]->first_small == 0) blk.push_back(i);
-        else {
+        const int lds = jobs[i]->hdesc.pack.lds;
+        if (jobs[i]->first_small == 0) {
+            blk.push_back(i);
+            lds_blk = std::max(lds_blk, lds);
+        } else {
             grid.push_back(i);
             Fmax = std::max(Fmax, jobs[i]->first_small);
+            lds_grid = std::max(lds_grid, lds);
         }
     }
     // tile segments: level-0 rows; per grid level l: its rows, the next
@@ -1736,7 +2110,7 @@ int mg_batch_run(MgBatch *b, MgJob *const *jobs, int n, int iters)
             }
             hipLaunchKernelGGL(k_mgb_restrict, dim3(ublk(res[l].cnt)), dim3(KB), 0, st, tiles(res[l]), D);
         }
-        hipLaunchKernelGGL(k_mgb_vcycle_block, dim3(ng), dim3(MG_BT), 0, st, D, G);
+        hipLaunchKernelGGL(k_mgb_vcycle_block, dim3(ng), dim3(MG_BT), lds_grid, st, D, G);
         for (int l = Fmax - 1; l >= 0; --l) {
             if (lev[l].cnt == 0) continue;
             hipLaunchKernelGGL(k_mgb_prolong, dim3(ublk(pro[l].cnt)), dim3(KB), 0, st, tiles(pro[l]), D);
@@ -1746,7 +2120,7 @@ int mg_batch_run(MgBatch *b, MgJob *const *jobs, int n, int iters)
         hipLaunchKernelGGL(k_mgb_red<RED_BETA>, dim3(ng), dim3(KB), 0, st, D, G);
         hipLaunchKernelGGL(k_mgb_update_p, dim3(ublk(L0.cnt)), dim3(KB), 0, st, tiles(L0), D);
     }
-    if (nbk > 0) hipLaunchKernelGGL(k_mgb_pcg_block, dim3(nbk), dim3(MG_BT), 0, st, D, Bk, iters);
+    if (nbk > 0) hipLaunchKernelGGL(k_mgb_pcg_block, dim3(nbk), dim3(MG_BT), lds_blk, st, D, Bk, iters);
     hipLaunchKernelGGL(k_mgb_status, dim3(nblk(n, 256)), dim3(256), 0, st, D, n, b->dstat);
     GRMP_HIP(ctx, hipMemcpyAsync(b->hstat, b->dstat, n * sizeof(MgStatus), hipMemcpyDeviceToHost, st));
     GRMP_HIP(ctx, hipEventRecord(b->ev, st));
