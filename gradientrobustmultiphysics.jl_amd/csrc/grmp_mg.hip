@@ -131,7 +131,8 @@ __device__ __forceinline__ void mg_scalar(MgScal *sc, double a, double b)
 // bytes per nonzero.  The CG product (PCG_Q) and the true residual of the
 // convergence check (TRUE_RESID) read the FP64 values, so the accepted
 // solutions meet rtol against the FP64 operator.
-enum MgOp { OP_RESID = 0, OP_CHEB_PRE = 1, OP_CHEB_POST1 = 2, OP_CHEB_POST2 = 3, OP_PCG_Q = 4, OP_TRUE_RESID = 5 };
+enum MgOp { OP_RESID = 0, OP_CHEB_PRE = 1, OP_CHEB_POST1 = 2, OP_CHEB_POST2 = 3, OP_PCG_Q = 4, OP_TRUE_RESID = 5,
+            OP_AGG_POST1 = 6 };
 template <int OP>
 struct MgF64 {
     static constexpr bool value = OP == OP_PCG_Q || OP == OP_TRUE_RESID;
@@ -149,6 +150,8 @@ struct MgRows {
     const double *lam;   // Gershgorin bound of D^-1 A (device)
     const MgScal *sc;
     double *part;        // block partials (OP_PCG_Q: p.q; OP_CHEB_POST2 at level 0: r.z)
+    const int32_t *agg;  // OP_AGG_POST1: coarse row of each row, the scale of the correction
+    double scale;
 };
 
 // d0 = D^-1 b / theta, the first step of the pre-smoothing from x0 = 0.  The
@@ -170,6 +173,10 @@ __device__ __forceinline__ double cheb_first(bool fx, double dinv, double b, dou
 //   POST1   v = x:   d = D^-1 (b - A x) / theta -> o1,  x + d -> o2
 //   POST2   v = x1:  o1 = x1 + C1 d + C2 D^-1 (b - A x1)   [+ partials of b . o1]
 //   PCG_Q   o1 = A v                                        [+ partials of v . o1]
+//   AGG_POST1  POST1 with the aggregates' prolongation e = scale P v, v on the
+//           coarse rows, folded in: the columns are the aggregates of A's, so
+//           the product is A P v, and with b the residual of x = d
+//           d = D^-1 (b - A e) / theta -> o1,  x + e + d -> o2
 // Fixed rows get 0 (no residual, no correction).
 template <int OP>
 __device__ __forceinline__ double mg_epilogue(int64_t i, double s, bool fx, const double *__restrict__ v,
@@ -219,7 +226,17 @@ __device__ __forceinline__ void mg_rows_body(const MgRows &a, int64_t r0, int pi
     else s = csr_rows_lds<double, float, double, MG_ROWS_CAP>(a.rp, a.ci, a.val32, a.v, r0, r1, lds);
     const int64_t i = r0 + threadIdx.x;
     double pa = 0.0, pb = 0.0;
-    if (i < r1) pa = mg_epilogue<OP>(i, s, a.fixed[i] != 0, a.v, a.b, a.dinv, a.d, a.lam, a.o1, a.o2);
+    if constexpr (OP == OP_AGG_POST1) {
+        if (i < r1) {
+            const bool fx = a.fixed[i] != 0;
+            const double dd = fx ? 0.0 : a.dinv[i] * (a.b[i] - a.scale * s) * CHEB_ITHETA(*a.lam);
+            const double x = fx ? a.d[i] : a.d[i] + a.scale * a.v[a.agg[i]];
+            a.o1[i] = dd;
+            a.o2[i] = x + dd;
+        }
+    } else if (i < r1) {
+        pa = mg_epilogue<OP>(i, s, a.fixed[i] != 0, a.v, a.b, a.dinv, a.d, a.lam, a.o1, a.o2);
+    }
     if ((OP == OP_CHEB_POST2 || OP == OP_PCG_Q) && a.part) {
         block_sum2(pa, pb);
         if (threadIdx.x == 0) a.part[pidx] = pa;
@@ -2461,6 +2478,7 @@ struct AmgLevel {
     double *dinv = nullptr, *lam = nullptr;
     double *x = nullptr, *b = nullptr, *r = nullptr, *d = nullptr;  // level 0: x = z, b = r of the CG
     int32_t *agg = nullptr;                      // row -> row of the next level (-1: fixed)
+    int32_t *cagg = nullptr;                     // aggregate of each nonzero's column (fixed: the next level's n)
     int32_t *mptr = nullptr, *midx = nullptr;    // rows of this level: their members on the previous one
 };
 
@@ -2474,6 +2492,9 @@ struct grmp_amg {
     double *part = nullptr, *part2 = nullptr;
     MgScal *sc = nullptr;
     int nb0 = 0;
+    MgPack pack;            // levels first .. nlev-1 run in one workgroup (nlev > 1)
+    int first = 0;
+    char *img = nullptr;    // their LDS image
     MgStatus *h = nullptr;  // pinned
     hipEvent_t ev = nullptr;
     std::vector<void *> mem;  // device allocations of the hierarchy
@@ -2710,15 +2731,29 @@ __global__ void k_amg_restrict(const int32_t *__restrict__ mptr, const int32_t *
     dc[I] = cheb_first(fixed_c[I] != 0, dinv_c[I], s, *lam_c);
 }
 
-// prolongation x_i += scale x_c[agg i] on the free rows
-__global__ void k_amg_prolong(const int32_t *__restrict__ agg, const double *__restrict__ xc, double scale,
-                              double *__restrict__ x, int64_t n, const MgScal *sc)
+// the aggregate of every nonzero's column, nc where the column is fixed (the
+// coarse vectors hold a zero there)
+__global__ void k_amg_cagg(const int32_t *__restrict__ ci, const int32_t *__restrict__ agg, int64_t nnz, int32_t nc,
+                           int32_t *__restrict__ cagg)
 {
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= nnz) return;
+    const int32_t a = agg[ci[k]];
+    cagg[k] = a < 0 ? nc : a;
+}
+
+// the coarse end of the cycle: x = V(b) on the packed levels.  Launched level
+// by level these few hundred rows took six launches of 2.5-5 us a level.
+__global__ __launch_bounds__(MG_BT) void k_amg_vcycle_block(MgPack P, const double *__restrict__ b,
+                                                            double *__restrict__ x, const MgScal *sc)
+{
+    extern __shared__ __align__(16) char pk_lds[];
     if (sc->done) return;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int32_t a = agg[i];
-    if (a >= 0) x[i] += scale * xc[a];
+    double inv[4];
+    pk_load_inv(P, inv);
+    pk_stage(P, pk_lds);
+    __syncthreads();
+    pk_apply(P, pk_lds, inv, b, x);
 }
 
 // One pairwise pass over a level (rp, ci, val, fixed): agg[n], *nc.
@@ -2978,7 +3013,9 @@ static int amg_build(grmp_amg *m)
             L.x = m->z;
             L.b = m->r;
         } else {
-            GRMP_TRY(amg_alloc(m, &L.x, L.n));
+            // one entry more, kept 0: what the fixed columns' cagg points to
+            GRMP_TRY(amg_alloc(m, &L.x, L.n + 1));
+            GRMP_HIP(ctx, hipMemsetAsync(L.x + L.n, 0, sizeof(double), st));
             GRMP_TRY(amg_alloc(m, &L.b, L.n));
         }
         GRMP_TRY(amg_alloc(m, &L.r, L.n));
@@ -2987,6 +3024,40 @@ static int amg_build(grmp_amg *m)
     const AmgLevel &C = m->lv[m->nlev - 1];
     GRMP_TRY(amg_alloc(m, &m->inv, C.n * C.n));
     hipLaunchKernelGGL(k_mg_dense_inv, dim3(1), dim3(256), 0, st, C.rp, C.ci, C.val, C.fixed, (int)C.n, m->inv);
+    memset(&m->pack, 0, sizeof(m->pack));
+    if (m->nlev > 1) {
+        // the most levels from the coarsest up that fit one workgroup's LDS (the coarsest always does)
+        MgPackShape sh[AMG_MAX_LEVELS];
+        for (int l = 0; l < m->nlev; ++l) sh[l] = MgPackShape{m->lv[l].n, m->lv[l].nnz, 0, 0, 1, TR_AGG};
+        m->first = 0;
+        for (int f = m->nlev - 1; f >= 1; --f) {
+            MgPack P;
+            if (!mg_pack_layout(P, sh + f, m->nlev - f)) break;
+            m->pack = P;
+            m->first = f;
+        }
+        GRMP_CHECK(ctx, m->first >= 1, GRMP_ERR_UNSUPPORTED, "AMG: the coarsest level does not fit LDS");
+        GRMP_TRY(mg_allow_lds(ctx, (const void *)k_amg_vcycle_block));
+        GRMP_TRY(amg_alloc(m, &m->img, m->pack.image));
+        m->pack.img = m->img;
+        m->pack.inv = m->inv;
+        m->pack.scale = AMG_SCALE;
+        for (int k = 0; k < m->pack.nlev; ++k) {
+            const AmgLevel &L = m->lv[m->first + k];
+            const AmgLevel *N = k + 1 < m->pack.nlev ? &m->lv[m->first + k + 1] : nullptr;
+            const MgPackSrc S{L.rp, L.ci, L.val32, L.dinv, L.lam, L.fixed, N ? L.agg : nullptr,
+                              N ? N->mptr : nullptr, N ? N->midx : nullptr, (int32_t)L.nnz,
+                              N ? (int32_t)N->n : 0};
+            const int64_t items = std::max(std::max(L.nnz, L.n + 1), N ? N->n + 1 : (int64_t)0);
+            hipLaunchKernelGGL(k_mg_pack, dim3(nblk(items, 256)), dim3(256), 0, st, m->pack.lv[k], S, m->img);
+        }
+        for (int l = 0; l < m->first; ++l) {
+            AmgLevel &L = m->lv[l];
+            GRMP_TRY(amg_alloc(m, &L.cagg, L.nnz));
+            hipLaunchKernelGGL(k_amg_cagg, dim3(nblk(L.nnz, 256)), dim3(256), 0, st, L.ci, L.agg, L.nnz,
+                               (int32_t)m->lv[l + 1].n, L.cagg);
+        }
+    }
     GRMP_HIP(ctx, hipGetLastError());
     GRMP_HIP(ctx, hipStreamSynchronize(st));
     return GRMP_OK;
@@ -3010,8 +3081,14 @@ static void amg_rows(MgRows &a, const AmgLevel &L, const grmp_amg *m)
 static void amg_vcycle(grmp_amg *m)
 {
     hipStream_t st = m->ctx->stream;
-    const int L1 = m->nlev - 1;
-    for (int l = 0; l < L1; ++l) {
+    if (m->nlev == 1) {  // z = the dense solve, partials of r.z
+        const AmgLevel &C = m->lv[0];
+        hipLaunchKernelGGL(k_mg_dense_apply, dim3(1), dim3(MG_DENSE_MAX), 0, st, m->inv, C.b, (int)C.n, C.x, m->sc);
+        hipLaunchKernelGGL(k_mg_dot, dim3(m->nb0), dim3(KB), 0, st, m->r, m->z, C.n, m->part, m->sc);
+        return;
+    }
+    const int F = m->first;
+    for (int l = 0; l < F; ++l) {
         const AmgLevel &L = m->lv[l], &C = m->lv[l + 1];
         MgRows a;
         amg_rows(a, L, m);
@@ -3027,19 +3104,23 @@ static void amg_vcycle(grmp_amg *m)
         hipLaunchKernelGGL(k_amg_restrict, dim3(nblk(C.n, 256)), dim3(256), 0, st, C.mptr, C.midx, L.r, C.fixed,
                            C.dinv, C.lam, C.b, C.d, C.n, m->sc);
     }
-    const AmgLevel &C = m->lv[L1];
-    hipLaunchKernelGGL(k_mg_dense_apply, dim3(1), dim3(MG_DENSE_MAX), 0, st, m->inv, C.b, (int)C.n, C.x, m->sc);
-    for (int l = L1 - 1; l >= 0; --l) {
-        const AmgLevel &L = m->lv[l], &Cc = m->lv[l + 1];
-        hipLaunchKernelGGL(k_amg_prolong, dim3(nblk(L.n, 256)), dim3(256), 0, st, L.agg, Cc.x, AMG_SCALE, L.x, L.n,
-                           m->sc);
+    hipLaunchKernelGGL(k_amg_vcycle_block, dim3(1), dim3(MG_BT), m->pack.lds, st, m->pack, m->lv[F].b, m->lv[F].x,
+                       m->sc);
+    for (int l = F - 1; l >= 0; --l) {
+        // the prolongation is part of the first smoothing step: A (x + e) = A x + (A P) v with the residual of x
+        // still in r, so the pass over x goes and the gathers read the coarse vector
+        const AmgLevel &L = m->lv[l], &C = m->lv[l + 1];
         MgRows a;
         amg_rows(a, L, m);
-        a.v = L.x;
-        a.b = L.b;
+        a.ci = L.cagg;
+        a.v = C.x;
+        a.b = L.r;
+        a.d = L.x;
+        a.agg = L.agg;
+        a.scale = AMG_SCALE;
         a.o1 = L.d;
         a.o2 = L.r;
-        hipLaunchKernelGGL(k_mg_rows<OP_CHEB_POST1>, dim3(nblk(L.n, KB)), dim3(KB), 0, st, a);
+        hipLaunchKernelGGL(k_mg_rows<OP_AGG_POST1>, dim3(nblk(L.n, KB)), dim3(KB), 0, st, a);
         amg_rows(a, L, m);
         a.v = L.r;
         a.b = L.b;
@@ -3047,9 +3128,6 @@ static void amg_vcycle(grmp_amg *m)
         a.o1 = L.x;
         a.part = l == 0 ? m->part : nullptr;
         hipLaunchKernelGGL(k_mg_rows<OP_CHEB_POST2>, dim3(nblk(L.n, KB)), dim3(KB), 0, st, a);
-    }
-    if (L1 == 0) {  // one level: z = the dense solve, partials of r.z
-        hipLaunchKernelGGL(k_mg_dot, dim3(m->nb0), dim3(KB), 0, st, m->r, m->z, C.n, m->part, m->sc);
     }
 }
 
