@@ -25,3 +25,46 @@ def test_coarse_end_matches_lu(grmp, O, batch):
             x = _reference(grmp, O, *spec, 40 + k)
             err = np.linalg.norm(S.solution(t) - x) / max(np.linalg.norm(x), 1e-300)
             assert r.status == 0 and r.iterations <= 40 and err <= 1e-8, (spec, r.status, r.iterations, err)
+
+
+def _fan(k):
+    """k triangles around one vertex: its row has k + 1 columns"""
+    t = 2.0 * np.pi * np.arange(k) / k
+    r = 1.0 + 0.2 * np.cos(3.0 * t)
+    coords = np.vstack([[0.03, 0.02], np.column_stack([r * np.cos(t), r * np.sin(t)])])
+    cells = np.column_stack([np.zeros(k, int), 1 + np.arange(k), 1 + (np.arange(k) + 1) % k])
+    return coords, cells
+
+
+# row widths at the pattern kernel's set sizes (32, 64, 255 columns)
+@pytest.mark.parametrize("width", [4, 31, 32, 33, 64, 65, 200, 255])
+def test_pattern_row_widths(grmp, O, width):
+    """The pattern is the oracle's exactly, and so are the values."""
+    print(f"[case] pattern of a row with {width} columns", flush=True)
+    coords, cells = _fan(width - 1)
+    grid = grmp.ExtendableGrid.from_arrays(coords, cells)
+    fes = grmp.FESpace(grmp.H1P1(1), grid)
+    A = grmp.FEMatrix([fes])
+    form, keep = grmp.LaplaceOperator(0.7).form(fes, 0, 0, fes.ctx)
+    A.add_form(form, keep)
+    A.set_fixed(np.array([1, 3]))
+    A.build_pattern()
+    A.assemble()
+    cp, rv, nz = A.csc()
+    ref = O.assemble_matrix(fes.ndofs, [dict(kind=O.BLF_LAPLACE, fe=O.FE_P1, quadorder=0, factor=0.7, coords=coords,
+                                             cells=cells, celldofs=cells)], fixed=np.array([1, 3]))
+    assert A.info()[2] == width
+    assert np.array_equal(cp, ref.colptr) and np.array_equal(rv, ref.rowval) and np.array_equal(nz, ref.nzval)
+
+
+def test_pattern_row_too_wide(grmp):
+    print("[case] pattern of a row with 256 columns", flush=True)
+    coords, cells = _fan(255)
+    grid = grmp.ExtendableGrid.from_arrays(coords, cells)
+    fes = grmp.FESpace(grmp.H1P1(1), grid)
+    A = grmp.FEMatrix([fes])
+    form, keep = grmp.LaplaceOperator(1.0).form(fes, 0, 0, fes.ctx)
+    A.add_form(form, keep)
+    with pytest.raises(grmp.GrmpError) as e:
+        A.build_pattern()
+    assert e.value.code == grmp._abi.ERR_UNSUPPORTED
