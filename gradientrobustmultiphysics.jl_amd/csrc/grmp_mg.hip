@@ -623,21 +623,6 @@ __global__ void k_mg_update_p(double *__restrict__ p, const double *__restrict__
     if (i < n) p[i] = z[i] + be * p[i];
 }
 
-// one block: the fixed-order sum of nb partials, then the scalar step
-template <int W>
-__global__ __launch_bounds__(KB) void k_mg_red(const double *__restrict__ part, int nb, const double *__restrict__ part2,
-                                               MgScal *sc)
-{
-    if (sc->done) return;
-    double a = 0.0, b = 0.0;
-    for (int k = threadIdx.x; k < nb; k += KB) {
-        a += part[k];
-        if (W == RED_INIT) b += part2[k];
-    }
-    block_sum2(a, b);
-    if (threadIdx.x == 0) mg_scalar<W>(sc, a, b);
-}
-
 // a check was requested: resume the kernels for it
 __global__ void k_mg_verify_begin(MgScal *sc)
 {
@@ -715,6 +700,35 @@ __device__ double blk_sum(double v)
 #pragma unroll
     for (int k = 0; k < MG_BT / 64; ++k) t += ws[k];
     return t;
+}
+
+// The fixed-order sum of nb partials by one workgroup of MG_BT threads, the
+// same for a request alone and in a batch.  One workgroup, so bound by the
+// latency of its loads: eight are in flight per thread, which takes the 16,385
+// partials of 4.2M rows in two rounds (256 threads with one load at a time:
+// 17 us, and three of them an iteration).
+#define MG_RED_U 8
+__device__ double red_sum(const double *__restrict__ part, int nb)
+{
+    double a = 0.0;
+    for (int k = threadIdx.x; k < nb; k += MG_RED_U * MG_BT) {
+        double v[MG_RED_U];
+#pragma unroll
+        for (int u = 0; u < MG_RED_U; ++u) v[u] = k + u * MG_BT < nb ? part[k + u * MG_BT] : 0.0;
+#pragma unroll
+        for (int u = 0; u < MG_RED_U; ++u) a += v[u];
+    }
+    return blk_sum(a);
+}
+
+// one block: the sum of the partials, then the scalar step
+template <int W>
+__global__ __launch_bounds__(MG_BT) void k_mg_red(const double *__restrict__ part, int nb,
+                                                  const double *__restrict__ part2, MgScal *sc)
+{
+    if (sc->done) return;
+    const double a = red_sum(part, nb), b = W == RED_INIT ? red_sum(part2, nb) : 0.0;
+    if (threadIdx.x == 0) mg_scalar<W>(sc, a, b);
 }
 
 // rows of level L through the epilogue OP; returns this thread's partial
@@ -1242,14 +1256,13 @@ __global__ __launch_bounds__(KB) void k_mgb_update_p(const MgTile *__restrict__ 
 
 // one block per request: the fixed-order sum of its partials, then step W
 template <int W>
-__global__ __launch_bounds__(KB) void k_mgb_red(const MgBDesc *const *__restrict__ Dp, const int32_t *__restrict__ reqs)
+__global__ __launch_bounds__(MG_BT) void k_mgb_red(const MgBDesc *const *__restrict__ Dp,
+                                                   const int32_t *__restrict__ reqs)
 {
     const MgBDesc &D = *Dp[reqs[blockIdx.x]];
     if (D.sc->done) return;
-    double a = 0.0, b = 0.0;
-    for (int k = threadIdx.x; k < D.nb0; k += KB) a += D.part[k];
-    block_sum2(a, b);
-    if (threadIdx.x == 0) mg_scalar<W>(D.sc, a, b);
+    const double a = red_sum(D.part, D.nb0);
+    if (threadIdx.x == 0) mg_scalar<W>(D.sc, a, 0.0);
 }
 
 __global__ __launch_bounds__(MG_BT) void k_mgb_vcycle_block(const MgBDesc *const *__restrict__ Dp,
@@ -1758,7 +1771,7 @@ static int mg_job_start(MgJob *j, double rtol, int maxit)
                        j->lv[0].lam, j->r, j->lv[0].d, n);
     mg_vcycle(j);
     hipLaunchKernelGGL(k_mg_dot, dim3(j->nb0), dim3(KB), 0, st, j->r, j->r, n, j->part2, j->sc);
-    hipLaunchKernelGGL(k_mg_red<RED_INIT>, dim3(1), dim3(KB), 0, st, j->part, j->nb0, j->part2, j->sc);
+    hipLaunchKernelGGL(k_mg_red<RED_INIT>, dim3(1), dim3(MG_BT), 0, st, j->part, j->nb0, j->part2, j->sc);
     hipLaunchKernelGGL(k_mg_update_p, dim3(nblk(n, 256)), dim3(256), 0, st, j->p, j->z, n, j->sc);
     GRMP_HIP(ctx, hipGetLastError());
     return GRMP_OK;
@@ -1859,12 +1872,12 @@ static int mg_iterate_grid(MgJob *j, int iters)
         a.o1 = j->q;
         a.part = j->part;
         launch_rows<OP_PCG_Q>(j, a);
-        hipLaunchKernelGGL(k_mg_red<RED_ALPHA>, dim3(1), dim3(KB), 0, j->st, j->part, j->nb0, nullptr, j->sc);
+        hipLaunchKernelGGL(k_mg_red<RED_ALPHA>, dim3(1), dim3(MG_BT), 0, j->st, j->part, j->nb0, nullptr, j->sc);
         hipLaunchKernelGGL(k_mg_axpy, dim3(j->nb0), dim3(KB), 0, j->st, j->x, j->r, j->p, j->q, L0.in.A->fixed,
                            L0.dinv, L0.lam, L0.d, n, j->part, j->sc);
-        hipLaunchKernelGGL(k_mg_red<RED_CONV>, dim3(1), dim3(KB), 0, j->st, j->part, j->nb0, nullptr, j->sc);
+        hipLaunchKernelGGL(k_mg_red<RED_CONV>, dim3(1), dim3(MG_BT), 0, j->st, j->part, j->nb0, nullptr, j->sc);
         mg_vcycle(j);
-        hipLaunchKernelGGL(k_mg_red<RED_BETA>, dim3(1), dim3(KB), 0, j->st, j->part, j->nb0, nullptr, j->sc);
+        hipLaunchKernelGGL(k_mg_red<RED_BETA>, dim3(1), dim3(MG_BT), 0, j->st, j->part, j->nb0, nullptr, j->sc);
         hipLaunchKernelGGL(k_mg_update_p, dim3(nblk(n, 256)), dim3(256), 0, j->st, j->p, j->z, n, j->sc);
     }
     GRMP_HIP(j->ctx, hipGetLastError());
@@ -1902,9 +1915,9 @@ int mg_job_verify(MgJob *j)
     a.o2 = L0.d;
     launch_rows<OP_TRUE_RESID>(j, a, L0.nnz);
     hipLaunchKernelGGL(k_mg_dot, dim3(j->nb0), dim3(KB), 0, j->st, j->r, j->r, n, j->part, j->sc);
-    hipLaunchKernelGGL(k_mg_red<RED_VERIFY>, dim3(1), dim3(KB), 0, j->st, j->part, j->nb0, nullptr, j->sc);
+    hipLaunchKernelGGL(k_mg_red<RED_VERIFY>, dim3(1), dim3(MG_BT), 0, j->st, j->part, j->nb0, nullptr, j->sc);
     mg_vcycle(j);
-    hipLaunchKernelGGL(k_mg_red<RED_RESTART>, dim3(1), dim3(KB), 0, j->st, j->part, j->nb0, nullptr, j->sc);
+    hipLaunchKernelGGL(k_mg_red<RED_RESTART>, dim3(1), dim3(MG_BT), 0, j->st, j->part, j->nb0, nullptr, j->sc);
     hipLaunchKernelGGL(k_mg_update_p, dim3(nblk(n, 256)), dim3(256), 0, j->st, j->p, j->z, n, j->sc);
     GRMP_HIP(j->ctx, hipGetLastError());
     return GRMP_OK;
@@ -2103,9 +2116,9 @@ int mg_batch_run(MgBatch *b, MgJob *const *jobs, int n, int iters)
     for (int k = 0; k < iters && ng > 0; ++k) {
         const MgSeg &L0 = lev[0];
         hipLaunchKernelGGL(k_mgb_rows<OP_PCG_Q>, dim3(ublk(L0.cnt)), dim3(KB), 0, st, tiles(L0), D);
-        hipLaunchKernelGGL(k_mgb_red<RED_ALPHA>, dim3(ng), dim3(KB), 0, st, D, G);
+        hipLaunchKernelGGL(k_mgb_red<RED_ALPHA>, dim3(ng), dim3(MG_BT), 0, st, D, G);
         hipLaunchKernelGGL(k_mgb_axpy, dim3(ublk(L0.cnt)), dim3(KB), 0, st, tiles(L0), D);
-        hipLaunchKernelGGL(k_mgb_red<RED_CONV>, dim3(ng), dim3(KB), 0, st, D, G);
+        hipLaunchKernelGGL(k_mgb_red<RED_CONV>, dim3(ng), dim3(MG_BT), 0, st, D, G);
         for (int l = 0; l < Fmax; ++l) {
             if (lev[l].cnt == 0) continue;
             hipLaunchKernelGGL(k_mgb_rows<OP_CHEB_PRE>, dim3(ublk(lev[l].cnt)), dim3(KB), 0, st, tiles(lev[l]), D);
@@ -2134,7 +2147,7 @@ int mg_batch_run(MgBatch *b, MgJob *const *jobs, int n, int iters)
             hipLaunchKernelGGL(k_mgb_rows<OP_CHEB_POST1>, dim3(ublk(lev[l].cnt)), dim3(KB), 0, st, tiles(lev[l]), D);
             hipLaunchKernelGGL(k_mgb_rows<OP_CHEB_POST2>, dim3(ublk(lev[l].cnt)), dim3(KB), 0, st, tiles(lev[l]), D);
         }
-        hipLaunchKernelGGL(k_mgb_red<RED_BETA>, dim3(ng), dim3(KB), 0, st, D, G);
+        hipLaunchKernelGGL(k_mgb_red<RED_BETA>, dim3(ng), dim3(MG_BT), 0, st, D, G);
         hipLaunchKernelGGL(k_mgb_update_p, dim3(ublk(L0.cnt)), dim3(KB), 0, st, tiles(L0), D);
     }
     if (nbk > 0) hipLaunchKernelGGL(k_mgb_pcg_block, dim3(nbk), dim3(MG_BT), lds_blk, st, D, Bk, iters);
@@ -3143,12 +3156,12 @@ static void amg_iterate(grmp_amg *m, int iters)
         a.o1 = m->q;
         a.part = m->part;
         hipLaunchKernelGGL(k_mg_rows<OP_PCG_Q>, dim3(nblk(n, KB)), dim3(KB), 0, st, a);
-        hipLaunchKernelGGL(k_mg_red<RED_ALPHA>, dim3(1), dim3(KB), 0, st, m->part, m->nb0, nullptr, m->sc);
+        hipLaunchKernelGGL(k_mg_red<RED_ALPHA>, dim3(1), dim3(MG_BT), 0, st, m->part, m->nb0, nullptr, m->sc);
         hipLaunchKernelGGL(k_mg_axpy, dim3(m->nb0), dim3(KB), 0, st, m->x, m->r, m->p, m->q, L0.fixed, L0.dinv, L0.lam,
                            L0.d, n, m->part, m->sc);
-        hipLaunchKernelGGL(k_mg_red<RED_CONV>, dim3(1), dim3(KB), 0, st, m->part, m->nb0, nullptr, m->sc);
+        hipLaunchKernelGGL(k_mg_red<RED_CONV>, dim3(1), dim3(MG_BT), 0, st, m->part, m->nb0, nullptr, m->sc);
         amg_vcycle(m);
-        hipLaunchKernelGGL(k_mg_red<RED_BETA>, dim3(1), dim3(KB), 0, st, m->part, m->nb0, nullptr, m->sc);
+        hipLaunchKernelGGL(k_mg_red<RED_BETA>, dim3(1), dim3(MG_BT), 0, st, m->part, m->nb0, nullptr, m->sc);
         hipLaunchKernelGGL(k_mg_update_p, dim3(nblk(n, 256)), dim3(256), 0, st, m->p, m->z, n, m->sc);
     }
 }
@@ -3168,9 +3181,9 @@ static void amg_verify(grmp_amg *m)
     a.o2 = L0.d;
     hipLaunchKernelGGL(k_mg_rows<OP_TRUE_RESID>, dim3(nblk(n, KB)), dim3(KB), 0, st, a);
     hipLaunchKernelGGL(k_mg_dot, dim3(m->nb0), dim3(KB), 0, st, m->r, m->r, n, m->part, m->sc);
-    hipLaunchKernelGGL(k_mg_red<RED_VERIFY>, dim3(1), dim3(KB), 0, st, m->part, m->nb0, nullptr, m->sc);
+    hipLaunchKernelGGL(k_mg_red<RED_VERIFY>, dim3(1), dim3(MG_BT), 0, st, m->part, m->nb0, nullptr, m->sc);
     amg_vcycle(m);
-    hipLaunchKernelGGL(k_mg_red<RED_RESTART>, dim3(1), dim3(KB), 0, st, m->part, m->nb0, nullptr, m->sc);
+    hipLaunchKernelGGL(k_mg_red<RED_RESTART>, dim3(1), dim3(MG_BT), 0, st, m->part, m->nb0, nullptr, m->sc);
     hipLaunchKernelGGL(k_mg_update_p, dim3(nblk(n, 256)), dim3(256), 0, st, m->p, m->z, n, m->sc);
 }
 
@@ -3287,7 +3300,7 @@ extern "C" int grmp_amg_apply(grmp_amg *m, const grmp_vector *b, grmp_vector *x,
         hipLaunchKernelGGL(k_mg_rows<OP_TRUE_RESID>, dim3(nblk(n, KB)), dim3(KB), 0, st, a);
         amg_vcycle(m);
         hipLaunchKernelGGL(k_mg_dot, dim3(m->nb0), dim3(KB), 0, st, m->r, m->r, n, m->part2, m->sc);
-        hipLaunchKernelGGL(k_mg_red<RED_INIT>, dim3(1), dim3(KB), 0, st, m->part, m->nb0, m->part2, m->sc);
+        hipLaunchKernelGGL(k_mg_red<RED_INIT>, dim3(1), dim3(MG_BT), 0, st, m->part, m->nb0, m->part2, m->sc);
         hipLaunchKernelGGL(k_mg_update_p, dim3(nblk(n, 256)), dim3(256), 0, st, m->p, m->z, n, m->sc);
         amg_iterate(m, 4);
         if ((rc = amg_status(m))) break;
