@@ -21,6 +21,7 @@
 #include <type_traits>
 
 #include "grmp_internal.h"
+#include "grmp_rowset.h"
 
 #pragma clang fp contract(off)
 
@@ -704,39 +705,6 @@ using K_NLDIFF_P2 = Kind<6, row_nldiff_tri<2>>;
     }
 
 // ---------------------------------------------------------------- pattern
-// Per-thread sorted column set in LDS (layout set[k*B + tid]).
-template <int B>
-__device__ __forceinline__ bool set_insert(int32_t *set, int &n, int rmax, int32_t c)
-{
-    const int t = threadIdx.x;
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        int mid = (lo + hi) >> 1;
-        int32_t v = set[mid * B + t];
-        if (v < c) lo = mid + 1;
-        else hi = mid;
-    }
-    if (lo < n && set[lo * B + t] == c) return true;
-    if (n >= rmax) return false;
-    for (int k = n; k > lo; --k) set[k * B + t] = set[(k - 1) * B + t];
-    set[lo * B + t] = c;
-    ++n;
-    return true;
-}
-
-template <int B>
-__device__ __forceinline__ int set_find(const int32_t *set, int n, int32_t c)
-{
-    const int t = threadIdx.x;
-    int lo = 0, hi = n;
-    while (lo < hi) {
-        int mid = (lo + hi) >> 1;
-        if (set[mid * B + t] < c) lo = mid + 1;
-        else hi = mid;
-    }
-    return lo;
-}
-
 // Collects the columns with a nonzero local value of row i of form F, and
 // leaves in the slot map which local values are zero (byte 255) and which are
 // not (byte 0).  Kinds with a gather step keep K::ROW_NB cells' loads in

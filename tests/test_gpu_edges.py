@@ -68,3 +68,32 @@ def test_pattern_row_too_wide(grmp):
     with pytest.raises(grmp.GrmpError) as e:
         A.build_pattern()
     assert e.value.code == grmp._abi.ERR_UNSUPPORTED
+
+
+# coarse rows of the Galerkin product at its set sizes: aggregated pairs halve
+# a hub's columns (24 and 42 of 48 and 84, 125 of 250); three hubs in one
+# aggregate have about 376, more than a set holds
+@pytest.mark.parametrize("hubs,k", [(1, 48), (1, 84), (1, 250), (3, 250)])
+def test_amg_wide_coarse_rows(grmp, hubs, k):
+    """1e-8 against LU: the residual is 1e-12, the condition below 1e4"""
+    print(f"[case] algebraic multigrid, {hubs} hub(s) of {k} cells", flush=True)
+    import scipy.sparse.linalg as spla
+    co, ce = [], []
+    for h in range(hubs):
+        c, e = _fan(k)
+        t = 2.0 * np.pi * h / 3.0
+        co.append(c + 5.0 * np.array([np.cos(t), np.sin(t)]))
+        ce.append(e + h * (k + 1))
+    if hubs == 3:
+        ce.append(np.array([[0, k + 1, 2 * (k + 1)]]))
+    grid = grmp.ExtendableGrid.from_arrays(np.vstack(co), np.vstack(ce))
+    fes = grmp.FESpace(grmp.H1P1(1), grid)
+    pde = grmp.PoissonProblem(1.0)
+    pde.add_operator((0, 0), grmp.ReactionOperator(0.01))
+    pde.add_rhsdata(0, grmp.LinearForm(grmp.Identity, grmp.DataFunction([1.0])))
+    pde.add_rhsdata(0, grmp.LinearForm(grmp.Identity, grmp.PolynomialData([0.0, 1.0, -0.5])))
+    sol = grmp.FEVector([fes])
+    info, A, b = grmp.solve(sol, pde, solver="amg", rtol=1e-12)
+    x = spla.spsolve(A.to_scipy().tocsc(), b.entries())
+    err = np.linalg.norm(sol.entries() - x) / np.linalg.norm(x)
+    assert info.status == 0 and err <= 1e-8, (info.iterations, err)
