@@ -1524,23 +1524,39 @@ extern "C" int grmp_matrix_add_form(grmp_matrix *A, const grmp_form *form)
     return GRMP_OK;
 }
 
+__global__ void k_fixed_mask(const int64_t *__restrict__ fixed, int64_t cnt, uint8_t *__restrict__ mask)
+{
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < cnt) mask[fixed[k] - 1] = 1;
+}
+
+// the mask is set on the device from the list: the boundary's dofs travel, not
+// a byte for every row
 extern "C" int grmp_matrix_set_fixed(grmp_matrix *A, int64_t nfixed, const int64_t *fixed, double penalty)
 {
     if (!A || nfixed < 0 || (nfixed && !fixed)) return GRMP_ERR_ARG;
     grmp_ctx *ctx = A->ctx;
-    std::vector<uint8_t> mask(A->n, 0);
-    for (int64_t k = 0; k < nfixed; ++k) {
+    for (int64_t k = 0; k < nfixed; ++k)
         GRMP_CHECK(ctx, fixed[k] >= 1 && fixed[k] <= A->n, GRMP_ERR_ARG, "grmp_matrix_set_fixed: dof %lld out of range",
                    (long long)fixed[k]);
-        mask[fixed[k] - 1] = 1;
-    }
     std::lock_guard<std::mutex> g(ctx->mu);
     matrix_free_pattern(A);
     A->fixed_host.assign(fixed, fixed + nfixed);
     A->penalty = penalty;
     if (!A->fixed) GRMP_TRY(dalloc(ctx, &A->fixed, A->n));
-    GRMP_HIP(ctx, hipMemcpyAsync(A->fixed, mask.data(), A->n, hipMemcpyHostToDevice, ctx->stream));
-    GRMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    GRMP_HIP(ctx, hipMemsetAsync(A->fixed, 0, A->n, ctx->stream));
+    if (nfixed == 0) return GRMP_OK;
+    int64_t *d = nullptr;
+    GRMP_TRY(dalloc(ctx, &d, nfixed));
+    hipError_t e = hipMemcpyAsync(d, fixed, sizeof(int64_t) * nfixed, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_fixed_mask, dim3(nblk(nfixed, 256)), dim3(256), 0, ctx->stream, d, nfixed, A->fixed);
+        e = hipGetLastError();
+    }
+    const hipError_t e2 = hipStreamSynchronize(ctx->stream);  // the caller's list is borrowed for the call
+    dfree(ctx, d);
+    GRMP_HIP(ctx, e);
+    GRMP_HIP(ctx, e2);
     return GRMP_OK;
 }
 
@@ -1548,10 +1564,12 @@ extern "C" int grmp_matrix_set_fixed(grmp_matrix *A, int64_t nfixed, const int64
 // returns the device pack of block row rb
 // the pattern pass uploads Newton forms without their iterate: every local
 // pair then enters the pattern, whatever the iterate's values
-static int upload_forms(grmp_matrix *A, bool pattern, std::vector<DevForm> *host = nullptr)
+static int upload_forms(grmp_matrix *A, bool pattern)
 {
     grmp_ctx *ctx = A->ctx;
-    std::vector<DevForm> h;
+    std::vector<DevForm> &h = A->hforms;
+    if (!h.empty()) GRMP_HIP(ctx, hipStreamSynchronize(ctx->stream));  // an earlier copy may still read it
+    h.clear();
     A->form_first.assign(A->nblocks + 1, 0);
     for (int rb = 0; rb < A->nblocks; ++rb) {
         A->form_first[rb] = (int)h.size();
@@ -1566,9 +1584,6 @@ static int upload_forms(grmp_matrix *A, bool pattern, std::vector<DevForm> *host
     A->form_first[A->nblocks] = (int)h.size();
     if (!A->dforms) GRMP_TRY(dalloc(ctx, &A->dforms, A->nblocks * MAXFORMS));
     GRMP_HIP(ctx, hipMemcpyAsync(A->dforms, h.data(), sizeof(DevForm) * h.size(), hipMemcpyHostToDevice, ctx->stream));
-    // the copy source is a host vector: finish it before returning
-    GRMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    if (host) *host = std::move(h);
     return GRMP_OK;
 }
 
@@ -1581,7 +1596,7 @@ static FormPack row_block_pack(const grmp_matrix *A, int rb)
 }
 
 template <int B, int RMAX>
-static int pattern_pass(grmp_matrix *A, const std::vector<DevForm> &hf, int32_t *count)
+static int pattern_pass(grmp_matrix *A, int32_t *count)
 {
     grmp_ctx *ctx = A->ctx;
     for (int rb = 0; rb < A->nblocks; ++rb) {
@@ -1591,7 +1606,7 @@ static int pattern_pass(grmp_matrix *A, const std::vector<DevForm> &hf, int32_t 
         const dim3 grid(nblk(g1 - g0, B)), blk(B);
         bool done = false;
         if (P.n == 1) {
-            const DevForm F = hf[A->form_first[rb]];
+            const DevForm F = A->hforms[A->form_first[rb]];
             GRMP_DISPATCH(F, hipLaunchKernelGGL((k_pattern<KT, B, RMAX>), grid, blk, 0, ctx->stream, P, g0, g1, g0,
                                                 A->fixed, count, A->diagpos, ctx->dflag);
                           done = true);
@@ -1616,46 +1631,45 @@ extern "C" int grmp_matrix_build_pattern(grmp_matrix *A)
         GRMP_HIP(ctx, hipMemsetAsync(A->fixed, 0, A->n, ctx->stream));
     }
     for (auto &r : A->forms) GRMP_TRY(dalloc(ctx, &r.pos, (size_t)r.rs->mesh->ncells * r.rs->nloc * r.words));
-    std::vector<DevForm> hf;
-    GRMP_TRY(upload_forms(A, true, &hf));
-    int32_t *count = nullptr;
-    GRMP_TRY(dalloc(ctx, &count, A->n));
+    GRMP_TRY(upload_forms(A, true));
+    struct Count {
+        grmp_ctx *ctx;
+        int32_t *d = nullptr;
+        int64_t *total = nullptr;
+        ~Count()
+        {
+            dfree(ctx, d);
+            dfree(ctx, total);
+        }
+    } C{ctx};
+    GRMP_TRY(dalloc(ctx, &C.d, A->n));
+    GRMP_TRY(dalloc(ctx, &C.total, 1));
     GRMP_TRY(dalloc(ctx, &A->rowptr, A->n + 1));
     GRMP_TRY(dalloc(ctx, &A->diagpos, A->n));
-    int flags[2] = {0, 0};
-    int big = 0;
     // rows of up to 32 columns (every P1 and P2 pattern of a regular mesh) leave 20 waves' sets in a CU's LDS,
     // longer ones 10; the last pass takes the slot map's 255
-    for (;; ++big) {
+    int *flags = reinterpret_cast<int *>(ctx->pin);
+    int64_t *total = reinterpret_cast<int64_t *>(ctx->pin + 64);
+    for (int big = 0;; ++big) {
         GRMP_HIP(ctx, hipMemsetAsync(ctx->dflag, 0, 2 * sizeof(int), ctx->stream));
-        if (big == 0) GRMP_TRY((pattern_pass<64, 32>(A, hf, count)));
-        else if (big == 1) GRMP_TRY((pattern_pass<64, 64>(A, hf, count)));
-        else GRMP_TRY((pattern_pass<64, 255>(A, hf, count)));
+        if (big == 0) GRMP_TRY((pattern_pass<64, 32>(A, C.d)));
+        else if (big == 1) GRMP_TRY((pattern_pass<64, 64>(A, C.d)));
+        else GRMP_TRY((pattern_pass<64, 255>(A, C.d)));
+        // the row pointers are int32: the total is checked in 64 bits before the scan
+        GRMP_TRY(sum_i32_as_i64(ctx, C.d, A->n, C.total));
         GRMP_HIP(ctx, hipMemcpyAsync(flags, ctx->dflag, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+        GRMP_HIP(ctx, hipMemcpyAsync(total, C.total, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream));
         GRMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (!flags[0]) break;
-        if (big == 2) {
-            dfree(ctx, count);
-            return grmp_fail(ctx, GRMP_ERR_UNSUPPORTED, "grmp_matrix_build_pattern: a row has more than 255 entries");
-        }
+        GRMP_CHECK(ctx, big < 2, GRMP_ERR_UNSUPPORTED, "grmp_matrix_build_pattern: a row has more than 255 entries");
     }
     A->max_row = flags[1];
-    // the row pointers are int32: check the total in 64 bits before the scan
-    int64_t total = 0;
-    int rc64 = sum_i32_as_i64(ctx, count, A->n, &total);
     const int64_t limit = std::min<int64_t>(GRMP_MAX_NNZ, ctx->max_nnz);
-    if (!rc64 && total > limit)
-        rc64 = grmp_fail(ctx, GRMP_ERR_UNSUPPORTED, "grmp_matrix_build_pattern: %lld nonzeros exceed the limit %lld "
-                         "(int32 CSR: %lld)", (long long)total, (long long)limit, (long long)GRMP_MAX_NNZ);
-    if (rc64) {
-        dfree(ctx, count);
-        return rc64;
-    }
-    GRMP_TRY(exclusive_scan_i32(ctx, count, A->rowptr, A->n));
-    int32_t nnz32 = 0;
-    GRMP_HIP(ctx, hipMemcpyAsync(&nnz32, A->rowptr + A->n, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
-    GRMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    A->nnz = nnz32;
+    GRMP_CHECK(ctx, *total <= limit, GRMP_ERR_UNSUPPORTED,
+               "grmp_matrix_build_pattern: %lld nonzeros exceed the limit %lld (int32 CSR: %lld)", (long long)*total,
+               (long long)limit, (long long)GRMP_MAX_NNZ);
+    GRMP_TRY(exclusive_scan_i32(ctx, C.d, A->rowptr, A->n));
+    A->nnz = *total;
     GRMP_TRY(dalloc(ctx, &A->cols, A->nnz));
     for (int rb = 0; rb < A->nblocks; ++rb) {
         const int64_t g0 = A->offs[rb], g1 = A->offs[rb + 1];
@@ -1664,8 +1678,6 @@ extern "C" int grmp_matrix_build_pattern(grmp_matrix *A)
                            g0, g1, g0, A->fixed, A->rowptr, A->diagpos, A->cols);
         GRMP_HIP(ctx, hipGetLastError());
     }
-    GRMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    dfree(ctx, count);
     A->have_pattern = true;
     return GRMP_OK;
 }
@@ -1701,18 +1713,8 @@ extern "C" int grmp_matrix_assemble(grmp_matrix *A, int values)
             for (auto &r : A->forms)
                 if (r.f.row_block == rb) fill_devform(A, r, hf[k++]);
     }
-    // the event pair lives until the function returns, whatever the path
-    struct EventPair {
-        hipEvent_t a = nullptr, b = nullptr;
-        ~EventPair()
-        {
-            if (a) (void)hipEventDestroy(a);
-            if (b) (void)hipEventDestroy(b);
-        }
-    } ev;
-    GRMP_HIP(ctx, hipEventCreate(&ev.a));
-    GRMP_HIP(ctx, hipEventCreate(&ev.b));
-    GRMP_HIP(ctx, hipEventRecord(ev.a, ctx->stream));
+    hipEvent_t *ev = ctx->asm_ev;
+    GRMP_HIP(ctx, hipEventRecord(ev[0], ctx->stream));
     for (int rb = 0; rb < A->nblocks; ++rb) {
         FormPack P = row_block_pack(A, rb);
         int64_t g0 = A->offs[rb], g1 = A->offs[rb + 1];
@@ -1723,9 +1725,9 @@ extern "C" int grmp_matrix_assemble(grmp_matrix *A, int values)
                         (values & GRMP_VALUES_FP32) ? A->val32 : nullptr, A->dinv64, A->dinv32, ctx->stream);
         GRMP_HIP(ctx, hipGetLastError());
     }
-    GRMP_HIP(ctx, hipEventRecord(ev.b, ctx->stream));
-    GRMP_HIP(ctx, hipEventSynchronize(ev.b));
-    GRMP_HIP(ctx, hipEventElapsedTime(&A->last_asm_ms, ev.a, ev.b));
+    GRMP_HIP(ctx, hipEventRecord(ev[1], ctx->stream));
+    GRMP_HIP(ctx, hipEventSynchronize(ev[1]));
+    GRMP_HIP(ctx, hipEventElapsedTime(&A->last_asm_ms, ev[0], ev[1]));
     A->values |= values;
     return GRMP_OK;
 }
@@ -1838,7 +1840,7 @@ int assemble_batch(grmp_ctx *ctx, hipStream_t st, const AsmBatchItem *items, int
                "batched assembly: rows of %d entries exceed a tile's LDS (at most 32)", maxrow);
     const size_t bi = sizeof(AsmItemDev) * hi.size(), bt = sizeof(AsmTile) * ht.size();
     char *dbuf = nullptr;
-    GRMP_HIP(ctx, hipMallocAsync((void **)&dbuf, bi + bt, st));
+    GRMP_HIP(ctx, ctx_malloc(ctx, (void **)&dbuf, bi + bt, st));
     hipError_t e = hipMemcpyAsync(dbuf, hi.data(), bi, hipMemcpyHostToDevice, st);
     if (e == hipSuccess) e = hipMemcpyAsync(dbuf + bi, ht.data(), bt, hipMemcpyHostToDevice, st);
     const int ntiles = (int)ht.size();

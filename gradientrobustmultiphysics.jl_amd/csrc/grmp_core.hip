@@ -41,7 +41,7 @@ int ensure_scratch(grmp_ctx *ctx, size_t bytes)
     if (ctx->scratch) GRMP_HIP(ctx, hipFreeAsync(ctx->scratch, ctx->stream));
     ctx->scratch = nullptr;
     size_t nb = bytes + bytes / 2 + 4096;
-    GRMP_HIP(ctx, hipMallocAsync(&ctx->scratch, nb, ctx->stream));
+    GRMP_HIP(ctx, ctx_malloc(ctx, &ctx->scratch, nb, ctx->stream));
     ctx->scratch_bytes = nb;
     return GRMP_OK;
 }
@@ -140,10 +140,24 @@ extern "C" int grmp_ctx_create(int device, grmp_ctx **out)
         delete c;
         return GRMP_ERR_HIP;
     }
-    if (hipMalloc(&c->dflag, 64) != hipSuccess) {
-        (void)hipStreamDestroy(c->stream);
-        delete c;
+    if (hipMalloc(&c->dflag, 64) != hipSuccess ||
+        hipHostMalloc((void **)&c->pin, GRMP_PIN_BYTES, hipHostMallocDefault) != hipSuccess ||
+        hipEventCreate(&c->asm_ev[0]) != hipSuccess || hipEventCreate(&c->asm_ev[1]) != hipSuccess) {
+        grmp_ctx_destroy(c);
         return GRMP_ERR_OOM;
+    }
+    hipMemPoolProps props;
+    memset(&props, 0, sizeof(props));
+    props.allocType = hipMemAllocationTypePinned;
+    props.location.type = hipMemLocationTypeDevice;
+    props.location.id = device;
+    size_t mfree = 0, mtotal = 0;
+    if (hipMemPoolCreate(&c->pool, &props) == hipSuccess) {
+        uint64_t keep = hipMemGetInfo(&mfree, &mtotal) == hipSuccess ? mtotal / 32 : 0;
+        (void)hipMemPoolSetAttribute(c->pool, hipMemPoolAttrReleaseThreshold, &keep);
+    } else {
+        c->pool = nullptr;  // the default pool then
+        (void)hipGetLastError();
     }
     // the shipped tuning table, when present (a missing file keeps the built-in launch shapes)
     const std::string fn = tune_default_path();
@@ -160,8 +174,13 @@ extern "C" int grmp_ctx_destroy(grmp_ctx *ctx)
     if (!ctx) return GRMP_OK;
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
-    if (ctx->scratch) (void)hipFree(ctx->scratch);
+    if (ctx->scratch) (void)hipFreeAsync(ctx->scratch, ctx->stream);
     if (ctx->dflag) (void)hipFree(ctx->dflag);
+    if (ctx->pin) (void)hipHostFree(ctx->pin);
+    for (hipEvent_t e : ctx->asm_ev)
+        if (e) (void)hipEventDestroy(e);
+    (void)hipStreamSynchronize(ctx->stream);
+    if (ctx->pool) (void)hipMemPoolDestroy(ctx->pool);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return GRMP_OK;
@@ -200,17 +219,13 @@ int exclusive_scan_i32(grmp_ctx *ctx, const int32_t *in, int32_t *out, int64_t n
 
 int sum_i32_as_i64(grmp_ctx *ctx, const int32_t *in, int64_t n, int64_t *total)
 {
-    int64_t *d = nullptr;
-    GRMP_TRY(dalloc(ctx, &d, 1));
     size_t tmp = 0;
-    hipError_t e = rocprim::reduce(nullptr, tmp, in, d, (int64_t)0, (size_t)n, rocprim::plus<int64_t>(), ctx->stream);
-    int rc = e == hipSuccess ? ensure_scratch(ctx, tmp) : GRMP_ERR_HIP;
-    if (!rc) e = rocprim::reduce(ctx->scratch, tmp, in, d, (int64_t)0, (size_t)n, rocprim::plus<int64_t>(), ctx->stream);
-    if (!rc && e == hipSuccess) e = hipMemcpyAsync(total, d, sizeof(int64_t), hipMemcpyDeviceToHost, ctx->stream);
-    if (!rc && e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
-    dfree(ctx, d);
-    if (!rc && e != hipSuccess) rc = grmp_fail(ctx, GRMP_ERR_HIP, "64-bit sum: %s", hipGetErrorString(e));
-    return rc;
+    GRMP_HIP(ctx, rocprim::reduce(nullptr, tmp, in, total, (int64_t)0, (size_t)n, rocprim::plus<int64_t>(),
+                                  ctx->stream));
+    GRMP_TRY(ensure_scratch(ctx, tmp));
+    GRMP_HIP(ctx, rocprim::reduce(ctx->scratch, tmp, in, total, (int64_t)0, (size_t)n, rocprim::plus<int64_t>(),
+                                  ctx->stream));
+    return GRMP_OK;
 }
 
 // ------------------------------------------ sorts and run sums (rocPRIM)
@@ -1211,6 +1226,13 @@ static int boundary_dofs_faces(grmp_ctx *ctx, const grmp_space *s, int64_t *coun
     return rc;
 }
 
+// boundary nodes of the generated unit square in ascending order
+static void square_boundary(int64_t N, std::vector<int64_t> &b)
+{
+    for (int64_t j = 0; j <= N; ++j)
+        for (int64_t i = 0; i <= N; i += (j == 0 || j == N) ? 1 : N) b.push_back(j * (N + 1) + i);
+}
+
 extern "C" int grmp_space_boundary_dofs(const grmp_space *s, int64_t *count, int64_t *out)
 {
     if (!s || !count) return GRMP_ERR_ARG;
@@ -1232,9 +1254,7 @@ extern "C" int grmp_space_boundary_dofs(const grmp_space *s, int64_t *count, int
     if (m->kind == MESH_UNITSQUARE && s->fe == GRMP_FE_H1BR) {
         // BFaceDofs "N1i1": both components of boundary nodes, and the bubble of each boundary face
         std::vector<int64_t> nodes;
-        for (int64_t j = 0; j <= N; ++j)
-            for (int64_t i = 0; i <= N; ++i)
-                if (i == 0 || j == 0 || i == N || j == N) nodes.push_back(j * n1 + i);
+        square_boundary(N, nodes);
         for (int64_t v : nodes) {
             b.push_back(v);
             b.push_back(v + m->nnodes);
@@ -1254,9 +1274,7 @@ extern "C" int grmp_space_boundary_dofs(const grmp_space *s, int64_t *count, int
         return GRMP_OK;
     }
     if (m->kind == MESH_UNITSQUARE) {
-        for (int64_t j = 0; j <= N; ++j)
-            for (int64_t i = 0; i <= N; ++i)
-                if (i == 0 || j == 0 || i == N || j == N) b.push_back(j * n1 + i);
+        square_boundary(N, b);
         if (s->fe == GRMP_FE_H1P2) {
             for (int64_t i = 0; i < N; ++i) {
                 b.push_back(m->nnodes + sq_H(N, i, 0));
@@ -1269,9 +1287,10 @@ extern "C" int grmp_space_boundary_dofs(const grmp_space *s, int64_t *count, int
         }
     } else {
         for (int64_t k = 0; k <= N; ++k)
-            for (int64_t j = 0; j <= N; ++j)
-                for (int64_t i = 0; i <= N; ++i)
-                    if (i == 0 || j == 0 || k == 0 || i == N || j == N || k == N) b.push_back((k * n1 + j) * n1 + i);
+            for (int64_t j = 0; j <= N; ++j) {  // whole lines on the outer faces, their two ends inside
+                const bool face = j == 0 || k == 0 || j == N || k == N;
+                for (int64_t i = 0; i <= N; i += face ? 1 : N) b.push_back((k * n1 + j) * n1 + i);
+            }
     }
     int64_t per = s->ndofs / s->ncomp;
     size_t nb = b.size();

@@ -1583,7 +1583,7 @@ int mg_job_create(grmp_ctx *ctx, hipStream_t st, const MgLevelIn *in, int nlev, 
         j->lv[l].nc = in[l].sp->mesh->ncells;
     }
     j->bytes = mg_layout(j, false);
-    hipError_t e = hipMallocAsync((void **)&j->buf, j->bytes, st);
+    hipError_t e = ctx_malloc(ctx, (void **)&j->buf, j->bytes, st);
     if (e != hipSuccess) {
         delete j;
         return grmp_fail(ctx, e == hipErrorOutOfMemory ? GRMP_ERR_OOM : GRMP_ERR_HIP, "multigrid: device buffer");
@@ -2031,7 +2031,7 @@ static int batch_reserve(MgBatch *b, size_t tiles, int reqs)
         }
         b->dtiles = nullptr;
         b->htiles = nullptr;
-        GRMP_HIP(ctx, hipMallocAsync((void **)&b->dtiles, cap * sizeof(MgTile), b->st));
+        GRMP_HIP(ctx, ctx_malloc(ctx, (void **)&b->dtiles, cap * sizeof(MgTile), b->st));
         GRMP_HIP(ctx, hipHostMalloc((void **)&b->htiles, cap * sizeof(MgTile), hipHostMallocDefault));
         b->tcap = cap;
     }

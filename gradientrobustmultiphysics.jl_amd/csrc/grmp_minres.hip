@@ -458,18 +458,13 @@ int minres_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solve_
         if ((rc = dalloc(ctx, &H.dS, 1))) break;
         if ((rc = dalloc(ctx, &H.part, MR_GRID))) break;
         if ((rc = dalloc(ctx, &dsg, n))) break;
-        if (hipHostMalloc((void **)&H.hS, sizeof(MrScal), hipHostMallocDefault) != hipSuccess) {
-            rc = grmp_fail(ctx, GRMP_ERR_HIP, "MINRES: pinned status allocation failed");
-            break;
-        }
+        H.hS = reinterpret_cast<MrScal *>(ctx->pin);
         if (ir) {
             if ((rc = dalloc(ctx, &dsg32, n))) break;
             if ((rc = dalloc(ctx, &dx, n))) break;
             if ((rc = dalloc(ctx, &r64, n))) break;
-            if (hipHostMalloc((void **)&hres, sizeof(double) * MR_GRID, hipHostMallocDefault) != hipSuccess) {
-                rc = grmp_fail(ctx, GRMP_ERR_HIP, "MINRES: pinned allocation failed");
-                break;
-            }
+            static_assert(1024 + sizeof(double) * MR_GRID <= GRMP_PIN_BYTES && sizeof(MrScal) <= 1024, "pinned scratch");
+            hres = reinterpret_cast<double *>(ctx->pin + 1024);
         }
         hipLaunchKernelGGL(k_mr_diag, dim3(nblk(n, 256)), dim3(256), 0, H.st, A->rowptr, A->cols, A->val64, A->fixed,
                            A->dinv64, dsg, dsg32, n);
@@ -531,8 +526,6 @@ int minres_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solve_
     info.outer = outer;
     info.relres = relres;
     info.status = rc ? rc : status;
-    if (H.hS) (void)hipHostFree(H.hS);
-    if (hres) (void)hipHostFree(hres);
     dfree(ctx, H.dS);
     dfree(ctx, H.part);
     dfree(ctx, dsg);

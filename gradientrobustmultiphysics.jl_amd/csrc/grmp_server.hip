@@ -267,7 +267,7 @@ static int job_start(grmp_server *S, Job *j)
     size_t o_k = take(nc * 8), o_v64 = take(nnz * 8), o_v32 = take(nnz * 4), o_d64 = take(n * 8), o_d32 = take(n * 4);
     size_t o_b = take(n * 8), o_x = take(n * 8), o_r = take(n * 8), o_f = take(4 * n * 4), o_df = take(sizeof(DevForm) * 4);
     j->dbytes = off;
-    GRMP_HIP(c, hipMallocAsync((void **)&j->dbuf, off, st));
+    GRMP_HIP(c, ctx_malloc(c, (void **)&j->dbuf, off, st));
     j->kappa = (double *)(j->dbuf + o_k);
     j->val64 = (double *)(j->dbuf + o_v64);
     j->val32 = (float *)(j->dbuf + o_v32);

@@ -312,7 +312,6 @@ int plain_cg_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solv
         PlainScal *dsc = nullptr, *hsc = nullptr;
         ~Bufs()
         {
-            if (hsc) (void)hipHostFree(hsc);
             dfree(ctx, r);
             dfree(ctx, z);
             dfree(ctx, p);
@@ -327,7 +326,7 @@ int plain_cg_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solv
     GRMP_TRY(dalloc(ctx, &B.q, n));
     GRMP_TRY(dalloc(ctx, &B.part, 2 * PGRID_ROWS + 2));
     GRMP_TRY(dalloc(ctx, &B.dsc, 1));
-    GRMP_HIP(ctx, hipHostMalloc((void **)&B.hsc, sizeof(PlainScal), hipHostMallocDefault));
+    B.hsc = reinterpret_cast<PlainScal *>(ctx->pin);
     double *r = B.r, *z = B.z, *p = B.p, *q = B.q, *part = B.part;
     PlainScal *dsc = B.dsc, *hsc = B.hsc;
     double *fold = part + 2 * PGRID_ROWS;
@@ -533,12 +532,11 @@ int bicgstab_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solv
         double *hp = nullptr;
         ~Bufs()
         {
-            if (hp) (void)hipHostFree(hp);
             dfree(ctx, w);
         }
     } B{ctx};
     GRMP_TRY(dalloc(ctx, &B.w, 8 * (size_t)n + 2 * PGRID_ROWS + 2));
-    GRMP_HIP(ctx, hipHostMalloc((void **)&B.hp, 2 * sizeof(double), hipHostMallocDefault));
+    B.hp = reinterpret_cast<double *>(ctx->pin);
     double *r = B.w, *rh = r + n, *p = rh + n, *v = p + n, *s = v + n, *t = s + n, *ph = t + n, *sh = ph + n;
     double *part = sh + n, *fold = part + 2 * PGRID_ROWS;
     const int grid = (int)std::min<int64_t>(PGRID_ROWS, std::max<int64_t>(1, (n + PB - 1) / PB));
