@@ -170,7 +170,27 @@ struct PlainScal {
     double rz, rr, bb, rtol2, alpha, beta;
     long long it, maxit;
     int done, status;
+    int first, pad;  // fused form: no direction yet
 };
+
+// the iteration count and the tests made before each iteration on the new
+// rz = a and rr = b: non-finite, converged, iteration cap
+__device__ __forceinline__ void plain_advance(PlainScal &s, double a, double b)
+{
+    s.beta = a / s.rz;
+    s.rz = a;
+    s.rr = b;
+    s.it += 1;
+    if (!(b == b) || isinf(b)) {
+        s.done = 1;
+        s.status = GRMP_ERR_NONFINITE;
+    } else if (b <= s.rtol2 * s.bb || b == 0.0) {
+        s.done = 1;
+    } else if (s.it >= s.maxit) {
+        s.done = 1;
+        s.status = GRMP_ERR_NOCONV;
+    }
+}
 
 // q = A p on free rows; partial p.q
 __global__ __launch_bounds__(PB) void k_plain_spmv(const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
@@ -243,8 +263,7 @@ __global__ __launch_bounds__(PB) void k_plain_alpha(const double *__restrict__ p
     if (threadIdx.x == 0) S->alpha = S->rz / a;
 }
 
-// beta = rz' / rz, the iteration count and the tests the host loop made
-// before each iteration: non-finite, converged, iteration cap
+// beta = rz' / rz, the iteration count and the tests
 __global__ __launch_bounds__(PB) void k_plain_beta(const double *__restrict__ part, int grid, PlainScal *S)
 {
     if (S->done) return;
@@ -254,20 +273,147 @@ __global__ __launch_bounds__(PB) void k_plain_beta(const double *__restrict__ pa
         b += part[2 * k + 1];
     }
     block_sum2(a, b);
+    if (threadIdx.x == 0) plain_advance(*S, a, b);
+}
+
+// ---- two launches an iteration for small systems
+// An iteration of five kernels is launch-bound below some 10^5 rows (16,641
+// rows: 15.8 us of kernels of which the product is 5.5).  Here each kernel's
+// workgroups fold the previous kernel's partials themselves, in the order of
+// the fold kernels, and the direction update p = z + beta p happens where the
+// product gathers it: the same iterates, 7.08 -> 4.21 ms for the whole solve of
+// those rows.  Folding costs every workgroup a read of all partials, so it ends
+// at PLAIN_FUSE_GRID workgroups.
+#define PLAIN_FUSE_GRID 512
+__device__ __forceinline__ void plain_fold_all(const double *__restrict__ part, int np, double &a, double &b)
+{
+    __shared__ double sh[2];
+    a = 0.0;
+    b = 0.0;
+    for (int k = threadIdx.x; k < np; k += PB) {
+        a += part[2 * k];
+        b += part[2 * k + 1];
+    }
+    block_sum2(a, b);
     if (threadIdx.x == 0) {
-        S->beta = a / S->rz;
-        S->rz = a;
-        S->rr = b;
-        S->it += 1;
-        if (!(b == b) || isinf(b)) {
-            S->done = 1;
-            S->status = GRMP_ERR_NONFINITE;
-        } else if (b <= S->rtol2 * S->bb || b == 0.0) {
-            S->done = 1;
-        } else if (S->it >= S->maxit) {
-            S->done = 1;
-            S->status = GRMP_ERR_NOCONV;
+        sh[0] = a;
+        sh[1] = b;
+    }
+    __syncthreads();
+    a = sh[0];
+    b = sh[1];
+}
+
+// beta and the tests from the residual's partials pin; p = z + beta pold;
+// q = A p on free rows; partials of p.q.  The scalars go from Sin to Sout
+// (every workgroup forms the same, the first one writes them).
+__global__ __launch_bounds__(PB) void k_plain_ap(const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
+                                                const double *__restrict__ v, const uint8_t *__restrict__ fixed,
+                                                const double *__restrict__ z, const double *__restrict__ pold,
+                                                double *__restrict__ p, double *__restrict__ q, int64_t n,
+                                                const double *__restrict__ pin, double *__restrict__ part,
+                                                const PlainScal *__restrict__ Sin, PlainScal *__restrict__ Sout)
+{
+    __shared__ double lds[SPMV_CAP64];
+    PlainScal s = *Sin;
+    const int t = threadIdx.x;
+    if (!s.done) {
+        double a, b;
+        plain_fold_all(pin, gridDim.x, a, b);
+        if (s.first) {
+            s.first = 0;
+            s.rz = a;
+            s.rr = b;
+            s.beta = 0.0;
+        } else {
+            plain_advance(s, a, b);
         }
+    }
+    if (blockIdx.x == 0 && t == 0) *Sout = s;
+    if (s.done) return;
+    const double beta = s.beta;
+    const int64_t r0 = (int64_t)blockIdx.x * PB, r1 = r0 + PB < n ? r0 + PB : n, r = r0 + t;
+    const int32_t base = rp[r0], end = rp[r1];
+    int32_t my0 = 0, my1 = 0;
+    if (r < r1) {
+        my0 = rp[r];
+        my1 = rp[r + 1];
+    }
+    double sum = 0.0;
+    for (int32_t c0 = base; c0 < end; c0 += SPMV_CAP64) {  // csr_rows_lds64 with two gathers
+        const int32_t c1 = c0 + SPMV_CAP64 < end ? c0 + SPMV_CAP64 : end;
+        __syncthreads();
+        constexpr int U = SPMV_UNROLL;
+        for (int32_t k = c0 + t; k < c1; k += U * PB) {
+            int32_t c[U];
+            double w[U], zv[U], pv[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                c[u] = 0;
+                w[u] = 0.0;
+                if (k + u * PB < c1) {
+                    c[u] = ci[k + u * PB];
+                    w[u] = v[k + u * PB];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                zv[u] = 0.0;
+                pv[u] = 0.0;
+                if (k + u * PB < c1) {
+                    zv[u] = z[c[u]];
+                    pv[u] = pold[c[u]];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (k + u * PB < c1) lds[k + u * PB - c0] = w[u] * (zv[u] + beta * pv[u]);
+        }
+        __syncthreads();
+        const int32_t a = my0 > c0 ? my0 : c0, b = my1 < c1 ? my1 : c1;
+        for (int32_t k = a; k < b; ++k) sum += lds[k - c0];
+    }
+    double a0 = 0.0, a1 = 0.0;
+    if (r < r1) {
+        const double pi = z[r] + beta * pold[r];
+        const double qi = fixed[r] ? 0.0 : sum;
+        p[r] = pi;
+        q[r] = qi;
+        a0 = pi * qi;
+    }
+    block_sum2(a0, a1);
+    if (t == 0) {
+        part[2 * blockIdx.x] = a0;
+        part[2 * blockIdx.x + 1] = a1;
+    }
+}
+
+// alpha from the product's partials pin, then k_plain_axpy's update
+__global__ __launch_bounds__(PB) void k_plain_xr(const PlainScal *__restrict__ S, const double *__restrict__ pin,
+                                                const double *__restrict__ p, const double *__restrict__ q,
+                                                const double *__restrict__ dinv, double *__restrict__ x,
+                                                double *__restrict__ r, double *__restrict__ z, int64_t n,
+                                                double *__restrict__ part)
+{
+    if (S->done) return;
+    double pq, dummy;
+    plain_fold_all(pin, gridDim.x, pq, dummy);
+    const double alpha = S->rz / pq;
+    double a0 = 0.0, a1 = 0.0;
+    const int64_t i = (int64_t)blockIdx.x * PB + threadIdx.x;
+    if (i < n) {
+        x[i] += alpha * p[i];
+        const double ri = r[i] - alpha * q[i];
+        const double zi = dinv[i] * ri;
+        r[i] = ri;
+        z[i] = zi;
+        a0 = ri * zi;
+        a1 = ri * ri;
+    }
+    block_sum2(a0, a1);
+    if (threadIdx.x == 0) {
+        part[2 * blockIdx.x] = a0;
+        part[2 * blockIdx.x + 1] = a1;
     }
 }
 
@@ -308,7 +454,7 @@ int plain_cg_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solv
     // every exit path releases the work vectors and the scalar records
     struct Bufs {
         grmp_ctx *ctx;
-        double *r = nullptr, *z = nullptr, *p = nullptr, *q = nullptr, *part = nullptr;
+        double *r = nullptr, *z = nullptr, *p = nullptr, *q = nullptr, *part = nullptr, *p2 = nullptr;
         PlainScal *dsc = nullptr, *hsc = nullptr;
         ~Bufs()
         {
@@ -317,6 +463,7 @@ int plain_cg_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solv
             dfree(ctx, p);
             dfree(ctx, q);
             dfree(ctx, part);
+            dfree(ctx, p2);
             dfree(ctx, dsc);
         }
     } B{ctx};
@@ -325,7 +472,7 @@ int plain_cg_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solv
     GRMP_TRY(dalloc(ctx, &B.p, n));
     GRMP_TRY(dalloc(ctx, &B.q, n));
     GRMP_TRY(dalloc(ctx, &B.part, 2 * PGRID_ROWS + 2));
-    GRMP_TRY(dalloc(ctx, &B.dsc, 1));
+    GRMP_TRY(dalloc(ctx, &B.dsc, 2));
     B.hsc = reinterpret_cast<PlainScal *>(ctx->pin);
     double *r = B.r, *z = B.z, *p = B.p, *q = B.q, *part = B.part;
     PlainScal *dsc = B.dsc, *hsc = B.hsc;
@@ -356,11 +503,28 @@ int plain_cg_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solv
             s0.rtol2 = o.rtol * o.rtol;
             s0.maxit = o.maxit;
             *hsc = s0;
-            if (hipMemcpyAsync(dsc, hsc, sizeof(PlainScal), hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
+            const bool fused = grid <= PLAIN_FUSE_GRID;
+            if (fused) {
+                s0.first = 1;
+                *hsc = s0;
+                rc = dalloc(ctx, &B.p2, n);
+            }
+            if (rc == GRMP_OK &&
+                hipMemcpyAsync(dsc, hsc, sizeof(PlainScal), hipMemcpyHostToDevice, ctx->stream) != hipSuccess)
                 rc = grmp_fail(ctx, GRMP_ERR_HIP, "plain CG: scalars");
-            const int chunk = 8;
+            const int chunk = fused ? 16 : 8;
+            // fused: p and the scalars change places each iteration, so a chunk of an even number ends where it
+            // began; the residual's partials lie in part, the product's behind them
+            double *part2 = part + 2 * PLAIN_FUSE_GRID;
             while (rc == GRMP_OK) {
-                for (int k = 0; k < chunk; ++k) {
+                for (int k = 0; k < chunk && fused; ++k) {
+                    double *pold = k & 1 ? B.p2 : p, *pnew = k & 1 ? p : B.p2;
+                    hipLaunchKernelGGL(k_plain_ap, dim3(grid), dim3(PB), 0, ctx->stream, A->rowptr, A->cols, A->val64,
+                                       A->fixed, z, pold, pnew, q, n, part, part2, dsc + (k & 1), dsc + (1 - (k & 1)));
+                    hipLaunchKernelGGL(k_plain_xr, dim3(grid), dim3(PB), 0, ctx->stream, dsc + (1 - (k & 1)), part2, pnew,
+                                       q, A->dinv64, xd, r, z, n, part);
+                }
+                for (int k = 0; k < chunk && !fused; ++k) {
                     hipLaunchKernelGGL(k_plain_spmv, dim3(grid), dim3(PB), 0, ctx->stream, A->rowptr, A->cols,
                                        A->val64, A->fixed, p, q, n, part, dsc);
                     hipLaunchKernelGGL(k_plain_alpha, dim3(1), dim3(PB), 0, ctx->stream, part, grid, dsc);
@@ -1322,7 +1486,11 @@ static int solve_engine(grmp_matrix *A, const grmp_vector *b, grmp_vector *x, co
     GRMP_TRY(dalloc(ctx, &buf, 4 * n));
     hipLaunchKernelGGL(k_plain_init, dim3(nblk(n, 256)), dim3(256), 0, ctx->stream, A->rowptr, A->diagpos, A->val64, A->fixed,
                        b->d, x->d, n);
-    KEngine eng(ctx, ctx->stream, 1, (int)((n + ENGINE_TILE_ROWS - 1) / ENGINE_TILE_ROWS) + 1, ENGINE_TILE_ROWS);
+    // one problem alone: about 2048 tiles, so that a small one still fills the chip (439,000 rows in tiles of
+    // ENGINE_TILE_ROWS are 214 workgroups on 256 CUs: 33 us per product of 55 MB, 28.7 ms for the solve that takes
+    // 19.1 ms now), of whole 256-row chunks
+    const int tile = (int)std::min<int64_t>(ENGINE_TILE_ROWS, (n / 2048 + KB - 1) / KB * KB + (n < 2048 ? KB : 0));
+    KEngine eng(ctx, ctx->stream, 1, (int)((n + tile - 1) / tile) + 1, tile);
     GRMP_TRY(eng.init());
     KProb p;
     memset(&p, 0, sizeof(p));

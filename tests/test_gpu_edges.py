@@ -97,3 +97,44 @@ def test_amg_wide_coarse_rows(grmp, hubs, k):
     x = spla.spsolve(A.to_scipy().tocsc(), b.entries())
     err = np.linalg.norm(sol.entries() - x) / np.linalg.norm(x)
     assert info.status == 0 and err <= 1e-8, (info.iterations, err)
+
+
+# plain CG: two launches an iteration up to 512 workgroups of 256 rows, five
+# beyond (P1 361 x 361 nodes: 130,321 rows, 510 workgroups; 363 x 363: 515);
+# FP32 sweeps: tiles of one problem alone
+@pytest.mark.parametrize("precision", ["fp64", "fp32_ir"])
+@pytest.mark.parametrize("N", [1, 2, 15, 16, 63, 360, 362])
+def test_krylov_cg_sizes(grmp, O, N, precision):
+    """1e-8 against LU: the residual is 1e-12, the condition of these systems
+    at most 1e5"""
+    print(f"[case] Jacobi CG, P1 {N}x{N}, {precision}", flush=True)
+    grid = grmp.grid_unitsquare(N)
+    fes = grmp.FESpace(grmp.H1P1(1), grid)
+    pde = grmp.PoissonProblem(1.0)
+    pde.add_rhsdata(0, grmp.LinearForm(grmp.Identity, grmp.DataFunction([1.0])))
+    pde.add_boundarydata(0)
+    sol = grmp.FEVector([fes])
+    info, A, b = grmp.solve(sol, pde, precision=precision, rtol=1e-12)
+    import scipy.sparse.linalg as spla
+    x = spla.spsolve(A.to_scipy().tocsc(), b.entries())
+    err = np.linalg.norm(sol.entries() - x) / max(np.linalg.norm(x), 1e-300)
+    assert info.status == 0 and err <= 1e-8, (info.iterations, err)
+
+
+def test_krylov_cg_iteration_cap(grmp):
+    """The cap and a start at the solution end both forms as before."""
+    print("[case] Jacobi CG, iteration cap", flush=True)
+    for N in (40, 400):
+        grid = grmp.grid_unitsquare(N)
+        fes = grmp.FESpace(grmp.H1P1(1), grid)
+        pde = grmp.PoissonProblem(1.0)
+        pde.add_rhsdata(0, grmp.LinearForm(grmp.Identity, grmp.DataFunction([1.0])))
+        pde.add_boundarydata(0)
+        sol = grmp.FEVector([fes])
+        with pytest.raises(grmp.GrmpError) as e:
+            grmp.solve(sol, pde, rtol=1e-12, maxiterations=5)
+        assert e.value.code == grmp._abi.ERR_NOCONV and "after 5 iterations" in str(e.value)
+        pde0 = grmp.PoissonProblem(1.0)
+        pde0.add_boundarydata(0)
+        info, A, b = grmp.solve(grmp.FEVector([fes]), pde0, rtol=1e-12)
+        assert info.status == 0 and info.iterations == 0
