@@ -2354,14 +2354,15 @@ extern "C" int grmp_mg_apply(grmp_mg *m, const grmp_vector *b, grmp_vector *x, d
 // reset so the V-cycle kernels run (a finished CG leaves done set)
 __global__ void k_mg_pc_in(const double *__restrict__ v, const uint8_t *__restrict__ fixed,
                            const double *__restrict__ dinv, const double *__restrict__ lam, double *__restrict__ r,
-                           double *__restrict__ d, MgScal *__restrict__ sc, int64_t n)
+                           double *__restrict__ d, MgScal *__restrict__ sc, int64_t n, const int *__restrict__ skip)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int sk = skip ? *skip : 0;  // skip: the V-cycle's kernels see a finished solve
     if (i == 0) {
-        sc->done = 0;
+        sc->done = sk ? 1 : 0;
         sc->status = 0;
     }
-    if (i >= n) return;
+    if (i >= n || sk) return;
     const bool fx = fixed[i] != 0;
     const double ri = fx ? 0.0 : v[i];
     r[i] = ri;
@@ -2416,11 +2417,11 @@ int mg_precond_apply_pair(grmp_mg *m, const double *v0, double *z0, const double
     GRMP_HIP(m->ctx, hipEventRecord(m->fork, st));
     GRMP_HIP(m->ctx, hipStreamWaitEvent(m->st2, m->fork, 0));
     hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, m->st2, v1, m->A0->fixed, j2->lv[0].dinv,
-                       j2->lv[0].lam, j2->r, j2->lv[0].d, j2->sc, n);
+                       j2->lv[0].lam, j2->r, j2->lv[0].d, j2->sc, n, nullptr);
     mg_vcycle(j2);
     GRMP_HIP(m->ctx, hipMemcpyAsync(z1, j2->z, sizeof(double) * n, hipMemcpyDeviceToDevice, m->st2));
     hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, st, v0, m->A0->fixed, j->lv[0].dinv,
-                       j->lv[0].lam, j->r, j->lv[0].d, j->sc, n);
+                       j->lv[0].lam, j->r, j->lv[0].d, j->sc, n, nullptr);
     mg_vcycle(j);
     GRMP_HIP(m->ctx, hipMemcpyAsync(z0, j->z, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
     GRMP_HIP(m->ctx, hipEventRecord(m->join, m->st2));
@@ -2435,7 +2436,7 @@ int mg_precond_apply(grmp_mg *m, const double *v, double *z, hipStream_t st)
     const int64_t n = m->n;
     GRMP_CHECK(m->ctx, st == j->st, GRMP_ERR_ARG, "multigrid preconditioner: not the hierarchy's stream");
     hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, st, v, m->A0->fixed, j->lv[0].dinv, j->lv[0].lam,
-                       j->r, j->lv[0].d, j->sc, n);
+                       j->r, j->lv[0].d, j->sc, n, nullptr);
     mg_vcycle(j);
     GRMP_HIP(m->ctx, hipMemcpyAsync(z, j->z, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
     GRMP_HIP(m->ctx, hipGetLastError());
@@ -3375,15 +3376,18 @@ extern "C" int grmp_amg_destroy(grmp_amg *m)
 // z = V v: one V-cycle of the hierarchy from a zero start (fixed rows 0), as
 // the right preconditioner of BiCGStab on a matrix of the hierarchy's rows,
 // e.g. the Newton matrix it was built from
-int amg_precond_apply(grmp_amg *m, const double *v, double *z, hipStream_t st)
+int amg_precond_apply(grmp_amg *m, const double *v, double *z, hipStream_t st, const int *skip)
 {
     GRMP_CHECK(m->ctx, st == m->ctx->stream, GRMP_ERR_ARG,
                "algebraic multigrid preconditioner: not the hierarchy's stream");
-    const AmgLevel &L0 = m->lv[0];
+    AmgLevel &L0 = m->lv[0];
     hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(L0.n, 256)), dim3(256), 0, st, v, L0.fixed, L0.dinv, L0.lam, m->r, L0.d, m->sc,
-                       L0.n);
+                       L0.n, skip);
+    // level 0 works in the caller's z (the cycle writes every row of it), so nothing is copied out
+    double *own = L0.x;
+    L0.x = z;
     amg_vcycle(m);
-    GRMP_HIP(m->ctx, hipMemcpyAsync(z, m->z, sizeof(double) * L0.n, hipMemcpyDeviceToDevice, st));
+    L0.x = own;
     GRMP_HIP(m->ctx, hipGetLastError());
     return GRMP_OK;
 }

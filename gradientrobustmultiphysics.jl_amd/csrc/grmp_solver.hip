@@ -559,19 +559,91 @@ int plain_cg_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solv
 // ------------------------------------------------------ BiCGStab (FP64)
 // For the nonsymmetric Newton matrices of NonlinearForms: BiCGStab (van der
 // Vorst 1992) with right Jacobi preconditioning, fixed dofs eliminated as in
-// the plain CG (x_d = b_d / A_dd, rows masked).  Host-driven: the dot
-// products are folded on the device in a fixed order and read back.
+// the plain CG (x_d = b_d / A_dd, rows masked).  The dot products are folded
+// on the device in a fixed order.
 // Near-breakdowns (the shadow residual nearly orthogonal to r or to A p, or
 // omega = 0) restart the recurrence from the true residual with a new
 // shadow residual; on Newton matrices of P2 forms at 10^5 dofs and more
 // they happen every few hundred iterations.
 
-// y = A x on free rows (0 on fixed rows); partials (w.y, y.y)
+// The scalars live on the device: a fold kernel after each product or update
+// forms alpha, omega and beta and makes the iteration's tests, and the host
+// reads the record once per chunk of iterations.  Read back at each dot
+// product, five waits an iteration were a fifth of the Newton loop's time.
+enum { BIC_RUN = 0, BIC_DONE = 1, BIC_BREAK = 2 };  // BIC_BREAK: near-breakdown, restart from the true residual
+struct BicScal {
+    double rho, rhh, rr, tol2, alpha, omega, beta;
+    long long it, maxit;
+    int state, status;
+    int half;   // |s| met the tolerance: the iteration ends with x += alpha ph
+    int nosec;  // no second half: state set or half
+};
+#define BIC_BRK 1e-15  // near-breakdown: |cosine| below this
+
+// the tests at the top of an iteration on the residual rr and rho
+__device__ __host__ inline void bic_top(BicScal &s)
+{
+    if (!(s.rr == s.rr) || std::isinf(s.rr)) {
+        s.state = BIC_DONE;
+        s.status = GRMP_ERR_NONFINITE;
+    } else if (s.rr <= s.tol2 || s.rr == 0.0) {
+        s.state = BIC_DONE;
+    } else if (s.it >= s.maxit) {
+        s.state = BIC_DONE;
+        s.status = GRMP_ERR_NOCONV;
+    } else if (fabs(s.rho) <= BIC_BRK * sqrt(s.rhh * s.rr)) {
+        s.state = BIC_BREAK;
+    }
+}
+
+enum { BIC_RV = 0, BIC_SS = 1, BIC_TS = 2, BIC_RHO = 3 };
+// folds the partial pairs as k_plain_fold does, then the scalar step of W:
+// RV (rh.v, v.v), SS (s.s), TS (s.t, t.t), RHO (rh.r, r.r of the new r)
+template <int W>
+__global__ __launch_bounds__(PB) void k_bic_fold(const double *__restrict__ part, int grid, BicScal *S)
+{
+    if (S->state || (W == BIC_TS && S->nosec)) return;
+    double a = 0.0, b = 0.0;
+    for (int k = threadIdx.x; k < grid; k += PB) {
+        a += part[2 * k];
+        b += part[2 * k + 1];
+    }
+    block_sum2(a, b);
+    if (threadIdx.x != 0) return;
+    BicScal s = *S;
+    if (W == BIC_RV) {
+        if (fabs(a) <= BIC_BRK * sqrt(s.rhh * b)) s.state = BIC_BREAK;
+        else s.alpha = s.rho / a;
+    } else if (W == BIC_SS) {
+        s.it += 1;
+        s.half = a <= s.tol2;
+        s.omega = 0.0;
+    } else if (W == BIC_TS) {
+        s.omega = b > 0.0 ? a / b : 0.0;
+    } else {
+        s.rr = b;
+        if (s.half) {
+            s.state = BIC_DONE;
+        } else if (s.omega == 0.0) {  // x and r advanced by alpha only: restart from there
+            s.state = b <= s.tol2 ? BIC_DONE : BIC_BREAK;
+        } else {
+            s.beta = (a / s.rho) * (s.alpha / s.omega);
+            s.rho = a;
+            bic_top(s);
+        }
+    }
+    s.nosec = s.state != BIC_RUN || s.half;
+    *S = s;
+}
+
+// y = A x on free rows (0 on fixed rows); partials (w.y, y.y); nothing while *skip
 __global__ __launch_bounds__(PB) void k_bic_spmv(const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
                                                 const double *__restrict__ v, const uint8_t *__restrict__ fixed,
                                                 const double *__restrict__ x, const double *__restrict__ w,
-                                                double *__restrict__ y, int64_t n, double *__restrict__ part)
+                                                double *__restrict__ y, int64_t n, double *__restrict__ part,
+                                                const int *__restrict__ skip)
 {
+    if (*skip) return;
     __shared__ double lds[SPMV_CAP64];
     double a0 = 0.0, a1 = 0.0;
     for (int64_t r0 = (int64_t)blockIdx.x * PB; r0 < n; r0 += (int64_t)gridDim.x * PB) {
@@ -636,9 +708,12 @@ __global__ void k_bic_scale(const double *__restrict__ d, const double *__restri
 }
 
 // s = r - alpha v; partials (s.s, 0)
-__global__ __launch_bounds__(PB) void k_bic_s(const double *__restrict__ r, const double *__restrict__ v, double alpha,
-                                             double *__restrict__ s, int64_t n, double *__restrict__ part)
+__global__ __launch_bounds__(PB) void k_bic_s(const double *__restrict__ r, const double *__restrict__ v,
+                                             double *__restrict__ s, int64_t n, double *__restrict__ part,
+                                             const BicScal *__restrict__ S)
 {
+    if (S->state) return;
+    const double alpha = S->alpha;
     double a0 = 0.0, a1 = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * PB + threadIdx.x; i < n; i += (int64_t)gridDim.x * PB) {
         const double si = r[i] - alpha * v[i];
@@ -652,13 +727,20 @@ __global__ __launch_bounds__(PB) void k_bic_s(const double *__restrict__ r, cons
     }
 }
 
-// x += alpha ph + omega sh; r = s - omega t; partials (rh.r, r.r)
+// x += alpha ph + omega sh; r = s - omega t (sh and t of this iteration unless
+// it ends at half); partials (rh.r, r.r)
 __global__ __launch_bounds__(PB) void k_bic_update(double *__restrict__ x, const double *__restrict__ ph,
-                                                  const double *__restrict__ sh, double alpha, double omega,
-                                                  const double *__restrict__ s, const double *__restrict__ t,
-                                                  double *__restrict__ r, const double *__restrict__ rh, int64_t n,
-                                                  double *__restrict__ part)
+                                                  const double *__restrict__ sh, const double *__restrict__ s,
+                                                  const double *__restrict__ t, double *__restrict__ r,
+                                                  const double *__restrict__ rh, int64_t n,
+                                                  double *__restrict__ part, const BicScal *__restrict__ S)
 {
+    if (S->state) return;
+    const double alpha = S->alpha, omega = S->omega;
+    if (S->half) {
+        sh = ph;
+        t = s;
+    }
     double a0 = 0.0, a1 = 0.0;
     for (int64_t i = (int64_t)blockIdx.x * PB + threadIdx.x; i < n; i += (int64_t)gridDim.x * PB) {
         x[i] += alpha * ph[i] + omega * sh[i];
@@ -674,9 +756,11 @@ __global__ __launch_bounds__(PB) void k_bic_update(double *__restrict__ x, const
     }
 }
 
-__global__ void k_bic_p(const double *__restrict__ r, const double *__restrict__ v, double beta, double omega,
-                        double *__restrict__ p, int64_t n)
+__global__ void k_bic_p(const double *__restrict__ r, const double *__restrict__ v, double *__restrict__ p, int64_t n,
+                        const BicScal *__restrict__ S)
 {
+    if (S->state) return;
+    const double beta = S->beta, omega = S->omega;
     for (int64_t i = (int64_t)blockIdx.x * PB + threadIdx.x; i < n; i += (int64_t)gridDim.x * PB)
         p[i] = r[i] + beta * (p[i] - omega * v[i]);
 }
@@ -694,12 +778,15 @@ int bicgstab_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solv
         grmp_ctx *ctx;
         double *w = nullptr;
         double *hp = nullptr;
+        BicScal *S = nullptr;
         ~Bufs()
         {
             dfree(ctx, w);
+            dfree(ctx, S);
         }
     } B{ctx};
     GRMP_TRY(dalloc(ctx, &B.w, 8 * (size_t)n + 2 * PGRID_ROWS + 2));
+    GRMP_TRY(dalloc(ctx, &B.S, 1));
     B.hp = reinterpret_cast<double *>(ctx->pin);
     double *r = B.w, *rh = r + n, *p = rh + n, *v = p + n, *s = v + n, *t = s + n, *ph = t + n, *sh = ph + n;
     double *part = sh + n, *fold = part + 2 * PGRID_ROWS;
@@ -723,80 +810,61 @@ int bicgstab_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solv
         hipLaunchKernelGGL(k_bic_guess, dim3(gride), dim3(PB), 0, ctx->stream, A->fixed, sh, xd, n);
         GRMP_TRY(restart(rho, rr));
     }
-    double rhh = rr;              // rh.rh
-    const double brk = 1e-15;     // near-breakdown: |cosine| below this
-    const int max_restarts = 200;
+    BicScal h;
+    memset(&h, 0, sizeof(h));
+    h.rho = rho;
+    h.rr = h.rhh = rr;
+    h.tol2 = tol2;
+    h.maxit = o.maxit;
+    bic_top(h);
+    const int max_restarts = 200, chunk = 2;
     int restarts = 0;
-    int64_t it = 0;
-    int status = GRMP_OK;
-    while (true) {
-        if (!(rr == rr) || std::isinf(rr)) {
-            status = GRMP_ERR_NONFINITE;
-            break;
-        }
-        if (rr <= tol2 || rr == 0.0) break;
-        if (it >= o.maxit) {
-            status = GRMP_ERR_NOCONV;
-            break;
-        }
-        if (std::fabs(rho) <= brk * std::sqrt(rhh * rr)) {
+    BicScal *S = B.S, *hS = reinterpret_cast<BicScal *>(ctx->pin + 64);
+    bool upload = true;
+    while (h.state != BIC_DONE) {
+        if (h.state == BIC_BREAK) {
             if (++restarts > max_restarts) {
-                status = GRMP_ERR_NOCONV;
+                h.status = GRMP_ERR_NOCONV;
                 break;
             }
-            GRMP_TRY(restart(rho, rr));
-            rhh = rr;
+            GRMP_TRY(restart(h.rho, h.rr));
+            h.rhh = h.rr;
+            h.state = BIC_RUN;
+            h.half = h.nosec = 0;
+            bic_top(h);
+            upload = true;
             continue;
         }
-        double rv, vv, ss, dummy, ts, tt;
-        if (pc) GRMP_TRY(amg_precond_apply(pc, p, ph, ctx->stream));
-        else hipLaunchKernelGGL(k_bic_scale, dim3(gride), dim3(PB), 0, ctx->stream, A->dinv64, p, ph, n);
-        hipLaunchKernelGGL(k_bic_spmv, dim3(grid), dim3(PB), 0, ctx->stream, A->rowptr, A->cols, A->val64, A->fixed, ph,
-                           rh, v, n, part);
-        GRMP_TRY(plain_sum(ctx, part, fold, B.hp, grid, rv, vv));
-        if (std::fabs(rv) <= brk * std::sqrt(rhh * vv)) {
-            if (++restarts > max_restarts) {
-                status = GRMP_ERR_NOCONV;
-                break;
-            }
-            GRMP_TRY(restart(rho, rr));
-            rhh = rr;
-            continue;
+        if (upload) {
+            *hS = h;
+            GRMP_HIP(ctx, hipMemcpyAsync(S, hS, sizeof(BicScal), hipMemcpyHostToDevice, ctx->stream));
+            upload = false;
         }
-        const double alpha = rho / rv;
-        hipLaunchKernelGGL(k_bic_s, dim3(gride), dim3(PB), 0, ctx->stream, r, v, alpha, s, n, part);
-        GRMP_TRY(plain_sum(ctx, part, fold, B.hp, gride, ss, dummy));
-        ++it;
-        if (ss <= tol2) {  // x += alpha ph; the residual is s
-            hipLaunchKernelGGL(k_bic_update, dim3(gride), dim3(PB), 0, ctx->stream, xd, ph, ph, alpha, 0.0, s, s, r, rh,
-                               n, part);
-            GRMP_TRY(plain_sum(ctx, part, fold, B.hp, gride, dummy, rr));
-            break;
+        for (int k = 0; k < chunk; ++k) {
+            if (pc) GRMP_TRY(amg_precond_apply(pc, p, ph, ctx->stream, &S->state));
+            else hipLaunchKernelGGL(k_bic_scale, dim3(gride), dim3(PB), 0, ctx->stream, A->dinv64, p, ph, n);
+            hipLaunchKernelGGL(k_bic_spmv, dim3(grid), dim3(PB), 0, ctx->stream, A->rowptr, A->cols, A->val64, A->fixed,
+                               ph, rh, v, n, part, &S->state);
+            hipLaunchKernelGGL(k_bic_fold<BIC_RV>, dim3(1), dim3(PB), 0, ctx->stream, part, grid, S);
+            hipLaunchKernelGGL(k_bic_s, dim3(gride), dim3(PB), 0, ctx->stream, r, v, s, n, part, S);
+            hipLaunchKernelGGL(k_bic_fold<BIC_SS>, dim3(1), dim3(PB), 0, ctx->stream, part, gride, S);
+            if (pc) GRMP_TRY(amg_precond_apply(pc, s, sh, ctx->stream, &S->nosec));
+            else hipLaunchKernelGGL(k_bic_scale, dim3(gride), dim3(PB), 0, ctx->stream, A->dinv64, s, sh, n);
+            hipLaunchKernelGGL(k_bic_spmv, dim3(grid), dim3(PB), 0, ctx->stream, A->rowptr, A->cols, A->val64, A->fixed,
+                               sh, s, t, n, part, &S->nosec);
+            hipLaunchKernelGGL(k_bic_fold<BIC_TS>, dim3(1), dim3(PB), 0, ctx->stream, part, grid, S);
+            hipLaunchKernelGGL(k_bic_update, dim3(gride), dim3(PB), 0, ctx->stream, xd, ph, sh, s, t, r, rh, n, part, S);
+            hipLaunchKernelGGL(k_bic_fold<BIC_RHO>, dim3(1), dim3(PB), 0, ctx->stream, part, gride, S);
+            hipLaunchKernelGGL(k_bic_p, dim3(gride), dim3(PB), 0, ctx->stream, r, v, p, n, S);
         }
-        if (pc) GRMP_TRY(amg_precond_apply(pc, s, sh, ctx->stream));
-        else hipLaunchKernelGGL(k_bic_scale, dim3(gride), dim3(PB), 0, ctx->stream, A->dinv64, s, sh, n);
-        hipLaunchKernelGGL(k_bic_spmv, dim3(grid), dim3(PB), 0, ctx->stream, A->rowptr, A->cols, A->val64, A->fixed, sh,
-                           s, t, n, part);
-        GRMP_TRY(plain_sum(ctx, part, fold, B.hp, grid, ts, tt));
-        const double omega = tt > 0.0 ? ts / tt : 0.0;
-        hipLaunchKernelGGL(k_bic_update, dim3(gride), dim3(PB), 0, ctx->stream, xd, ph, sh, alpha, omega, s, t, r, rh,
-                           n, part);
-        double rho2;
-        GRMP_TRY(plain_sum(ctx, part, fold, B.hp, gride, rho2, rr));
-        if (omega == 0.0) {   // x and r advanced by alpha only: restart from there
-            if (rr <= tol2) break;
-            if (++restarts > max_restarts) {
-                status = GRMP_ERR_NOCONV;
-                break;
-            }
-            GRMP_TRY(restart(rho, rr));
-            rhh = rr;
-            continue;
-        }
-        const double beta = (rho2 / rho) * (alpha / omega);
-        rho = rho2;
-        hipLaunchKernelGGL(k_bic_p, dim3(gride), dim3(PB), 0, ctx->stream, r, v, beta, omega, p, n);
+        GRMP_HIP(ctx, hipGetLastError());
+        GRMP_HIP(ctx, hipMemcpyAsync(hS, S, sizeof(BicScal), hipMemcpyDeviceToHost, ctx->stream));
+        GRMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        h = *hS;
     }
+    const int64_t it = h.it;
+    const int status = h.status;
+    rr = h.rr;
     GRMP_HIP(ctx, hipGetLastError());
     GRMP_HIP(ctx, hipStreamSynchronize(ctx->stream));
     info.iterations = it;
