@@ -76,7 +76,7 @@ int grmp_fail(grmp_ctx *ctx, int code, const char *fmt, ...);
         if (rc_ != GRMP_OK) return rc_; \
     } while (0)
 
-#define GRMP_PIN_BYTES 16384  // bytes of grmp_ctx::pin
+#define GRMP_PIN_BYTES 65536  // bytes of grmp_ctx::pin
 
 // device allocation helpers (stream-ordered, from the context's pool)
 inline hipError_t ctx_malloc(grmp_ctx *ctx, void **p, size_t bytes, hipStream_t st)

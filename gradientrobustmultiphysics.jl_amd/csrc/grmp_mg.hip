@@ -2407,6 +2407,22 @@ int mg_pair_prepare(grmp_mg *m)
     return GRMP_OK;
 }
 
+// z = V(r), d0 of r in place, into the caller's z: level 0 works there (the
+// cycle writes every row of it) unless the whole cycle is one workgroup's
+static int mg_vcycle_into(MgJob *j, double *z)
+{
+    if (j->first_small == 0) {
+        mg_vcycle(j);
+        GRMP_HIP(j->ctx, hipMemcpyAsync(z, j->z, sizeof(double) * j->lv[0].n, hipMemcpyDeviceToDevice, j->st));
+        return GRMP_OK;
+    }
+    double *own = j->lv[0].x;
+    j->lv[0].x = z;
+    mg_vcycle(j);
+    j->lv[0].x = own;
+    return GRMP_OK;
+}
+
 // z0 = V v0 on the hierarchy's stream st and z1 = V v1 on the second
 // hierarchy's stream, at the same time; st waits for both
 int mg_precond_apply_pair(grmp_mg *m, const double *v0, double *z0, const double *v1, double *z1, hipStream_t st)
@@ -2418,12 +2434,10 @@ int mg_precond_apply_pair(grmp_mg *m, const double *v0, double *z0, const double
     GRMP_HIP(m->ctx, hipStreamWaitEvent(m->st2, m->fork, 0));
     hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, m->st2, v1, m->A0->fixed, j2->lv[0].dinv,
                        j2->lv[0].lam, j2->r, j2->lv[0].d, j2->sc, n, nullptr);
-    mg_vcycle(j2);
-    GRMP_HIP(m->ctx, hipMemcpyAsync(z1, j2->z, sizeof(double) * n, hipMemcpyDeviceToDevice, m->st2));
+    GRMP_TRY(mg_vcycle_into(j2, z1));
     hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, st, v0, m->A0->fixed, j->lv[0].dinv,
                        j->lv[0].lam, j->r, j->lv[0].d, j->sc, n, nullptr);
-    mg_vcycle(j);
-    GRMP_HIP(m->ctx, hipMemcpyAsync(z0, j->z, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
+    GRMP_TRY(mg_vcycle_into(j, z0));
     GRMP_HIP(m->ctx, hipEventRecord(m->join, m->st2));
     GRMP_HIP(m->ctx, hipStreamWaitEvent(st, m->join, 0));
     GRMP_HIP(m->ctx, hipGetLastError());
@@ -2437,8 +2451,7 @@ int mg_precond_apply(grmp_mg *m, const double *v, double *z, hipStream_t st)
     GRMP_CHECK(m->ctx, st == j->st, GRMP_ERR_ARG, "multigrid preconditioner: not the hierarchy's stream");
     hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, st, v, m->A0->fixed, j->lv[0].dinv, j->lv[0].lam,
                        j->r, j->lv[0].d, j->sc, n, nullptr);
-    mg_vcycle(j);
-    GRMP_HIP(m->ctx, hipMemcpyAsync(z, j->z, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
+    GRMP_TRY(mg_vcycle_into(j, z));
     GRMP_HIP(m->ctx, hipGetLastError());
     return GRMP_OK;
 }

@@ -39,7 +39,11 @@
 
 static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
+// Workgroups of the vector kernels, and at most of the row kernels: 1024 of
+// them (four a CU, seven row chunks one after the other on 1.8M rows) with
+// 32 KB of staging left the product waiting for its own loads, 85 us.
 #define MR_GRID 1024
+#define MR_GRID_ROWS 4096
 
 struct MrScal {
     double g, gp;          // gamma_j, gamma_{j-1}
@@ -60,7 +64,13 @@ __device__ __forceinline__ bool isfin_d(double v) { return v == v && fabs(v) <= 
 __device__ __forceinline__ double fixed_sum(const double *__restrict__ part, int n)
 {
     double a = 0.0, b = 0.0;
-    for (int k = threadIdx.x; k < n; k += KB) a += part[k];
+    for (int k = threadIdx.x; k < n; k += 8 * KB) {  // eight loads in flight, added in order
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = k + u * KB < n ? part[k + u * KB] : 0.0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) a += v[u];
+    }
     block_sum2(a, b);
     return a;
 }
@@ -146,6 +156,7 @@ __global__ __launch_bounds__(KB) void k_mr_start(MrScal *__restrict__ S, const d
 }
 
 // ------------------------------------------------------------ iteration
+#define MR_CAP (SPMV_CAP / 2)  // nonzeros staged per chunk: 16 KB in FP64
 // K1: deferred w/x update of the previous iteration, then
 //     q = S A z_j / gamma_j (0 on fixed rows), partial q.z_j / gamma_j
 template <class T, class V, class X>
@@ -157,7 +168,7 @@ __global__ __launch_bounds__(KB) void k_mr_apply(const int32_t *__restrict__ rp,
                                                  X *__restrict__ x, T *__restrict__ q, int64_t n,
                                                  const MrScal *__restrict__ S, double *__restrict__ part)
 {
-    __shared__ T lds[SPMV_CAP];
+    __shared__ T lds[MR_CAP];
     const int status = S->status;
     if (status == 2) return;
     const bool pend = S->pending != 0;
@@ -173,7 +184,7 @@ __global__ __launch_bounds__(KB) void k_mr_apply(const int32_t *__restrict__ rp,
             x[i] = (X)((double)x[i] + uce * wn);
         }
         if (status == 0) {
-            const T s = csr_rows_lds<T>(rp, ci, a, z, r0, r1, lds);
+            const T s = csr_rows_lds<T, V, T, MR_CAP>(rp, ci, a, z, r0, r1, lds);
             if (i < r1) {
                 const double d = (double)dsg[i];
                 double qi = fixed[i] ? 0.0 : (double)s * ig;
@@ -441,7 +452,7 @@ int minres_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solve_
     MrHost H;
     H.ctx = ctx;
     H.st = ctx->stream;
-    H.grid = (int)std::min<int64_t>(MR_GRID, std::max<int64_t>(1, (n + KB - 1) / KB));
+    H.grid = (int)std::min<int64_t>(MR_GRID_ROWS, std::max<int64_t>(1, (n + KB - 1) / KB));
     H.gride = (int)std::min<int64_t>(MR_GRID, std::max<int64_t>(1, (n + KB - 1) / KB));
     H.dS = nullptr;
     H.hS = nullptr;
@@ -456,14 +467,15 @@ int minres_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solve_
     int status = GRMP_OK;
     do {
         if ((rc = dalloc(ctx, &H.dS, 1))) break;
-        if ((rc = dalloc(ctx, &H.part, MR_GRID))) break;
+        if ((rc = dalloc(ctx, &H.part, MR_GRID_ROWS))) break;
         if ((rc = dalloc(ctx, &dsg, n))) break;
         H.hS = reinterpret_cast<MrScal *>(ctx->pin);
         if (ir) {
             if ((rc = dalloc(ctx, &dsg32, n))) break;
             if ((rc = dalloc(ctx, &dx, n))) break;
             if ((rc = dalloc(ctx, &r64, n))) break;
-            static_assert(1024 + sizeof(double) * MR_GRID <= GRMP_PIN_BYTES && sizeof(MrScal) <= 1024, "pinned scratch");
+            static_assert(1024 + sizeof(double) * MR_GRID_ROWS <= GRMP_PIN_BYTES && sizeof(MrScal) <= 1024,
+                          "pinned scratch");
             hres = reinterpret_cast<double *>(ctx->pin + 1024);
         }
         hipLaunchKernelGGL(k_mr_diag, dim3(nblk(n, 256)), dim3(256), 0, H.st, A->rowptr, A->cols, A->val64, A->fixed,
