@@ -138,3 +138,19 @@ def test_krylov_cg_iteration_cap(grmp):
         pde0.add_boundarydata(0)
         info, A, b = grmp.solve(grmp.FEVector([fes]), pde0, rtol=1e-12)
         assert info.status == 0 and info.iterations == 0
+
+
+# The levels' FP32 values and bounds: rows in whole blocks of 256 (P1 15, 31
+# and 127, elasticity 63) and just past them (P1 16), more than 2048 nonzeros
+# in a block (P2, elasticity)
+@pytest.mark.parametrize("spec", [(1, 1, 15), (1, 1, 16), (1, 1, 31), (1, 1, 127), (1, 2, 15), (1, 2, 63), (2, 1, 63)])
+def test_level_setup_matches_lu(grmp, O, spec):
+    """1e-8: the residual is 1e-12 and these systems' condition below 1e4; a
+    wrong value or bound shows in the iterations"""
+    print(f"[case] level setup {spec}", flush=True)
+    with grmp.Server("mg", mg_block_rows=64) as S:
+        t = S.submit(*spec, 7, rtol=1e-12)
+        r = S.wait(t)
+        x = _reference(grmp, O, *spec, 7)
+        err = np.linalg.norm(S.solution(t) - x) / np.linalg.norm(x)
+        assert r.status == 0 and r.iterations <= 60 and err <= 1e-8, (r.status, r.iterations, err)
