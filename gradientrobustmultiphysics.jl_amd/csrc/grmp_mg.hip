@@ -57,13 +57,29 @@ static bool ev_take(std::vector<hipEvent_t> &pool, hipEvent_t &e0, hipEvent_t &e
 #define MG_MAX_LEVELS 16
 #define MG_DENSE_MAX 64  // dofs of the coarsest level (P1 x 2 on 4 x 4: 50)
 
-// Chebyshev degree 2 on [lmax/8, lmax]: theta = 9/16 lmax, delta = 7/16 lmax,
-// rho0 = 7/9, rho1 = 63/113.
-//   x1 = x0 + d0,  d0 = D^-1 r0 / theta
-//   x2 = x1 + C1 d0 + C2 D^-1 (b - A x1),  C1 = rho1 rho0, C2 = 2 rho1 / delta
-#define CHEB_ITHETA(l) (16.0 / (9.0 * (l)))
-#define CHEB_C1 (49.0 / 113.0)
-#define CHEB_C2(l) (288.0 / (113.0 * (l)))
+// The smoother is a degree-2 Chebyshev polynomial of D^-1 A,
+//   x1 = x0 + d0,  d0 = it / lmax D^-1 r0
+//   x2 = x1 + c1 d0 + c2 / lmax D^-1 (b - A x1),
+// pre- and post-smoothing alike, so the cycle stays symmetric.  Two choices
+// of its coefficients, by the operator of the level:
+//   first kind on [lmax/8, lmax]:  theta = 9/16 lmax, delta = 7/16 lmax,
+//     rho0 = 7/9, rho1 = 63/113;  it = 16/9, c1 = rho1 rho0, c2 = 288/113
+//   fourth kind (Lottes, "Optimal polynomial smoothers for multigrid
+//     V-cycles", 2023):  it = 4/3, c1 = 1/5, c2 = 12/5.  No lower end of the
+//     interval: it weighs the middle of the spectrum by what the coarse
+//     correction leaves of it.
+// CG iterations with the first and the fourth kind (1e-10; P1 200^2 21 and 18,
+// P1 1000^2 28 and 22, a heat step on 1024^2 24 and 18; P2 500^2 22 and 22,
+// P2 1023^2 24 and 24, elasticity 383^2 39 and 42; aggregation on tetrahedra 33
+// and 34): hierarchies of one P1 component under CG take the fourth kind, the
+// others the first.  So does the velocity block of MINRES, which gains less
+// than the counts vary with the mesh (256^2: 234 and 224).
+struct MgCheb {
+    double lam;           // Gershgorin bound of D^-1 A
+    double it, c1, c2;
+};
+#define CHEB_FIRST_KIND {0.0, 16.0 / 9.0, 49.0 / 113.0, 288.0 / 113.0}
+#define CHEB_FOURTH_KIND {0.0, 4.0 / 3.0, 1.0 / 5.0, 12.0 / 5.0}
 
 // done: 0 iterating, 2 the updated residual met rtol (the true residual is
 // checked next), 1 finished (status says how)
@@ -148,7 +164,7 @@ struct MgRows {
     const double *v;     // the vector A multiplies
     const double *b, *dinv, *d;
     double *o1, *o2;
-    const double *lam;   // Gershgorin bound of D^-1 A (device)
+    const MgCheb *ch;
     const MgScal *sc;
     double *part;        // block partials (OP_PCG_Q: p.q; OP_CHEB_POST2 at level 0: r.z)
     const int32_t *agg;  // OP_AGG_POST1: coarse row of each row, the scale of the correction
@@ -162,9 +178,9 @@ struct MgRows {
 // nonzero.  Forming d0 inside the product gathered b, D^-1 and the mask per
 // nonzero: 59 us on 4.2M P1 rows against 45 us with d0 stored (the
 // producers take 16 bytes a row more).
-__device__ __forceinline__ double cheb_first(bool fx, double dinv, double b, double lam)
+__device__ __forceinline__ double cheb_first(bool fx, double dinv, double b, const MgCheb &ch)
 {
-    return fx ? 0.0 : dinv * b * CHEB_ITHETA(lam);
+    return fx ? 0.0 : dinv * b * (ch.it / ch.lam);
 }
 
 // 256 rows per block through the LDS-staged row product, then the epilogue:
@@ -182,7 +198,7 @@ __device__ __forceinline__ double cheb_first(bool fx, double dinv, double b, dou
 template <int OP>
 __device__ __forceinline__ double mg_epilogue(int64_t i, double s, bool fx, const double *__restrict__ v,
                                               const double *__restrict__ b, const double *__restrict__ dinv,
-                                              const double *__restrict__ d, const double *__restrict__ lam,
+                                              const double *__restrict__ d, const MgCheb *__restrict__ ch,
                                               double *__restrict__ o1, double *__restrict__ o2)
 {
     if (OP == OP_RESID) {
@@ -190,18 +206,15 @@ __device__ __forceinline__ double mg_epilogue(int64_t i, double s, bool fx, cons
     } else if (OP == OP_TRUE_RESID) {
         const double r = fx ? 0.0 : b[i] - s;
         o1[i] = r;
-        o2[i] = cheb_first(fx, dinv[i], r, *lam);
+        o2[i] = cheb_first(fx, dinv[i], r, *ch);
     } else if (OP == OP_CHEB_PRE) {
-        const double l = *lam;
-        o1[i] = fx ? 0.0 : (1.0 + CHEB_C1) * v[i] + CHEB_C2(l) * dinv[i] * (b[i] - s);
+        o1[i] = fx ? 0.0 : (1.0 + ch->c1) * v[i] + ch->c2 / ch->lam * dinv[i] * (b[i] - s);
     } else if (OP == OP_CHEB_POST1) {
-        const double l = *lam;
-        const double dd = fx ? 0.0 : dinv[i] * (b[i] - s) * CHEB_ITHETA(l);
+        const double dd = fx ? 0.0 : dinv[i] * (b[i] - s) * (ch->it / ch->lam);
         o1[i] = dd;
         o2[i] = v[i] + dd;
     } else if (OP == OP_CHEB_POST2) {
-        const double l = *lam;
-        const double z = fx ? 0.0 : v[i] + CHEB_C1 * d[i] + CHEB_C2(l) * dinv[i] * (b[i] - s);
+        const double z = fx ? 0.0 : v[i] + ch->c1 * d[i] + ch->c2 / ch->lam * dinv[i] * (b[i] - s);
         o1[i] = z;
         return b[i] * z;
     } else {
@@ -230,13 +243,13 @@ __device__ __forceinline__ void mg_rows_body(const MgRows &a, int64_t r0, int pi
     if constexpr (OP == OP_AGG_POST1) {
         if (i < r1) {
             const bool fx = a.fixed[i] != 0;
-            const double dd = fx ? 0.0 : a.dinv[i] * (a.b[i] - a.scale * s) * CHEB_ITHETA(*a.lam);
+            const double dd = fx ? 0.0 : a.dinv[i] * (a.b[i] - a.scale * s) * (a.ch->it / a.ch->lam);
             const double x = fx ? a.d[i] : a.d[i] + a.scale * a.v[a.agg[i]];
             a.o1[i] = dd;
             a.o2[i] = x + dd;
         }
     } else if (i < r1) {
-        pa = mg_epilogue<OP>(i, s, a.fixed[i] != 0, a.v, a.b, a.dinv, a.d, a.lam, a.o1, a.o2);
+        pa = mg_epilogue<OP>(i, s, a.fixed[i] != 0, a.v, a.b, a.dinv, a.d, a.ch, a.o1, a.o2);
     }
     if ((OP == OP_CHEB_POST2 || OP == OP_PCG_Q) && a.part) {
         block_sum2(pa, pb);
@@ -271,19 +284,19 @@ struct MgPrepLevel {
     const double *val, *dinv;
     const uint8_t *fixed;
     float *val32;
-    double *lam;
+    MgCheb *ch;
     int64_t n;
-    int blk0, pad;
+    int blk0, fourth;  // fourth: coefficients of the fourth kind
 };
 struct MgPrep {
     int nlev, blocks;
     MgPrepLevel lv[MG_MAX_LEVELS];
 };
 
-__global__ void k_mg_prep_zero(MgPrep P)
+__global__ void k_mg_prep_cheb(MgPrep P)
 {
     const int l = threadIdx.x;
-    if (l < P.nlev) P.lv[l].lam[0] = 0.0;
+    if (l < P.nlev) *P.lv[l].ch = P.lv[l].fourth ? MgCheb CHEB_FOURTH_KIND : MgCheb CHEB_FIRST_KIND;
 }
 
 // Bound by the values, 12 bytes a nonzero: they pass through LDS, read and
@@ -336,23 +349,37 @@ __global__ __launch_bounds__(KB) void k_mg_prep(MgPrep P)
     s = r < r1 && !fx ? s * fabs(L.dinv[r]) : 0.0;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) s = fmax(s, __shfl_down(s, o, 64));
-    unsigned long long *lam = (unsigned long long *)L.lam;
+    unsigned long long *lam = (unsigned long long *)&L.ch->lam;
     if ((t & 63) == 0 && s > 0.0) {
         const unsigned long long v = (unsigned long long)__double_as_longlong(s);
         if (v > __hip_atomic_load(lam, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(lam, v);
     }
 }
 
-static void mg_prep_add(MgPrep &P, const int32_t *rp, const double *val, const double *dinv, const uint8_t *fixed,
-                        float *val32, double *lam, int64_t n)
+// the coefficients of n levels (and of their copies in the LDS image), the bounds kept
+struct MgChebSet {
+    int n, fourth;
+    MgCheb *ch[2 * MG_MAX_LEVELS];
+};
+__global__ void k_mg_cheb_kind(MgChebSet P)
 {
-    P.lv[P.nlev++] = MgPrepLevel{rp, val, dinv, fixed, val32, lam, n, P.blocks, 0};
+    const int l = threadIdx.x;
+    if (l >= P.n) return;
+    MgCheb c = P.fourth ? MgCheb CHEB_FOURTH_KIND : MgCheb CHEB_FIRST_KIND;
+    c.lam = P.ch[l]->lam;
+    *P.ch[l] = c;
+}
+
+static void mg_prep_add(MgPrep &P, const int32_t *rp, const double *val, const double *dinv, const uint8_t *fixed,
+                        float *val32, MgCheb *ch, int64_t n, bool fourth)
+{
+    P.lv[P.nlev++] = MgPrepLevel{rp, val, dinv, fixed, val32, ch, n, P.blocks, fourth ? 1 : 0};
     P.blocks += (int)nblk(n, KB);
 }
 
 static void mg_prep_launch(const MgPrep &P, hipStream_t st)
 {
-    hipLaunchKernelGGL(k_mg_prep_zero, dim3(1), dim3(64), 0, st, P);
+    hipLaunchKernelGGL(k_mg_prep_cheb, dim3(1), dim3(64), 0, st, P);
     hipLaunchKernelGGL(k_mg_prep, dim3(P.blocks), dim3(KB), 0, st, P);
 }
 
@@ -514,7 +541,7 @@ __global__ void k_mg_prolong_p1(int64_t Nf, int64_t Nc, int ncomp, const double 
 // b_c = P^T r_f and, for the coarse level's smoothing, d_c = d0 of b_c
 __global__ void k_mg_restrict_p1(int64_t Nf, int64_t Nc, int ncomp, const double *__restrict__ rf,
                                  const uint8_t *__restrict__ fixed_c, const double *__restrict__ dinv_c,
-                                 const double *__restrict__ lam_c, double *__restrict__ bc, double *__restrict__ dc,
+                                 const MgCheb *__restrict__ ch_c, double *__restrict__ bc, double *__restrict__ dc,
                                  const MgScal *sc)
 {
     if (sc->done) return;
@@ -522,7 +549,7 @@ __global__ void k_mg_restrict_p1(int64_t Nf, int64_t Nc, int ncomp, const double
     if (t >= (Nc + 1) * (Nc + 1) * ncomp) return;
     const double b = restrict_p1_one(Nf, Nc, rf, fixed_c, t);
     bc[t] = b;
-    dc[t] = cheb_first(fixed_c[t] != 0, dinv_c[t], b, *lam_c);
+    dc[t] = cheb_first(fixed_c[t] != 0, dinv_c[t], b, *ch_c);
 }
 
 __global__ void k_mg_prolong_p2(int64_t N, const int32_t *__restrict__ cells, const int8_t *__restrict__ fsign,
@@ -535,7 +562,7 @@ __global__ void k_mg_prolong_p2(int64_t N, const int32_t *__restrict__ cells, co
 }
 
 __global__ void k_mg_restrict_p2(int64_t N, const double *__restrict__ r2, const uint8_t *__restrict__ fixed1,
-                                 const double *__restrict__ dinv1, const double *__restrict__ lam1,
+                                 const double *__restrict__ dinv1, const MgCheb *__restrict__ ch1,
                                  double *__restrict__ b1, double *__restrict__ d1, const MgScal *sc)
 {
     if (sc->done) return;
@@ -543,7 +570,7 @@ __global__ void k_mg_restrict_p2(int64_t N, const double *__restrict__ r2, const
     if (v >= (N + 1) * (N + 1)) return;
     const double b = restrict_p2_one(N, r2, fixed1, v);
     b1[v] = b;
-    d1[v] = cheb_first(fixed1[v] != 0, dinv1[v], b, *lam1);
+    d1[v] = cheb_first(fixed1[v] != 0, dinv1[v], b, *ch1);
 }
 
 // coarse coefficient: geometric mean of the fine cells whose centroid lies in
@@ -653,18 +680,19 @@ __global__ void k_mg_dot(const double *__restrict__ a, const double *__restrict_
 // x += alpha p, r -= alpha q; partials of r.r; d = d0 of the new r
 __global__ void k_mg_axpy(double *__restrict__ x, double *__restrict__ r, const double *__restrict__ p,
                           const double *__restrict__ q, const uint8_t *__restrict__ fixed,
-                          const double *__restrict__ dinv, const double *__restrict__ lam, double *__restrict__ d,
+                          const double *__restrict__ dinv, const MgCheb *__restrict__ ch, double *__restrict__ d,
                           int64_t n, double *part, const MgScal *sc)
 {
     if (sc->done) return;
-    const double al = sc->alpha, l = *lam;
+    const double al = sc->alpha;
+    const MgCheb c = *ch;
     const int64_t i = (int64_t)blockIdx.x * KB + threadIdx.x;
     double pa = 0.0, pb = 0.0;
     if (i < n) {
         x[i] += al * p[i];
         const double ri = r[i] - al * q[i];
         r[i] = ri;
-        d[i] = cheb_first(fixed[i] != 0, dinv[i], ri, l);
+        d[i] = cheb_first(fixed[i] != 0, dinv[i], ri, c);
         pa = ri * ri;
     }
     block_sum2(pa, pb);
@@ -673,7 +701,7 @@ __global__ void k_mg_axpy(double *__restrict__ x, double *__restrict__ r, const 
 
 // r = rhs on the free rows, 0 on the fixed ones; d = d0 of it
 __global__ void k_mg_start(const double *__restrict__ rhs, const uint8_t *__restrict__ fixed,
-                           const double *__restrict__ dinv, const double *__restrict__ lam, double *__restrict__ r,
+                           const double *__restrict__ dinv, const MgCheb *__restrict__ ch, double *__restrict__ r,
                            double *__restrict__ d, int64_t n)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -681,7 +709,7 @@ __global__ void k_mg_start(const double *__restrict__ rhs, const uint8_t *__rest
     const bool fx = fixed[i] != 0;
     const double ri = fx ? 0.0 : rhs[i];
     r[i] = ri;
-    d[i] = cheb_first(fx, dinv[i], ri, *lam);
+    d[i] = cheb_first(fx, dinv[i], ri, *ch);
 }
 
 __global__ void k_mg_update_p(double *__restrict__ p, const double *__restrict__ z, int64_t n, const MgScal *sc)
@@ -712,7 +740,7 @@ struct MgBLevel {
     const float *val32;
     const uint8_t *fixed;
     double *x, *b, *r, *d;
-    const double *lam;
+    const MgCheb *ch;
     int64_t n;
     int N, fe, ncomp, pad;
     const int32_t *cells;  // P2 level: its mesh, for the P1 -> P2 prolongation
@@ -730,7 +758,7 @@ enum MgTransfer { TR_P1 = 0, TR_P2 = 1, TR_AGG = 2 };
 struct MgPackLevel {
     int32_t n, N, fe, ncomp;
     int32_t tr;                   // transfer to the next level
-    int32_t val, ci, rp, dinv, fix, lam;
+    int32_t val, ci, rp, dinv, fix, ch;
     int32_t agg, mptr, midx;      // TR_AGG: row -> coarse row, and the coarse rows' members
     int32_t x, b, r, d;
 };
@@ -812,7 +840,7 @@ __device__ double blk_rows(const MgBLevel &L, const double *v, const double *b, 
             for (int32_t k = L.rp[i]; k < L.rp[i + 1]; ++k) s += L.val[k] * v[L.ci[k]];
         else
             for (int32_t k = L.rp[i]; k < L.rp[i + 1]; ++k) s += (double)L.val32[k] * v[L.ci[k]];
-        part += mg_epilogue<OP>(i, s, L.fixed[i] != 0, v, b, L.dinv, d, L.lam, o1, o2);
+        part += mg_epilogue<OP>(i, s, L.fixed[i] != 0, v, b, L.dinv, d, L.ch, o1, o2);
     }
     return part;
 }
@@ -825,7 +853,7 @@ __device__ double blk_vcycle(const MgBDesc &D)
     for (int l = D.first; l < L1; ++l) {
         const MgBLevel &L = D.lv[l], &C = D.lv[l + 1];
         for (int64_t i = threadIdx.x; i < L.n; i += MG_BT)
-            L.d[i] = cheb_first(L.fixed[i] != 0, L.dinv[i], L.b[i], *L.lam);
+            L.d[i] = cheb_first(L.fixed[i] != 0, L.dinv[i], L.b[i], *L.ch);
         __syncthreads();
         blk_rows<OP_CHEB_PRE>(L, L.d, L.b, nullptr, L.x, nullptr);
         __syncthreads();
@@ -908,7 +936,7 @@ __device__ __forceinline__ double pk_rows(const MgPackLevel &L, char *lds, int o
     const double *v = reinterpret_cast<const double *>(lds + ov);
     const double *b = reinterpret_cast<const double *>(lds + L.b), *d = reinterpret_cast<const double *>(lds + L.d);
     const double *dinv = reinterpret_cast<const double *>(lds + L.dinv);
-    const double *lam = reinterpret_cast<const double *>(lds + L.lam);
+    const MgCheb *ch = reinterpret_cast<const MgCheb *>(lds + L.ch);
     const uint8_t *fix = reinterpret_cast<const uint8_t *>(lds + L.fix);
     double *o1 = reinterpret_cast<double *>(lds + oo1), *o2 = reinterpret_cast<double *>(lds + oo2);
     double part = 0.0;
@@ -932,7 +960,7 @@ __device__ __forceinline__ double pk_rows(const MgPackLevel &L, char *lds, int o
                 if (k + u < k1) s += (double)w[u] * xv[u];
         }
         // b and d are read before o1 / o2 of the same row are written
-        part += mg_epilogue<OP>(i, s, fix[i] != 0, v, b, dinv, d, lam, o1, o2);
+        part += mg_epilogue<OP>(i, s, fix[i] != 0, v, b, dinv, d, ch, o1, o2);
     }
     return part;
 }
@@ -949,8 +977,8 @@ __device__ double pk_vcycle(const MgPack &P, char *lds, const double inv[4])
         const double *dinv = reinterpret_cast<const double *>(lds + L.dinv);
         const uint8_t *fix = reinterpret_cast<const uint8_t *>(lds + L.fix);
         double *d = reinterpret_cast<double *>(lds + L.d);
-        const double lam = *reinterpret_cast<const double *>(lds + L.lam);
-        for (int i = threadIdx.x; i < L.n; i += MG_BT) d[i] = cheb_first(fix[i] != 0, dinv[i], b[i], lam);
+        const MgCheb ch = *reinterpret_cast<const MgCheb *>(lds + L.ch);
+        for (int i = threadIdx.x; i < L.n; i += MG_BT) d[i] = cheb_first(fix[i] != 0, dinv[i], b[i], ch);
     }
     __syncthreads();
     for (int l = 0; l < L1; ++l) {
@@ -963,7 +991,7 @@ __device__ double pk_vcycle(const MgPack &P, char *lds, const double inv[4])
         const double *dinv = reinterpret_cast<const double *>(lds + C.dinv);
         const uint8_t *fix = reinterpret_cast<const uint8_t *>(lds + C.fix);
         double *bc = reinterpret_cast<double *>(lds + C.b), *dc = reinterpret_cast<double *>(lds + C.d);
-        const double lam = *reinterpret_cast<const double *>(lds + C.lam);
+        const MgCheb ch = *reinterpret_cast<const MgCheb *>(lds + C.ch);
         for (int t = threadIdx.x; t < C.n; t += MG_BT) {
             double s;
             if (L.tr == TR_P1) {
@@ -977,7 +1005,7 @@ __device__ double pk_vcycle(const MgPack &P, char *lds, const double inv[4])
                 for (int k = mp[t]; k < mp[t + 1]; ++k) s += r[mi[k]];
             }
             bc[t] = s;
-            dc[t] = cheb_first(fix[t] != 0, dinv[t], s, lam);
+            dc[t] = cheb_first(fix[t] != 0, dinv[t], s, ch);
         }
         __syncthreads();
     }
@@ -1058,7 +1086,8 @@ __device__ double blk_coarse(const MgBDesc &D, char *lds)
 struct MgPackSrc {
     const int32_t *rp, *ci;
     const float *val32;
-    const double *dinv, *lam;
+    const double *dinv;
+    const MgCheb *ch;
     const uint8_t *fixed;
     const int32_t *agg, *mptr, *midx;  // aggregates (TR_AGG), or nullptr
     int32_t nnz, nc;                   // nonzeros; rows of the next level
@@ -1080,7 +1109,7 @@ __global__ void k_mg_pack(MgPackLevel L, MgPackSrc S, char *__restrict__ img)
         }
     }
     if (S.agg && t <= S.nc) reinterpret_cast<uint16_t *>(img + L.mptr)[t] = (uint16_t)S.mptr[t];
-    if (t == 0) *reinterpret_cast<double *>(img + L.lam) = *S.lam;
+    if (t == 0) *reinterpret_cast<MgCheb *>(img + L.ch) = *S.ch;
 }
 
 // coarse end of a V-cycle (levels D.first ..); at D.first == 0 also the
@@ -1202,7 +1231,7 @@ __device__ __forceinline__ MgRows mg_tile_rows(const MgBDesc &D, int level)
     a.d = nullptr;
     a.o1 = nullptr;
     a.o2 = nullptr;
-    a.lam = L.lam;
+    a.ch = L.ch;
     a.sc = D.sc;
     a.part = nullptr;
     return a;
@@ -1261,7 +1290,7 @@ __global__ __launch_bounds__(KB) void k_mgb_restrict(const MgTile *__restrict__ 
         const double b = F.fe == GRMP_FE_H1P2 ? restrict_p2_one(F.N, F.r, C.fixed, i)
                                               : restrict_p1_one(F.N, C.N, F.r, C.fixed, i);
         C.b[i] = b;
-        C.d[i] = cheb_first(C.fixed[i] != 0, C.dinv[i], b, *C.lam);
+        C.d[i] = cheb_first(C.fixed[i] != 0, C.dinv[i], b, *C.ch);
     }
 }
 
@@ -1291,7 +1320,8 @@ __global__ __launch_bounds__(KB) void k_mgb_axpy(const MgTile *__restrict__ T, c
     const MgBDesc &D = *Dp[t.req];
     if (D.sc->done) return;
     const MgBLevel &L = D.lv[0];
-    const double al = D.sc->alpha, l = *L.lam;
+    const double al = D.sc->alpha;
+    const MgCheb ch = *L.ch;
     const int64_t n = L.n;
     for (int c = 0; c < MG_TILE_CHUNKS; ++c) {
         const int64_t r0 = t.row0 + (int64_t)c * KB;
@@ -1302,7 +1332,7 @@ __global__ __launch_bounds__(KB) void k_mgb_axpy(const MgTile *__restrict__ T, c
             D.x[i] += al * D.p[i];
             const double ri = D.r[i] - al * D.q[i];
             D.r[i] = ri;
-            L.d[i] = cheb_first(L.fixed[i] != 0, L.dinv[i], ri, l);
+            L.d[i] = cheb_first(L.fixed[i] != 0, L.dinv[i], ri, ch);
             pa = ri * ri;
         }
         block_sum2(pa, pb);
@@ -1401,7 +1431,7 @@ static bool mg_pack_layout(MgPack &P, const MgPackShape *sh, int nlev)
         L.ncomp = S.ncomp;
         L.tr = S.tr;
         L.dinv = take(8 * S.n, 8);
-        L.lam = take(8, 8);
+        L.ch = take(sizeof(MgCheb), 8);
         L.val = take(4 * S.nnz, 4);
         L.ci = take(2 * S.nnz, 2);
         L.rp = take(2 * (S.n + 1), 2);
@@ -1442,7 +1472,7 @@ struct MgLevel {
     double *kappa = nullptr, *val = nullptr, *dinv = nullptr, *x = nullptr, *b = nullptr, *r = nullptr, *d = nullptr;
     float *dinv32 = nullptr;
     float *val32 = nullptr;  // FP32 copy of val for the V-cycle, fixed rows 0
-    double *lam = nullptr;
+    MgCheb *ch = nullptr;
     DevForm *dforms = nullptr;
     DevForm hforms[4];
 };
@@ -1459,6 +1489,7 @@ struct MgJob {
     MgScal *sc = nullptr;
     int nb0 = 0;
     int first_small = 0;      // first level that runs inside one workgroup
+    bool fourth = false;      // smoother coefficients of the fourth kind
     char *img = nullptr;      // LDS image of those levels
     MgBDesc hdesc;
     MgBDesc *ddesc = nullptr;
@@ -1501,7 +1532,7 @@ static size_t mg_layout(MgJob *j, bool assign)
         o[10 * l + 5] = l == 0 ? 0 : take(L.n * 8);  // b (level 0: r)
         o[10 * l + 6] = take(L.n * 8);
         o[10 * l + 7] = take(L.n * 8);
-        o[10 * l + 8] = take(8 + sizeof(DevForm) * 4);
+        o[10 * l + 8] = take(sizeof(MgCheb) + sizeof(DevForm) * 4);
         o[10 * l + 9] = take(L.nnz * 4);
     }
     if (!assign) return off;
@@ -1530,8 +1561,8 @@ static size_t mg_layout(MgJob *j, bool assign)
         L.b = l == 0 ? j->r : (double *)(B + o[10 * l + 5]);
         L.r = (double *)(B + o[10 * l + 6]);
         L.d = (double *)(B + o[10 * l + 7]);
-        L.lam = (double *)(B + o[10 * l + 8]);
-        L.dforms = (DevForm *)(B + o[10 * l + 8] + 8);
+        L.ch = (MgCheb *)(B + o[10 * l + 8]);
+        L.dforms = (DevForm *)(B + o[10 * l + 8] + sizeof(MgCheb));
         L.val32 = (float *)(B + o[10 * l + 9]);
     }
     return off;
@@ -1582,7 +1613,7 @@ static void fill_desc(MgJob *j)
         B.b = L.b;
         B.r = L.r;
         B.d = L.d;
-        B.lam = L.lam;
+        B.ch = L.ch;
         B.n = L.n;
         B.N = L.in.N;
         B.fe = L.in.fe;
@@ -1613,7 +1644,7 @@ static void mg_job_pack(MgJob *j)
     const MgPack &P = j->hdesc.pack;
     for (int k = 0; k < P.nlev; ++k) {
         const MgLevel &L = j->lv[j->first_small + k];
-        const MgPackSrc S{L.in.A->rowptr, L.in.A->cols, L.val32, L.dinv, L.lam, L.in.A->fixed,
+        const MgPackSrc S{L.in.A->rowptr, L.in.A->cols, L.val32, L.dinv, L.ch, L.in.A->fixed,
                           nullptr, nullptr, nullptr, (int32_t)L.nnz, 0};
         hipLaunchKernelGGL(k_mg_pack, dim3(nblk(std::max(L.nnz, L.n + 1), 256)), dim3(256), 0, j->st, P.lv[k], S,
                            j->img);
@@ -1699,7 +1730,7 @@ static void rows_args(MgRows &a, const MgLevel &L, const MgJob *j)
     a.fixed = L.in.A->fixed;
     a.n = L.n;
     a.dinv = L.dinv;
-    a.lam = L.lam;
+    a.ch = L.ch;
     a.sc = j->sc;
 }
 
@@ -1736,10 +1767,10 @@ static void mg_restrict(MgJob *j, int l)
     const MgLevel &F = j->lv[l], &C = j->lv[l + 1];
     if (F.in.fe == GRMP_FE_H1P2)
         hipLaunchKernelGGL(k_mg_restrict_p2, dim3(nblk(C.n, 256)), dim3(256), 0, j->st, (int64_t)F.in.N, F.r,
-                           C.in.A->fixed, C.dinv, C.lam, C.b, C.d, j->sc);
+                           C.in.A->fixed, C.dinv, C.ch, C.b, C.d, j->sc);
     else
         hipLaunchKernelGGL(k_mg_restrict_p1, dim3(nblk(C.n, 256)), dim3(256), 0, j->st, (int64_t)F.in.N,
-                           (int64_t)C.in.N, F.in.ncomp, F.r, C.in.A->fixed, C.dinv, C.lam, C.b, C.d, j->sc);
+                           (int64_t)C.in.N, F.in.ncomp, F.r, C.in.A->fixed, C.dinv, C.ch, C.b, C.d, j->sc);
 }
 
 static void mg_prolong(MgJob *j, int l)
@@ -1797,6 +1828,8 @@ static void mg_vcycle(MgJob *j)
     }
 }
 
+static bool mg_job_p1(const MgJob *j) { return j->lv[0].in.fe == GRMP_FE_H1P1 && j->lv[0].in.ncomp == 1; }
+
 // FP32 values and Gershgorin bounds of all levels
 static void mg_job_prep(MgJob *j)
 {
@@ -1804,9 +1837,27 @@ static void mg_job_prep(MgJob *j)
     P.nlev = P.blocks = 0;
     for (int l = 0; l < j->nlev; ++l) {
         MgLevel &L = j->lv[l];
-        mg_prep_add(P, L.in.A->rowptr, L.val, L.dinv, L.in.A->fixed, L.val32, L.lam, L.n);
+        mg_prep_add(P, L.in.A->rowptr, L.val, L.dinv, L.in.A->fixed, L.val32, L.ch, L.n, mg_job_p1(j));
     }
     mg_prep_launch(P, j->st);
+    j->fourth = mg_job_p1(j);
+}
+
+// the hierarchy's coefficients for CG (fourth) or as MINRES' preconditioner,
+// if they are not those already
+static int mg_job_kind(MgJob *j, bool fourth)
+{
+    if (!mg_job_p1(j) || fourth == j->fourth) return GRMP_OK;
+    MgChebSet P;
+    P.n = 0;
+    P.fourth = fourth ? 1 : 0;
+    for (int l = 0; l < j->nlev; ++l) P.ch[P.n++] = j->lv[l].ch;
+    for (int k = 0; k < j->hdesc.pack.nlev; ++k)
+        P.ch[P.n++] = reinterpret_cast<MgCheb *>(j->img + j->hdesc.pack.lv[k].ch);
+    hipLaunchKernelGGL(k_mg_cheb_kind, dim3(1), dim3(64), 0, j->st, P);
+    GRMP_HIP(j->ctx, hipGetLastError());
+    j->fourth = fourth;
+    return GRMP_OK;
 }
 
 // level values, smoother bounds and the coarsest inverse: once per operator
@@ -1836,6 +1887,7 @@ static int mg_job_start(MgJob *j, double rtol, int maxit)
 {
     grmp_ctx *ctx = j->ctx;
     hipStream_t st = j->st;
+    GRMP_TRY(mg_job_kind(j, true));
     MgScal s0;
     memset(&s0, 0, sizeof(s0));
     s0.rtol = rtol;
@@ -1845,7 +1897,7 @@ static int mg_job_start(MgJob *j, double rtol, int maxit)
     GRMP_HIP(ctx, hipMemsetAsync(j->x, 0, n * 8, st));
     GRMP_HIP(ctx, hipMemsetAsync(j->p, 0, n * 8, st));
     hipLaunchKernelGGL(k_mg_start, dim3(nblk(n, 256)), dim3(256), 0, st, j->rhs, j->lv[0].in.A->fixed, j->lv[0].dinv,
-                       j->lv[0].lam, j->r, j->lv[0].d, n);
+                       j->lv[0].ch, j->r, j->lv[0].d, n);
     mg_vcycle(j);
     hipLaunchKernelGGL(k_mg_dot, dim3(j->nb0), dim3(KB), 0, st, j->r, j->r, n, j->part2, j->sc);
     hipLaunchKernelGGL(k_mg_red<RED_INIT>, dim3(1), dim3(MG_BT), 0, st, j->part, j->nb0, j->part2, j->sc);
@@ -1944,7 +1996,7 @@ static int mg_iterate_grid(MgJob *j, int iters)
         launch_rows<OP_PCG_Q>(j, a);
         hipLaunchKernelGGL(k_mg_red<RED_ALPHA>, dim3(1), dim3(MG_BT), 0, j->st, j->part, j->nb0, nullptr, j->sc);
         hipLaunchKernelGGL(k_mg_axpy, dim3(j->nb0), dim3(KB), 0, j->st, j->x, j->r, j->p, j->q, L0.in.A->fixed,
-                           L0.dinv, L0.lam, L0.d, n, j->part, j->sc);
+                           L0.dinv, L0.ch, L0.d, n, j->part, j->sc);
         hipLaunchKernelGGL(k_mg_red<RED_CONV>, dim3(1), dim3(MG_BT), 0, j->st, j->part, j->nb0, nullptr, j->sc);
         mg_vcycle(j);
         hipLaunchKernelGGL(k_mg_red<RED_BETA>, dim3(1), dim3(MG_BT), 0, j->st, j->part, j->nb0, nullptr, j->sc);
@@ -2422,7 +2474,7 @@ extern "C" int grmp_mg_apply(grmp_mg *m, const grmp_vector *b, grmp_vector *x, d
 // r_0 = v with the fixed rows zeroed and d0 of it; the device scalars are
 // reset so the V-cycle kernels run (a finished CG leaves done set)
 __global__ void k_mg_pc_in(const double *__restrict__ v, const uint8_t *__restrict__ fixed,
-                           const double *__restrict__ dinv, const double *__restrict__ lam, double *__restrict__ r,
+                           const double *__restrict__ dinv, const MgCheb *__restrict__ ch, double *__restrict__ r,
                            double *__restrict__ d, MgScal *__restrict__ sc, int64_t n, const int *__restrict__ skip)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2435,7 +2487,7 @@ __global__ void k_mg_pc_in(const double *__restrict__ v, const uint8_t *__restri
     const bool fx = fixed[i] != 0;
     const double ri = fx ? 0.0 : v[i];
     r[i] = ri;
-    d[i] = cheb_first(fx, dinv[i], ri, *lam);
+    d[i] = cheb_first(fx, dinv[i], ri, *ch);
 }
 
 int64_t mg_level0_rows(const grmp_mg *m) { return m->n; }
@@ -2499,13 +2551,15 @@ int mg_precond_apply_pair(grmp_mg *m, const double *v0, double *z0, const double
     MgJob *j = m->job, *j2 = m->job2;
     const int64_t n = m->n;
     GRMP_CHECK(m->ctx, st == j->st && j2, GRMP_ERR_ARG, "multigrid preconditioner pair: not prepared");
+    GRMP_TRY(mg_job_kind(j, false));
+    GRMP_TRY(mg_job_kind(j2, false));
     GRMP_HIP(m->ctx, hipEventRecord(m->fork, st));
     GRMP_HIP(m->ctx, hipStreamWaitEvent(m->st2, m->fork, 0));
     hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, m->st2, v1, m->A0->fixed, j2->lv[0].dinv,
-                       j2->lv[0].lam, j2->r, j2->lv[0].d, j2->sc, n, nullptr);
+                       j2->lv[0].ch, j2->r, j2->lv[0].d, j2->sc, n, nullptr);
     GRMP_TRY(mg_vcycle_into(j2, z1));
     hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, st, v0, m->A0->fixed, j->lv[0].dinv,
-                       j->lv[0].lam, j->r, j->lv[0].d, j->sc, n, nullptr);
+                       j->lv[0].ch, j->r, j->lv[0].d, j->sc, n, nullptr);
     GRMP_TRY(mg_vcycle_into(j, z0));
     GRMP_HIP(m->ctx, hipEventRecord(m->join, m->st2));
     GRMP_HIP(m->ctx, hipStreamWaitEvent(st, m->join, 0));
@@ -2518,7 +2572,8 @@ int mg_precond_apply(grmp_mg *m, const double *v, double *z, hipStream_t st)
     MgJob *j = m->job;
     const int64_t n = m->n;
     GRMP_CHECK(m->ctx, st == j->st, GRMP_ERR_ARG, "multigrid preconditioner: not the hierarchy's stream");
-    hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, st, v, m->A0->fixed, j->lv[0].dinv, j->lv[0].lam,
+    GRMP_TRY(mg_job_kind(j, false));
+    hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(n, 256)), dim3(256), 0, st, v, m->A0->fixed, j->lv[0].dinv, j->lv[0].ch,
                        j->r, j->lv[0].d, j->sc, n, nullptr);
     GRMP_TRY(mg_vcycle_into(j, z));
     GRMP_HIP(m->ctx, hipGetLastError());
@@ -2572,7 +2627,8 @@ struct AmgLevel {
     const double *val = nullptr;                 // level 0: the matrix's FP64 values
     const uint8_t *fixed = nullptr;              // coarse levels: all zero
     float *val32 = nullptr;
-    double *dinv = nullptr, *lam = nullptr;
+    double *dinv = nullptr;
+    MgCheb *ch = nullptr;
     double *x = nullptr, *b = nullptr, *r = nullptr, *d = nullptr;  // level 0: x = z, b = r of the CG
     int32_t *agg = nullptr;                      // row -> row of the next level (-1: fixed)
     int32_t *cagg = nullptr;                     // aggregate of each nonzero's column (fixed: the next level's n)
@@ -2822,7 +2878,7 @@ __global__ void k_amg_dinv(const double *__restrict__ diag, const uint8_t *__res
 // restriction b_c[I] = sum of r over the members of I, in row order; d_c = d0 of b_c
 __global__ void k_amg_restrict(const int32_t *__restrict__ mptr, const int32_t *__restrict__ midx,
                                const double *__restrict__ r, const uint8_t *__restrict__ fixed_c,
-                               const double *__restrict__ dinv_c, const double *__restrict__ lam_c,
+                               const double *__restrict__ dinv_c, const MgCheb *__restrict__ ch_c,
                                double *__restrict__ bc, double *__restrict__ dc, int64_t nc, const MgScal *sc)
 {
     if (sc->done) return;
@@ -2831,7 +2887,7 @@ __global__ void k_amg_restrict(const int32_t *__restrict__ mptr, const int32_t *
     double s = 0.0;
     for (int32_t k = mptr[I]; k < mptr[I + 1]; ++k) s += r[midx[k]];
     bc[I] = s;
-    dc[I] = cheb_first(fixed_c[I] != 0, dinv_c[I], s, *lam_c);
+    dc[I] = cheb_first(fixed_c[I] != 0, dinv_c[I], s, *ch_c);
 }
 
 // the aggregate of every nonzero's column, nc where the column is fixed (the
@@ -3139,13 +3195,13 @@ static int amg_level_smoother(grmp_amg *m, AmgLevel &L)
     double *diag = nullptr;
     GRMP_TRY(amg_alloc(m, &L.val32, L.nnz));
     GRMP_TRY(amg_alloc(m, &L.dinv, L.n));
-    GRMP_TRY(amg_alloc(m, &L.lam, 1));
+    GRMP_TRY(amg_alloc(m, &L.ch, 1));
     GRMP_TRY(dalloc(ctx, &diag, L.n));
     hipLaunchKernelGGL(k_amg_diag, dim3(nblk(L.n, 256)), dim3(256), 0, st, L.rp, L.ci, L.val, L.n, diag);
     hipLaunchKernelGGL(k_amg_dinv, dim3(nblk(L.n, 256)), dim3(256), 0, st, diag, L.fixed, L.n, L.dinv);
     MgPrep P;
     P.nlev = P.blocks = 0;
-    mg_prep_add(P, L.rp, L.val, L.dinv, L.fixed, L.val32, L.lam, L.n);
+    mg_prep_add(P, L.rp, L.val, L.dinv, L.fixed, L.val32, L.ch, L.n, false);
     mg_prep_launch(P, st);
     dfree(ctx, diag);
     GRMP_HIP(ctx, hipGetLastError());
@@ -3305,7 +3361,7 @@ static int amg_build(grmp_amg *m)
         for (int k = 0; k < m->pack.nlev; ++k) {
             const AmgLevel &L = m->lv[m->first + k];
             const AmgLevel *N = k + 1 < m->pack.nlev ? &m->lv[m->first + k + 1] : nullptr;
-            const MgPackSrc S{L.rp, L.ci, L.val32, L.dinv, L.lam, L.fixed, N ? L.agg : nullptr,
+            const MgPackSrc S{L.rp, L.ci, L.val32, L.dinv, L.ch, L.fixed, N ? L.agg : nullptr,
                               N ? N->mptr : nullptr, N ? N->midx : nullptr, (int32_t)L.nnz,
                               N ? (int32_t)N->n : 0};
             const int64_t items = std::max(std::max(L.nnz, L.n + 1), N ? N->n + 1 : (int64_t)0);
@@ -3333,7 +3389,7 @@ static void amg_rows(MgRows &a, const AmgLevel &L, const grmp_amg *m)
     a.fixed = L.fixed;
     a.n = L.n;
     a.dinv = L.dinv;
-    a.lam = L.lam;
+    a.ch = L.ch;
     a.sc = m->sc;
 }
 
@@ -3362,7 +3418,7 @@ static void amg_vcycle(grmp_amg *m)
         a.o1 = L.r;
         hipLaunchKernelGGL(k_mg_rows<OP_RESID>, dim3(nblk(L.n, KB)), dim3(KB), 0, st, a);
         hipLaunchKernelGGL(k_amg_restrict, dim3(nblk(C.n, 256)), dim3(256), 0, st, C.mptr, C.midx, L.r, C.fixed,
-                           C.dinv, C.lam, C.b, C.d, C.n, m->sc);
+                           C.dinv, C.ch, C.b, C.d, C.n, m->sc);
     }
     hipLaunchKernelGGL(k_amg_vcycle_block, dim3(1), dim3(MG_BT), m->pack.lds, st, m->pack, m->lv[F].b, m->lv[F].x,
                        m->sc);
@@ -3404,7 +3460,7 @@ static void amg_iterate(grmp_amg *m, int iters)
         a.part = m->part;
         hipLaunchKernelGGL(k_mg_rows<OP_PCG_Q>, dim3(nblk(n, KB)), dim3(KB), 0, st, a);
         hipLaunchKernelGGL(k_mg_red<RED_ALPHA>, dim3(1), dim3(MG_BT), 0, st, m->part, m->nb0, nullptr, m->sc);
-        hipLaunchKernelGGL(k_mg_axpy, dim3(m->nb0), dim3(KB), 0, st, m->x, m->r, m->p, m->q, L0.fixed, L0.dinv, L0.lam,
+        hipLaunchKernelGGL(k_mg_axpy, dim3(m->nb0), dim3(KB), 0, st, m->x, m->r, m->p, m->q, L0.fixed, L0.dinv, L0.ch,
                            L0.d, n, m->part, m->sc);
         hipLaunchKernelGGL(k_mg_red<RED_CONV>, dim3(1), dim3(MG_BT), 0, st, m->part, m->nb0, nullptr, m->sc);
         amg_vcycle(m);
@@ -3462,7 +3518,7 @@ int amg_precond_apply(grmp_amg *m, const double *v, double *z, hipStream_t st, c
     GRMP_CHECK(m->ctx, st == m->ctx->stream, GRMP_ERR_ARG,
                "algebraic multigrid preconditioner: not the hierarchy's stream");
     AmgLevel &L0 = m->lv[0];
-    hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(L0.n, 256)), dim3(256), 0, st, v, L0.fixed, L0.dinv, L0.lam, m->r, L0.d, m->sc,
+    hipLaunchKernelGGL(k_mg_pc_in, dim3(nblk(L0.n, 256)), dim3(256), 0, st, v, L0.fixed, L0.dinv, L0.ch, m->r, L0.d, m->sc,
                        L0.n, skip);
     // level 0 works in the caller's z (the cycle writes every row of it), so nothing is copied out
     double *own = L0.x;
