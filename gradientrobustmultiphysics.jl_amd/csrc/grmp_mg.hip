@@ -2890,6 +2890,71 @@ __global__ void k_amg_restrict(const int32_t *__restrict__ mptr, const int32_t *
     dc[I] = cheb_first(fixed_c[I] != 0, dinv_c[I], s, *ch_c);
 }
 
+// The residual and its restriction in one launch: four lanes a coarse row,
+// each a member's row (a level's free rows are all members; the fixed ones'
+// residual is not read), the sums in row order as above.  The rows are read
+// uncoalesced, out of L2 on the levels it is taken for, where two launches are
+// bound by their latency: a solve on 211^2 P2 15.9 -> 15.6 ms, the 256^2 Newton
+// loop 78.4 -> 77.4.  Limits of 2^15 / 2^17 / 2^19 rows and none: the 128^3 tets
+// 53.8 / 54.3 / 55.3 / 59.4 ms.
+#define AMG_RR_LANES 4
+#ifndef AMG_RR_ROWS
+#define AMG_RR_ROWS (1 << 15)
+#endif
+__global__ __launch_bounds__(256) void k_amg_resid_restrict(MgRows a, const int32_t *__restrict__ mptr,
+                                                            const int32_t *__restrict__ midx,
+                                                            const uint8_t *__restrict__ fixed_c,
+                                                            const double *__restrict__ dinv_c,
+                                                            const MgCheb *__restrict__ ch_c, double *__restrict__ bc,
+                                                            double *__restrict__ dc, int64_t nc)
+{
+    if (a.sc->done) return;
+    const int64_t I = ((int64_t)blockIdx.x * 256 + threadIdx.x) / AMG_RR_LANES;
+    const int q = threadIdx.x % AMG_RR_LANES;
+    if (I >= nc) return;
+    const int32_t *__restrict__ rp = a.rp, *__restrict__ ci = a.ci;
+    const float *__restrict__ val = a.val32;
+    const double *__restrict__ v = a.v;
+    const int32_t m0 = mptr[I], m1 = mptr[I + 1];
+    double s = 0.0;
+    for (int32_t k0 = m0; k0 < m1; k0 += AMG_RR_LANES) {
+        double ri = 0.0;
+        if (k0 + q < m1) {
+            const int32_t i = midx[k0 + q], e0 = rp[i], e1 = rp[i + 1];
+            const double bi = a.b[i];
+            double p = 0.0;
+            for (int32_t e = e0; e < e1; e += 8) {  // past the row's end its last entry again, unused
+                int32_t c[8];
+                float w[8];
+                double xv[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int32_t f = e + u < e1 ? e + u : e1 - 1;
+                    c[u] = ci[f];
+                    w[u] = val[f];
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) xv[u] = v[c[u]];
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (e + u < e1) p += (double)w[u] * xv[u];
+            }
+            ri = bi - p;
+            a.o1[i] = ri;
+        }
+        const int left = m1 - k0;
+#pragma unroll
+        for (int u = 0; u < AMG_RR_LANES; ++u) {
+            const double ru = __shfl(ri, u, AMG_RR_LANES);
+            if (u < left) s += ru;
+        }
+    }
+    if (q == 0) {
+        bc[I] = s;
+        dc[I] = cheb_first(fixed_c[I] != 0, dinv_c[I], s, *ch_c);
+    }
+}
+
 // the aggregate of every nonzero's column, nc where the column is fixed (the
 // coarse vectors hold a zero there)
 __global__ void k_amg_cagg(const int32_t *__restrict__ ci, const int32_t *__restrict__ agg, int64_t nnz, int32_t nc,
@@ -3416,6 +3481,11 @@ static void amg_vcycle(grmp_amg *m)
         a.v = L.x;
         a.b = L.b;
         a.o1 = L.r;
+        if (L.n <= AMG_RR_ROWS) {
+            hipLaunchKernelGGL(k_amg_resid_restrict, dim3(nblk(C.n * AMG_RR_LANES, 256)), dim3(256), 0, st, a, C.mptr,
+                               C.midx, C.fixed, C.dinv, C.ch, C.b, C.d, C.n);
+            continue;
+        }
         hipLaunchKernelGGL(k_mg_rows<OP_RESID>, dim3(nblk(L.n, KB)), dim3(KB), 0, st, a);
         hipLaunchKernelGGL(k_amg_restrict, dim3(nblk(C.n, 256)), dim3(256), 0, st, C.mptr, C.midx, L.r, C.fixed,
                            C.dinv, C.ch, C.b, C.d, C.n, m->sc);

@@ -154,3 +154,22 @@ def test_level_setup_matches_lu(grmp, O, spec):
         x = _reference(grmp, O, *spec, 7)
         err = np.linalg.norm(S.solution(t) - x) / np.linalg.norm(x)
         assert r.status == 0 and r.iterations <= 60 and err <= 1e-8, (r.status, r.iterations, err)
+
+
+# the fused residual and restriction up to 32,768 rows (P1 180^2 has 32,761),
+# two launches beyond; constant coefficients on generated squares
+@pytest.mark.parametrize("N", [20, 180, 181])
+def test_amg_resid_restrict_sizes(grmp, O, N):
+    """3e-8 against LU: the residual is 1e-12, the condition below 4/pi^2 N^2
+    8/3 < 3.6e4"""
+    print(f"[case] algebraic multigrid, P1 {N}x{N}", flush=True)
+    import scipy.sparse.linalg as spla
+    fes = grmp.FESpace(grmp.H1P1(1), grmp.grid_unitsquare(N))
+    pde = grmp.PoissonProblem(1.0)
+    pde.add_rhsdata(0, grmp.LinearForm(grmp.Identity, grmp.DataFunction([1.0])))
+    pde.add_boundarydata(0)
+    sol = grmp.FEVector([fes])
+    info, A, b = grmp.solve(sol, pde, solver="amg", rtol=1e-12)
+    x = spla.spsolve(A.to_scipy().tocsc(), b.entries())
+    err = np.linalg.norm(sol.entries() - x) / np.linalg.norm(x)
+    assert info.status == 0 and err <= 3e-8, (info.iterations, err)
