@@ -2662,16 +2662,28 @@ static int amg_alloc(grmp_amg *m, T **p, size_t count)
     return GRMP_OK;
 }
 
+// Lanes of a row in the aggregation's row scans: each entry is a chain of
+// dependent loads (the neighbour's state, and a search of its row where the
+// matrix is not symmetric), so the row's entries go side by side.  On the
+// 128^3 tetrahedra a choice on the symmetric fine level takes 184 us (one lane:
+// 382), on a coarse one 50 (109), the diagonal 15 (24); the solve 53.8 -> 51.1
+// ms.  Eight lanes measured the same.
+#ifndef AMG_LANES
+#define AMG_LANES 4
+#endif
 // diagonal of each row (0 if it has none)
 __global__ void k_amg_diag(const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
                            const double *__restrict__ val, int64_t n, double *__restrict__ diag)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / AMG_LANES;
+    const int q = threadIdx.x % AMG_LANES;
     if (i >= n) return;
-    double d = 0.0;
-    for (int32_t k = rp[i]; k < rp[i + 1]; ++k)
-        if (ci[k] == i) d = val[k];
-    diag[i] = d;
+    int32_t at = -1;
+    for (int32_t k = rp[i] + q; k < rp[i + 1]; k += AMG_LANES)
+        if (ci[k] == i) at = k;
+#pragma unroll
+    for (int o = 1; o < AMG_LANES; o <<= 1) at = max(at, __shfl_xor(at, o, AMG_LANES));
+    if (q == 0) diag[i] = at < 0 ? 0.0 : val[at];
 }
 
 // -(a_ij + a_ji) / 2: the strength of the pair (i, j) seen from both rows, so
@@ -2717,27 +2729,38 @@ __global__ void k_amg_best(const int32_t *__restrict__ rp, const int32_t *__rest
                            const uint8_t *__restrict__ fixed, const int32_t *__restrict__ mate, int64_t n,
                            double theta, int32_t *__restrict__ best)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / AMG_LANES;
+    const int q = threadIdx.x % AMG_LANES;
     if (i >= n) return;
     int32_t bj = -1;
-    if (mate[i] < 0 && !(fixed && fixed[i]) && diag[i] > 0.0) {
+    const double di = diag[i];
+    if (mate[i] < 0 && !(fixed && fixed[i]) && di > 0.0) {
         double bs = 0.0;
         uint64_t bk = 0;
-        for (int32_t k = rp[i]; k < rp[i + 1]; ++k) {
-            const int32_t j = ci[k];
-            if (j == i || mate[j] >= 0 || (fixed && fixed[j]) || !(diag[j] > 0.0)) continue;
-            const double st = (SYM ? -val[k] : amg_pair_coupling(rp, ci, val, (int32_t)i, j, val[k])) /
-                              sqrt(diag[i] * diag[j]);
-            if (!(st > theta)) continue;
-            const uint64_t key = amg_pair_key((int32_t)i, j);
+        auto take = [&](double st, uint64_t key, int32_t j) {
             if (bj < 0 || st > bs || (st == bs && (key > bk || (key == bk && j < bj)))) {
                 bs = st;
                 bk = key;
                 bj = j;
             }
+        };
+        for (int32_t k = rp[i] + q; k < rp[i + 1]; k += AMG_LANES) {
+            const int32_t j = ci[k];
+            if (j == i || mate[j] >= 0 || (fixed && fixed[j]) || !(diag[j] > 0.0)) continue;
+            const double st = (SYM ? -val[k] : amg_pair_coupling(rp, ci, val, (int32_t)i, j, val[k])) /
+                              sqrt(di * diag[j]);
+            if (!(st > theta)) continue;
+            take(st, amg_pair_key((int32_t)i, j), j);
+        }
+#pragma unroll
+        for (int o = 1; o < AMG_LANES; o <<= 1) {  // the order is total, so the lanes' maxima give the row's
+            const double os = __shfl_xor(bs, o, AMG_LANES);
+            const uint64_t ok = __shfl_xor((unsigned long long)bk, o, AMG_LANES);
+            const int32_t oj = __shfl_xor(bj, o, AMG_LANES);
+            if (oj >= 0) take(os, ok, oj);
         }
     }
-    best[i] = bj;
+    if (q == 0) best[i] = bj;
 }
 
 // mutual choices pair up (each row writes only its own mate)
@@ -2757,24 +2780,34 @@ __global__ void k_amg_join(const int32_t *__restrict__ rp, const int32_t *__rest
                            const uint8_t *__restrict__ fixed, const int32_t *__restrict__ mate, int64_t n,
                            int32_t *__restrict__ join)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / AMG_LANES;
+    const int q = threadIdx.x % AMG_LANES;
     if (i >= n) return;
     int32_t bj = -1;
-    if (mate[i] < 0 && !(fixed && fixed[i]) && diag[i] > 0.0) {
+    const double di = diag[i];
+    if (mate[i] < 0 && !(fixed && fixed[i]) && di > 0.0) {
         double bs = 0.0;
-        for (int32_t k = rp[i]; k < rp[i + 1]; ++k) {
-            const int32_t j = ci[k];
-            if (j == i || mate[j] < 0 || (fixed && fixed[j]) || !(diag[j] > 0.0)) continue;
-            const double st = (SYM ? -val[k] : amg_pair_coupling(rp, ci, val, (int32_t)i, j, val[k])) /
-                              sqrt(diag[i] * diag[j]);
-            if (!(st > 0.0)) continue;
+        auto take = [&](double st, int32_t j) {
             if (bj < 0 || st > bs || (st == bs && j < bj)) {
                 bs = st;
                 bj = j;
             }
+        };
+        for (int32_t k = rp[i] + q; k < rp[i + 1]; k += AMG_LANES) {
+            const int32_t j = ci[k];
+            if (j == i || mate[j] < 0 || (fixed && fixed[j]) || !(diag[j] > 0.0)) continue;
+            const double st = (SYM ? -val[k] : amg_pair_coupling(rp, ci, val, (int32_t)i, j, val[k])) /
+                              sqrt(di * diag[j]);
+            if (st > 0.0) take(st, j);
+        }
+#pragma unroll
+        for (int o = 1; o < AMG_LANES; o <<= 1) {
+            const double os = __shfl_xor(bs, o, AMG_LANES);
+            const int32_t oj = __shfl_xor(bj, o, AMG_LANES);
+            if (oj >= 0) take(os, oj);
         }
     }
-    join[i] = bj;
+    if (q == 0) join[i] = bj;
 }
 
 // lead[i] = 1 for the first row of each pair and for rows left single
@@ -2992,25 +3025,25 @@ static int amg_pairwise(grmp_ctx *ctx, const int32_t *rp, const int32_t *ci, con
         if ((rc = dalloc(ctx, &diag, n)) || (rc = dalloc(ctx, &mate, n)) || (rc = dalloc(ctx, &best, n)) ||
             (rc = dalloc(ctx, &lead, n)) || (rc = dalloc(ctx, &id, n + 1)))
             break;
-        hipLaunchKernelGGL(k_amg_diag, dim3(nblk(n, 256)), dim3(256), 0, st, rp, ci, val, n, diag);
+        hipLaunchKernelGGL(k_amg_diag, dim3(nblk(n * AMG_LANES, 256)), dim3(256), 0, st, rp, ci, val, n, diag);
         if (hipMemsetAsync(mate, 0xff, sizeof(int32_t) * n, st) != hipSuccess) {
             rc = grmp_fail(ctx, GRMP_ERR_HIP, "AMG aggregation: memset");
             break;
         }
         for (int round = 0; round < 3; ++round) {
             if (sym)
-                hipLaunchKernelGGL(k_amg_best<true>, dim3(nblk(n, 256)), dim3(256), 0, st, rp, ci, val, diag, fixed,
+                hipLaunchKernelGGL(k_amg_best<true>, dim3(nblk(n * AMG_LANES, 256)), dim3(256), 0, st, rp, ci, val, diag, fixed,
                                    mate, n, AMG_THETA, best);
             else
-                hipLaunchKernelGGL(k_amg_best<false>, dim3(nblk(n, 256)), dim3(256), 0, st, rp, ci, val, diag, fixed,
+                hipLaunchKernelGGL(k_amg_best<false>, dim3(nblk(n * AMG_LANES, 256)), dim3(256), 0, st, rp, ci, val, diag, fixed,
                                    mate, n, AMG_THETA, best);
             hipLaunchKernelGGL(k_amg_match, dim3(nblk(n, 256)), dim3(256), 0, st, best, mate, n);
         }
         if (sym)
-            hipLaunchKernelGGL(k_amg_join<true>, dim3(nblk(n, 256)), dim3(256), 0, st, rp, ci, val, diag, fixed, mate, n,
+            hipLaunchKernelGGL(k_amg_join<true>, dim3(nblk(n * AMG_LANES, 256)), dim3(256), 0, st, rp, ci, val, diag, fixed, mate, n,
                                best);
         else
-            hipLaunchKernelGGL(k_amg_join<false>, dim3(nblk(n, 256)), dim3(256), 0, st, rp, ci, val, diag, fixed, mate,
+            hipLaunchKernelGGL(k_amg_join<false>, dim3(nblk(n * AMG_LANES, 256)), dim3(256), 0, st, rp, ci, val, diag, fixed, mate,
                                n, best);
         hipLaunchKernelGGL(k_amg_lead, dim3(nblk(n, 256)), dim3(256), 0, st, mate, best, fixed, n, lead);
         if ((rc = exclusive_scan_i32(ctx, lead, id, n))) break;
@@ -3262,7 +3295,7 @@ static int amg_level_smoother(grmp_amg *m, AmgLevel &L)
     GRMP_TRY(amg_alloc(m, &L.dinv, L.n));
     GRMP_TRY(amg_alloc(m, &L.ch, 1));
     GRMP_TRY(dalloc(ctx, &diag, L.n));
-    hipLaunchKernelGGL(k_amg_diag, dim3(nblk(L.n, 256)), dim3(256), 0, st, L.rp, L.ci, L.val, L.n, diag);
+    hipLaunchKernelGGL(k_amg_diag, dim3(nblk(L.n * AMG_LANES, 256)), dim3(256), 0, st, L.rp, L.ci, L.val, L.n, diag);
     hipLaunchKernelGGL(k_amg_dinv, dim3(nblk(L.n, 256)), dim3(256), 0, st, diag, L.fixed, L.n, L.dinv);
     MgPrep P;
     P.nlev = P.blocks = 0;
