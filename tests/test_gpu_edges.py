@@ -173,3 +173,27 @@ def test_amg_resid_restrict_sizes(grmp, O, N):
     x = spla.spsolve(A.to_scipy().tocsc(), b.entries())
     err = np.linalg.norm(sol.entries() - x) / np.linalg.norm(x)
     assert info.status == 0 and err <= 3e-8, (info.iterations, err)
+
+
+# 256 rows' columns are put together in LDS up to 6144 of them: hubs numbered
+# first, 21 (5355 and 235 rim rows of 4 are 6295) and 64 do not fit, 4 do; the
+# rim rows' blocks do
+@pytest.mark.parametrize("hubs,k", [(4, 254), (21, 254), (64, 254)])
+def test_pattern_columns_in_place(grmp, O, hubs, k):
+    """The pattern and values are the oracle's bit for bit."""
+    print(f"[case] pattern of {hubs} hubs of {k} cells", flush=True)
+    c0, e0 = _fan(k)
+    coords = np.vstack([c0[:1] + [5.0 * h, 0.0] for h in range(hubs)] +
+                       [c0[1:] + [5.0 * h, 0.0] for h in range(hubs)])
+    cells = np.vstack([np.where(e0 == 0, h, hubs + h * k + e0 - 1) for h in range(hubs)])
+    grid = grmp.ExtendableGrid.from_arrays(coords, cells)
+    fes = grmp.FESpace(grmp.H1P1(1), grid)
+    A = grmp.FEMatrix([fes])
+    form, keep = grmp.LaplaceOperator(0.7).form(fes, 0, 0, fes.ctx)
+    A.add_form(form, keep)
+    A.build_pattern()
+    A.assemble()
+    cp, rv, nz = A.csc()
+    ref = O.assemble_matrix(fes.ndofs, [dict(kind=O.BLF_LAPLACE, fe=O.FE_P1, quadorder=0, factor=0.7, coords=coords,
+                                             cells=cells, celldofs=cells)])
+    assert np.array_equal(cp, ref.colptr) and np.array_equal(rv, ref.rowval) and np.array_equal(nz, ref.nzval)
