@@ -197,3 +197,28 @@ def test_pattern_columns_in_place(grmp, O, hubs, k):
     ref = O.assemble_matrix(fes.ndofs, [dict(kind=O.BLF_LAPLACE, fe=O.FE_P1, quadorder=0, factor=0.7, coords=coords,
                                              cells=cells, celldofs=cells)])
     assert np.array_equal(cp, ref.colptr) and np.array_equal(rv, ref.rowval) and np.array_equal(nz, ref.nzval)
+
+
+# whole and partial blocks of 256 rows, and 1 to 24 incidences a dof, in fours
+# and not
+@pytest.mark.parametrize("n", [1, 2, 5, 6, 7])
+def test_tet_pattern_and_load_sizes(grmp, O, n):
+    """Pattern, values and load vector are the oracle's bit for bit."""
+    print(f"[case] tetrahedra n={n}", flush=True)
+    grid = grmp.grid_unitcube(n, 0.1, n)
+    c, cn = grid.download()
+    fes = grmp.FESpace(grmp.H1P1(1), grid)
+    A = grmp.FEMatrix([fes])
+    form, keep = grmp.LaplaceOperator(0.7).form(fes, 0, 0, fes.ctx)
+    A.add_form(form, keep)
+    A.build_pattern()
+    A.assemble()
+    cp, rv, nz = A.csc()
+    ref = O.assemble_matrix(fes.ndofs, [dict(kind=O.BLF_LAPLACE, geom=3, fe=O.FE_P1, quadorder=0, factor=0.7, coords=c,
+                                             cells=cn, celldofs=cn)])
+    assert np.array_equal(cp, ref.colptr) and np.array_equal(rv, ref.rowval) and np.array_equal(nz, ref.nzval)
+    b = grmp.FEVector([fes])
+    grmp.assemble_linearform(b, 0, grmp.LinearForm(grmp.Identity, grmp.DataFunction([1.5])))
+    bref = np.zeros(fes.ndofs)
+    O.assemble_lf_const(bref, O.FE_P1, 1, 1, [1.5], c, cn, cn, geom=3)
+    assert np.array_equal(b.entries(), bref)
