@@ -310,6 +310,7 @@ int mg_precond_apply_pair(grmp_mg *m, const double *v0, double *z0, const double
 int64_t mg_level0_rows(const grmp_mg *m);
 int mg_job_iterate(MgJob *j, int iters);
 int mg_job_verify(MgJob *j);         // after done == 2: check the true residual
+int mg_job_restart(MgJob *j);        // after done == 3: the restart a batch's check asked for
 bool mg_job_block(const MgJob *j);   // whole iterations in one workgroup (checks in place)
 void mg_job_set_stream(MgJob *j, hipStream_t st);
 int mg_job_status_async(MgJob *j, MgStatus *host);

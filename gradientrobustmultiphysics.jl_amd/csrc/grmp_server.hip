@@ -960,7 +960,7 @@ static void mg_batch_loop(grmp_server *S)
                 S->cv.notify_all();
                 continue;
             }
-            if (h.done == 2 && (rc = mg_job_verify(j->mg))) break;
+            if (h.done == 3 && (rc = mg_job_restart(j->mg))) break;
             keep.push_back(j);
         }
         if (rc) break;

@@ -222,3 +222,20 @@ def test_tet_pattern_and_load_sizes(grmp, O, n):
     bref = np.zeros(fes.ndofs)
     O.assemble_lf_const(bref, O.FE_P1, 1, 1, [1.5], c, cn, cn, geom=3)
     assert np.array_equal(b.entries(), bref)
+
+
+# Group setup: one request, a whole group and one more; single-level requests,
+# whole 256-row blocks and one row past them, levels in and out of LDS
+@pytest.mark.parametrize("count", [1, 16, 17])
+def test_group_setup_equals_alone(grmp, count):
+    """The same bits as each request set up and solved by itself"""
+    print(f"[case] setup of {count} requests", flush=True)
+    shapes = [(1, 1, 15), (1, 2, 33), (2, 1, 3), (1, 1, 2), (2, 1, 63), (1, 1, 16), (1, 2, 2), (1, 1, 127)]
+    reqs = [(*shapes[k % len(shapes)], 60 + k) for k in range(count)]
+    out = []
+    for kw in ({"mg_slots": 1, "mg_batch": 0}, {"mg_batch": 32, "mg_threads": 1}):
+        with grmp.Server("mg", mg_block_rows=1000, mg_coarse_rows=1000, **kw) as S:
+            ts = [S.submit(*r, rtol=1e-11) for r in reqs]
+            out.append([(S.wait(t).iterations, S.solution(t).copy()) for t in ts])
+    for r, (ia, xa), (ib, xb) in zip(reqs, *out):
+        assert ia == ib and np.array_equal(xa, xb), r
