@@ -959,27 +959,51 @@ __device__ __forceinline__ double spmv_tile64(const KProb &pr, int row0, int row
     return acc;
 }
 
+// r64 = b - A64 x on free rows of row0 .. row1 (FP64); returns the partial r.r
+__device__ __forceinline__ double resid_tile(const KProb &pr, int row0, int row1, double *lds)
+{
+    double acc = 0.0;
+    for (int r0 = row0; r0 < row1; r0 += KB) {
+        const int r1 = r0 + KB < row1 ? r0 + KB : row1;
+        const double s = csr_rows_lds64(pr.rowptr, pr.cols, pr.val64, pr.x, r0, r1, lds);
+        const int i = r0 + (int)threadIdx.x;
+        if (i < r1) {
+            double ri = pr.fixed[i] ? 0.0 : pr.b[i] - s;
+            pr.r64[i] = ri;
+            acc += ri * ri;
+        }
+    }
+    return acc;
+}
+
+// the products of the iterating problems, and the FP64 residuals of those
+// between two sweeps.  In a launch of their own, which most steps found empty,
+// the residuals took 3.6 us of the 39 us step of 439,000 rows: solve 18.7 ->
+// 17.9 ms.
 __global__ __launch_bounds__(KB) void k_eng_spmv(ENGINE_ARGS)
 {
-    // SPMV_CAP floats; FP64 fallback tiles stage SPMV_CAP / 2 doubles in it
+    // SPMV_CAP floats; FP64 tiles stage SPMV_CAP / 2 doubles in it
     __shared__ __align__(16) float lds32[SPMV_CAP];
     unsigned long long myb = 0;
     const int nt = *ntiles;
     for (int t = blockIdx.x; t < nt; t += gridDim.x) {
         const KTile tl = T[t];
         const int pi = tl.prob;
-        if (P[pi].phase != PH_ITER) continue;
+        const int ph = P[pi].phase;
+        if (ph != PH_ITER && ph != PH_RESID) continue;
         const KProb pr = P[pi];
-        double acc = pr.fp64 ? spmv_tile64(pr, tl.row0, tl.row1, (double *)lds32) : spmv_tile(pr, tl.row0, tl.row1, lds32);
+        double acc = ph == PH_RESID ? resid_tile(pr, tl.row0, tl.row1, (double *)lds32)
+                     : pr.fp64      ? spmv_tile64(pr, tl.row0, tl.row1, (double *)lds32)
+                                    : spmv_tile(pr, tl.row0, tl.row1, lds32);
         double dummy = 0.0;
         block_sum2(acc, dummy);
         if (threadIdx.x == 0) {
             part[2 * t] = acc;
-            // algorithmic bytes of this tile: values + columns, row pointers, x gather, y write
+            // algorithmic bytes of this tile: values + columns, row pointers, x gather, y write (residual: b too)
             const unsigned long long rows = (unsigned long long)(tl.row1 - tl.row0);
             const unsigned long long nz = (unsigned long long)(pr.rowptr[tl.row1] - pr.rowptr[tl.row0]);
-            const unsigned long long sv = pr.fp64 ? 8ull : 4ull;
-            myb += nz * (sv + 4ull) + 4ull * (rows + 1) + 2ull * sv * rows;
+            const unsigned long long sv = pr.fp64 || ph == PH_RESID ? 8ull : 4ull;
+            myb += nz * (sv + 4ull) + 4ull * (rows + 1) + (ph == PH_RESID ? 3ull : 2ull) * sv * rows;
         }
     }
     // per-block byte count, summed by k_eng_bytes (no atomics in the hot loop)
@@ -1110,38 +1134,6 @@ __global__ __launch_bounds__(KB) void k_eng_elem(ENGINE_ARGS)
     }
 }
 
-// r64 = b - A64 x on free rows of row0 .. row1 (FP64); returns the partial r.r
-__device__ __forceinline__ double resid_tile(const KProb &pr, int row0, int row1, double *lds)
-{
-    double acc = 0.0;
-    for (int r0 = row0; r0 < row1; r0 += KB) {
-        const int r1 = r0 + KB < row1 ? r0 + KB : row1;
-        const double s = csr_rows_lds64(pr.rowptr, pr.cols, pr.val64, pr.x, r0, r1, lds);
-        const int i = r0 + (int)threadIdx.x;
-        if (i < r1) {
-            double ri = pr.fixed[i] ? 0.0 : pr.b[i] - s;
-            pr.r64[i] = ri;
-            acc += ri * ri;
-        }
-    }
-    return acc;
-}
-
-__global__ __launch_bounds__(KB) void k_eng_resid(ENGINE_ARGS)
-{
-    __shared__ double lds[SPMV_CAP64];
-    const int nt = *ntiles;
-    for (int t = blockIdx.x; t < nt; t += gridDim.x) {
-        const KTile tl = T[t];
-        const int pi = tl.prob;
-        if (P[pi].phase != PH_RESID) continue;
-        const KProb pr = P[pi];
-        double acc = resid_tile(pr, tl.row0, tl.row1, lds), dummy = 0.0;
-        block_sum2(acc, dummy);
-        if (threadIdx.x == 0) part[2 * t] = acc;
-    }
-}
-
 // sums the tile partials of problem s in a fixed order (valid in thread 0)
 __device__ __forceinline__ void sum_parts(const KRange &rg, const double *part, double &a, double &b)
 {
@@ -1166,16 +1158,15 @@ __global__ __launch_bounds__(KB) void k_eng_reduce(KProb *__restrict__ P, const 
         const KRange rg = R[s];
         if (rg.nt == 0) continue;
         const int ph = P[s].phase;
-        if (WHICH == RED_A || WHICH == RED_B) {
-            if (ph != PH_ITER) continue;
-        } else if (ph != PH_UPDATE && ph != PH_INIT && ph != PH_REINIT && ph != PH_RESID && ph != PH_INIT64) {
+        if (WHICH == RED_A ? ph != PH_ITER && ph != PH_RESID
+            : WHICH == RED_B ? ph != PH_ITER
+                             : ph != PH_UPDATE && ph != PH_INIT && ph != PH_REINIT && ph != PH_INIT64)
             continue;
-        }
         double a = 0.0, b = 0.0;
         if (!(WHICH == RED_C && ph == PH_UPDATE)) sum_parts(rg, part, a, b);
         if (threadIdx.x != 0) continue;
         KProb &w = P[s];
-        if (WHICH == RED_A) {
+        if (WHICH == RED_A && ph == PH_ITER) {
             // a = p.q
             // Non-finite FP32 values with finite FP64 data are an overflow of
             // the inner recurrence (it can diverge at the FP64 noise floor):
@@ -1236,9 +1227,9 @@ __global__ __launch_bounds__(KB) void k_eng_reduce(KProb *__restrict__ P, const 
                     w.phase = PH_UPDATE;
                 }
             }
-        } else if (ph == PH_UPDATE) {
+        } else if (WHICH == RED_C && ph == PH_UPDATE) {
             w.phase = PH_RESID;
-        } else if (ph == PH_INIT || ph == PH_REINIT || ph == PH_INIT64) {
+        } else if (WHICH == RED_C) {
             w.rz = a;
             w.rmax = sqrt(b);
             w.phase = PH_ITER;
@@ -1443,7 +1434,6 @@ void KEngine::launch_kernels(int grid, bool timed)
     hipLaunchKernelGGL(k_eng_axpy, g, b, 0, st_, dP_, dT_, dR_, dpart_, dnt_, dbytes_);
     hipLaunchKernelGGL(k_eng_reduce<RED_B>, gr, b, 0, st_, dP_, dR_, dpart_, cap_p_);
     hipLaunchKernelGGL(k_eng_elem, g, b, 0, st_, dP_, dT_, dR_, dpart_, dnt_, dbytes_);
-    hipLaunchKernelGGL(k_eng_resid, g, b, 0, st_, dP_, dT_, dR_, dpart_, dnt_, dbytes_);
     hipLaunchKernelGGL(k_eng_reduce<RED_C>, gr, b, 0, st_, dP_, dR_, dpart_, cap_p_);
 }
 
