@@ -537,7 +537,8 @@ typedef struct grmp_kernel_stats {
                                  SpMV (mode 1), the multigrid residual on levels of >= 2^21 rows (mode 3) */
     int64_t spmv_launches;
     double spmv_bytes;        /* algorithmic bytes of those launches (engine: nnz*(4+4) + 4(n+1) + 4n (x)
-                                 + 4n (y) per row tile; multigrid residual: nnz*(8+4) + 4(n+1) + 8n (x)
+                                 + 4n (y) per row tile, FP64 residuals in the same launches
+                                 nnz*(8+4) + 4(n+1) + 24n (x, b, r); multigrid residual: nnz*(8+4) + 4(n+1) + 8n (x)
                                  + 8n (b) + 8n (r) + n (fixed mask)) */
     int64_t steps;            /* engine steps run */
     int64_t templates;        /* problem shapes built (mesh + dofmap + pattern) */

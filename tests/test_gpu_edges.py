@@ -239,3 +239,22 @@ def test_group_setup_equals_alone(grmp, count):
             out.append([(S.wait(t).iterations, S.solution(t).copy()) for t in ts])
     for r, (ia, xa), (ib, xb) in zip(reqs, *out):
         assert ia == ib and np.array_equal(xa, xb), r
+
+
+# rtol below the floor of b - A x: the check in the batch asks for restarts,
+# up to three, and accepts within 100 rtol
+@pytest.mark.parametrize("rtol", [1e-14, 3e-15])
+def test_batch_restarts_equal_alone(grmp, rtol):
+    """The same bits, iterations and status as each request by itself"""
+    print(f"[case] restarts in a batch, rtol {rtol}", flush=True)
+    reqs = [(1, 1, 65, 3), (1, 2, 48, 4), (2, 1, 40, 5), (1, 1, 120, 6), (1, 1, 9, 7)]
+    out = []
+    for kw in ({"mg_slots": 1, "mg_batch": 0}, {"mg_batch": 8}, {"mg_batch": 8, "mg_threads": -1}):
+        with grmp.Server("mg", mg_block_rows=256, mg_coarse_rows=256, **kw) as S:
+            ts = [S.submit(*r, rtol=rtol) for r in reqs]
+            res = [S.wait(t) for t in ts]
+            out.append([(r.status, r.iterations, r.relres, S.solution(t).copy()) for r, t in zip(res, ts)])
+    assert any(o[2] > rtol for o in out[0])  # at least one was checked and restarted
+    for got in out[1:]:
+        for r, a, b in zip(reqs, out[0], got):
+            assert a[:3] == b[:3] and np.array_equal(a[3], b[3]), (r, a[:3], b[:3])
