@@ -1502,6 +1502,7 @@ extern "C" int grmp_matrix_destroy(grmp_matrix *A)
     for (auto &r : A->forms)
         if (r.qtab) (void)hipFree(r.qtab);
     dfree(A->ctx, A->fixed);
+    dfree(A->ctx, A->dforms);
     delete A;
     return GRMP_OK;
 }

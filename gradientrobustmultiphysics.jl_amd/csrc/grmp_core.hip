@@ -186,6 +186,18 @@ extern "C" int grmp_ctx_destroy(grmp_ctx *ctx)
     return GRMP_OK;
 }
 
+extern "C" int grmp_pool_usage(const grmp_ctx *ctx, int64_t *used, int64_t *held)
+{
+    if (!ctx || !ctx->pool || !used || !held) return GRMP_ERR_ARG;
+    uint64_t u = 0, h = 0;
+    if (hipMemPoolGetAttribute(ctx->pool, hipMemPoolAttrUsedMemCurrent, &u) != hipSuccess ||
+        hipMemPoolGetAttribute(ctx->pool, hipMemPoolAttrReservedMemCurrent, &h) != hipSuccess)
+        return GRMP_ERR_HIP;
+    *used = (int64_t)u;
+    *held = (int64_t)h;
+    return GRMP_OK;
+}
+
 extern "C" const char *grmp_last_error(const grmp_ctx *ctx) { return ctx ? ctx->err.c_str() : "null context"; }
 
 extern "C" int grmp_ctx_synchronize(grmp_ctx *ctx)

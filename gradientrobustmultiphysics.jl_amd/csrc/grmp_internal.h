@@ -98,6 +98,9 @@ void dfree(grmp_ctx *ctx, T *&p)
     p = nullptr;
 }
 int ensure_scratch(grmp_ctx *ctx, size_t bytes);
+// bytes of the context's pool in use, and in all (with the freed blocks it
+// keeps); for the tests, not part of the public interface
+extern "C" int grmp_pool_usage(const grmp_ctx *ctx, int64_t *used, int64_t *held);
 
 // ------------------------------------------------------------------ objects
 struct grmp_vector {
