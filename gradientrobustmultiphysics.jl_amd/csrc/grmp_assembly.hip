@@ -1408,7 +1408,7 @@ int form_resolve(grmp_matrix *A, FormRec &r)
             tab[3 * q + 1] = xq[q][1];
             tab[3 * q + 2] = wq[q];
         }
-        GRMP_HIP(ctx, hipMalloc((void **)&r.qtab, sizeof(double) * tab.size()));
+        GRMP_HIP(ctx, ctx_malloc_fixed(ctx, (void **)&r.qtab, sizeof(double) * tab.size()));
         GRMP_HIP(ctx, hipMemcpy(r.qtab, tab.data(), sizeof(double) * tab.size(), hipMemcpyHostToDevice));
         r.nqt = nqt;
         r.kind = rs->fe == GRMP_FE_H1P1 ? FK_NLDIFF_P1TRI : FK_NLDIFF_P2TRI;

@@ -15,7 +15,9 @@
 #include <chrono>
 #include <cstdarg>
 #include <cstring>
+#include <map>
 
+#include "grmp_alloc.h"
 #include "grmp_internal.h"
 
 double wall_seconds()
@@ -127,6 +129,79 @@ extern "C" int grmp_tune_load(grmp_ctx *ctx, const char *path)
 
 extern "C" int grmp_tune_count(const grmp_ctx *ctx) { return ctx ? (int)ctx->tune.size() : -1; }
 
+// ------------------------------------------------------- device memory
+// The pool of a device and the contexts that use it.  The table lives until
+// the process ends: contexts may outlast static objects.
+struct DevicePool {
+    hipMemPool_t pool = nullptr;
+    int users = 0;
+};
+static std::mutex pool_mu;
+static std::map<int, DevicePool> &device_pools()
+{
+    static std::map<int, DevicePool> *m = new std::map<int, DevicePool>();
+    return *m;
+}
+
+// nullptr: no pool can be made; the context uses the default one
+static hipMemPool_t pool_acquire(int device)
+{
+    std::lock_guard<std::mutex> g(pool_mu);
+    DevicePool &D = device_pools()[device];
+    if (!D.pool) {
+        hipMemPoolProps props;
+        memset(&props, 0, sizeof(props));
+        props.allocType = hipMemAllocationTypePinned;
+        props.location.type = hipMemLocationTypeDevice;
+        props.location.id = device;
+        size_t mfree = 0, mtotal = 0;
+        if (hipMemPoolCreate(&D.pool, &props) != hipSuccess) {
+            D.pool = nullptr;
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        uint64_t keep = hipMemGetInfo(&mfree, &mtotal) == hipSuccess ? mtotal / 32 : 0;
+        (void)hipMemPoolSetAttribute(D.pool, hipMemPoolAttrReleaseThreshold, &keep);
+    }
+    ++D.users;
+    return D.pool;
+}
+
+// the context's stream has passed its last free
+static void pool_release(int device, hipMemPool_t pool)
+{
+    if (!pool) return;
+    std::lock_guard<std::mutex> g(pool_mu);
+    DevicePool &D = device_pools()[device];
+    if (--D.users > 0) {
+        (void)hipMemPoolTrimTo(D.pool, 0);
+        return;
+    }
+    (void)hipMemPoolDestroy(D.pool);
+    D.pool = nullptr;
+}
+
+// gives the pool's free blocks back, those freed on the stream st included
+static void pool_trim(grmp_ctx *ctx, hipStream_t st)
+{
+    (void)hipGetLastError();
+    (void)hipStreamSynchronize(st);
+    hipMemPool_t pool = ctx->pool;
+    if (pool || hipDeviceGetDefaultMemPool(&pool, ctx->device) == hipSuccess) (void)hipMemPoolTrimTo(pool, 0);
+}
+
+hipError_t ctx_malloc(grmp_ctx *ctx, void **p, size_t bytes, hipStream_t st)
+{
+    return alloc_or_release(
+        [&] { return ctx->pool ? hipMallocFromPoolAsync(p, bytes, ctx->pool, st) : hipMallocAsync(p, bytes, st); },
+        [&] { pool_trim(ctx, st); });
+}
+
+hipError_t ctx_malloc_fixed(grmp_ctx *ctx, void **p, size_t bytes)
+{
+    return alloc_or_release([&] { return hipMalloc(p, bytes); }, [&] { pool_trim(ctx, ctx->stream); });
+}
+
 extern "C" int grmp_ctx_create(int device, grmp_ctx **out)
 {
     if (!out) return GRMP_ERR_ARG;
@@ -140,24 +215,12 @@ extern "C" int grmp_ctx_create(int device, grmp_ctx **out)
         delete c;
         return GRMP_ERR_HIP;
     }
-    if (hipMalloc(&c->dflag, 64) != hipSuccess ||
+    c->pool = pool_acquire(device);
+    if (ctx_malloc_fixed(c, (void **)&c->dflag, 64) != hipSuccess ||
         hipHostMalloc((void **)&c->pin, GRMP_PIN_BYTES, hipHostMallocDefault) != hipSuccess ||
         hipEventCreate(&c->asm_ev[0]) != hipSuccess || hipEventCreate(&c->asm_ev[1]) != hipSuccess) {
         grmp_ctx_destroy(c);
         return GRMP_ERR_OOM;
-    }
-    hipMemPoolProps props;
-    memset(&props, 0, sizeof(props));
-    props.allocType = hipMemAllocationTypePinned;
-    props.location.type = hipMemLocationTypeDevice;
-    props.location.id = device;
-    size_t mfree = 0, mtotal = 0;
-    if (hipMemPoolCreate(&c->pool, &props) == hipSuccess) {
-        uint64_t keep = hipMemGetInfo(&mfree, &mtotal) == hipSuccess ? mtotal / 32 : 0;
-        (void)hipMemPoolSetAttribute(c->pool, hipMemPoolAttrReleaseThreshold, &keep);
-    } else {
-        c->pool = nullptr;  // the default pool then
-        (void)hipGetLastError();
     }
     // the shipped tuning table, when present (a missing file keeps the built-in launch shapes)
     const std::string fn = tune_default_path();
@@ -180,7 +243,7 @@ extern "C" int grmp_ctx_destroy(grmp_ctx *ctx)
     for (hipEvent_t e : ctx->asm_ev)
         if (e) (void)hipEventDestroy(e);
     (void)hipStreamSynchronize(ctx->stream);
-    if (ctx->pool) (void)hipMemPoolDestroy(ctx->pool);
+    pool_release(ctx->device, ctx->pool);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return GRMP_OK;

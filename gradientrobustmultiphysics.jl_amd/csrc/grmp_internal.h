@@ -40,12 +40,16 @@ struct grmp_ctx {
     void *scratch = nullptr;
     size_t scratch_bytes = 0;
     int *dflag = nullptr;  // device error/overflow flag
-    // Stream-ordered allocations come from this pool.  It keeps up to 1/32 of
-    // the device's memory (9 GB) of freed blocks for the next call; the
-    // default pool gives every free block back at each synchronization, and
-    // mapping them anew took longer than many kernels: with the pool (and fewer
-    // synchronizations) the 128^3 tets' solve went from 69.4 to 55.3 ms.
-    // The rest goes back at synchronizations, the pool with its context.
+    // Stream-ordered allocations come from this pool, one for all contexts of a
+    // device.  It keeps up to 1/32 of the device's memory (9 GB) of freed
+    // blocks for the next call; the default pool gives every free block back at
+    // each synchronization, and mapping them anew took longer than many
+    // kernels: with the pool (and fewer synchronizations) the 128^3 tets' solve
+    // went from 69.4 to 55.3 ms.  The rest goes back at synchronizations, every
+    // free block when a context is destroyed or an allocation finds no memory,
+    // the pool with the last context.  With a pool for each context the bound
+    // held for each (a server has ten), and blocks freed by one were of no use
+    // to the others.
     hipMemPool_t pool = nullptr;
     // page-locked scratch of the calls that read device scalars back; under mu
     char *pin = nullptr;
@@ -78,11 +82,11 @@ int grmp_fail(grmp_ctx *ctx, int code, const char *fmt, ...);
 
 #define GRMP_PIN_BYTES 65536  // bytes of grmp_ctx::pin
 
-// device allocation helpers (stream-ordered, from the context's pool)
-inline hipError_t ctx_malloc(grmp_ctx *ctx, void **p, size_t bytes, hipStream_t st)
-{
-    return ctx->pool ? hipMallocFromPoolAsync(p, bytes, ctx->pool, st) : hipMallocAsync(p, bytes, st);
-}
+// device allocation helpers: stream-ordered from the context's pool, and
+// hipMalloc; both give the pool's free blocks back and try once more before
+// they fail for lack of memory
+hipError_t ctx_malloc(grmp_ctx *ctx, void **p, size_t bytes, hipStream_t st);
+hipError_t ctx_malloc_fixed(grmp_ctx *ctx, void **p, size_t bytes);
 template <class T>
 int dalloc(grmp_ctx *ctx, T **p, size_t count)
 {

@@ -2321,9 +2321,9 @@ static int batch_reserve(MgBatch *b, size_t tiles, int reqs)
         if (b->hdesc) (void)hipHostFree((void *)b->hdesc);
         if (b->hreq) (void)hipHostFree(b->hreq);
         if (b->hstat) (void)hipHostFree(b->hstat);
-        GRMP_HIP(ctx, hipMalloc((void **)&b->ddesc, cap * sizeof(MgBDesc *)));
-        GRMP_HIP(ctx, hipMalloc((void **)&b->dreq, cap * sizeof(int32_t)));
-        GRMP_HIP(ctx, hipMalloc((void **)&b->dstat, cap * sizeof(MgStatus)));
+        GRMP_HIP(ctx, ctx_malloc_fixed(ctx, (void **)&b->ddesc, cap * sizeof(MgBDesc *)));
+        GRMP_HIP(ctx, ctx_malloc_fixed(ctx, (void **)&b->dreq, cap * sizeof(int32_t)));
+        GRMP_HIP(ctx, ctx_malloc_fixed(ctx, (void **)&b->dstat, cap * sizeof(MgStatus)));
         GRMP_HIP(ctx, hipHostMalloc((void **)&b->hdesc, cap * sizeof(MgBDesc *), hipHostMallocDefault));
         GRMP_HIP(ctx, hipHostMalloc((void **)&b->hreq, cap * sizeof(int32_t), hipHostMallocDefault));
         GRMP_HIP(ctx, hipHostMalloc((void **)&b->hstat, cap * sizeof(MgStatus), hipHostMallocDefault));

@@ -1321,13 +1321,13 @@ KEngine::~KEngine()
 int KEngine::init()
 {
     grmp_ctx *ctx = ctx_;
-    GRMP_HIP(ctx, hipMalloc(&dP_, sizeof(KProb) * cap_p_));
-    GRMP_HIP(ctx, hipMalloc(&dT_, sizeof(KTile) * cap_t_));
-    GRMP_HIP(ctx, hipMalloc(&dR_, sizeof(KRange) * cap_p_));
-    GRMP_HIP(ctx, hipMalloc(&dpart_, sizeof(double) * 2 * cap_t_));
-    GRMP_HIP(ctx, hipMalloc(&dnt_, sizeof(int)));
-    GRMP_HIP(ctx, hipMalloc(&dbytes_, sizeof(unsigned long long)));
-    GRMP_HIP(ctx, hipMalloc(&dbytes_blk_, sizeof(unsigned long long) * ENGINE_MAX_GRID));
+    GRMP_HIP(ctx, ctx_malloc_fixed(ctx, (void **)&dP_, sizeof(KProb) * cap_p_));
+    GRMP_HIP(ctx, ctx_malloc_fixed(ctx, (void **)&dT_, sizeof(KTile) * cap_t_));
+    GRMP_HIP(ctx, ctx_malloc_fixed(ctx, (void **)&dR_, sizeof(KRange) * cap_p_));
+    GRMP_HIP(ctx, ctx_malloc_fixed(ctx, (void **)&dpart_, sizeof(double) * 2 * cap_t_));
+    GRMP_HIP(ctx, ctx_malloc_fixed(ctx, (void **)&dnt_, sizeof(int)));
+    GRMP_HIP(ctx, ctx_malloc_fixed(ctx, (void **)&dbytes_, sizeof(unsigned long long)));
+    GRMP_HIP(ctx, ctx_malloc_fixed(ctx, (void **)&dbytes_blk_, sizeof(unsigned long long) * ENGINE_MAX_GRID));
     GRMP_HIP(ctx, hipMemsetAsync(dbytes_, 0, sizeof(unsigned long long), st_));
     for (auto &e : ev_) GRMP_HIP(ctx, hipEventCreate(&e));
     GRMP_HIP(ctx, hipHostMalloc((void **)&hP_, sizeof(KProb) * cap_p_, hipHostMallocDefault));

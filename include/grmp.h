@@ -154,7 +154,12 @@ typedef struct grmp_solve_info {
     double seconds;
 } grmp_solve_info;
 
-/* ------------------------------------------------------------- context */
+/* ------------------------------------------------------------- context
+ * The contexts of a device share one pool of device memory.  Between calls it
+ * keeps up to 1/32 of the device's memory in freed blocks (9 GB of 288), which
+ * other allocators of the process cannot use: they go back when a context is
+ * destroyed, the pool with the last one.  An allocation of this library that
+ * finds no memory gives them back and tries once more. */
 int grmp_ctx_create(int device, grmp_ctx **out);
 int grmp_ctx_destroy(grmp_ctx *ctx);
 const char *grmp_last_error(const grmp_ctx *ctx);
@@ -508,7 +513,10 @@ typedef struct grmp_result {
 typedef struct grmp_server_config {
     int mode;                 /* 1 = batched + FP32_IR (served), 2 = plain one-at-a-time FP64,
                                  3 = multigrid-preconditioned CG in FP64, mg_slots requests at once */
-    int64_t memory_budget;    /* bytes of HBM for resident problems */
+    int64_t memory_budget;    /* bytes of HBM for the buffers of requests in flight; resident shapes
+                                 (meshes, dofmaps, patterns) come on top, those that no request uses
+                                 kept up to half of it; so do the freed blocks of the contexts' pool
+                                 (grmp_ctx_create) */
     int max_active;           /* problems in flight */
     int graph;                /* capture the Krylov step (mode 1) or a request's chunk of CG
                                  iterations (mode 3) as a hipGraph */
