@@ -1502,7 +1502,7 @@ extern "C" int grmp_matrix_destroy(grmp_matrix *A)
     for (auto &r : A->forms)
         if (r.qtab) (void)hipFree(r.qtab);
     dfree(A->ctx, A->fixed);
-    dfree(A->ctx, A->dforms);
+    if (A->dforms) A->ctx->form_tables.push_back(A->dforms);
     delete A;
     return GRMP_OK;
 }
@@ -1600,7 +1600,11 @@ static int upload_forms(grmp_matrix *A, bool pattern)
             }
     }
     A->form_first[A->nblocks] = (int)h.size();
-    if (!A->dforms) GRMP_TRY(dalloc(ctx, &A->dforms, A->nblocks * MAXFORMS));
+    if (!A->dforms && !ctx->form_tables.empty()) {
+        A->dforms = (DevForm *)ctx->form_tables.back();
+        ctx->form_tables.pop_back();
+    }
+    if (!A->dforms) GRMP_TRY(dalloc(ctx, &A->dforms, 8 * MAXFORMS));  // of any matrix: up to 8 blocks
     GRMP_HIP(ctx, hipMemcpyAsync(A->dforms, h.data(), sizeof(DevForm) * h.size(), hipMemcpyHostToDevice, ctx->stream));
     return GRMP_OK;
 }

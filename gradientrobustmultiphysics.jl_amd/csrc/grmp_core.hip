@@ -238,6 +238,7 @@ extern "C" int grmp_ctx_destroy(grmp_ctx *ctx)
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->scratch) (void)hipFreeAsync(ctx->scratch, ctx->stream);
+    for (void *t : ctx->form_tables) (void)hipFreeAsync(t, ctx->stream);
     if (ctx->dflag) (void)hipFree(ctx->dflag);
     if (ctx->pin) (void)hipHostFree(ctx->pin);
     for (hipEvent_t e : ctx->asm_ev)

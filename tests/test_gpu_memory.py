@@ -18,8 +18,9 @@ def _usage(grmp, ctx):
 
 
 def test_destroyed_matrices_give_everything_back(grmp):
-    """After the first one (which grows the context's scratch) a matrix's life
-    leaves no byte of the pool in use."""
+    """After the first one (which grows the context's scratch and leaves its
+    table of forms for the next) a matrix's life leaves no byte of the pool in
+    use."""
     print("[case] matrices created, assembled and destroyed", flush=True)
     gc.collect()  # what other tests left behind
     grid = grmp.grid_unitsquare(9)
