@@ -297,7 +297,8 @@ struct MgStatus {            // host copy of the job's scalars
     int it, done, status, pad;
 };
 struct MgJob;
-int64_t mg_job_bytes(const MgLevelIn *in, int nlev);
+extern "C" int64_t mg_job_bytes(int nlev, const int64_t *n, const int64_t *nnz, const int64_t *nc, const int *N,
+                                int block_rows, int coarse_rows);
 // block_rows: a request with at most this many rows runs whole inside one
 // workgroup; coarse_rows: otherwise its levels with at most this many rows do;
 // graph: capture the grid-path chunk of iterations once and replay it

@@ -1660,6 +1660,7 @@ struct MgJob {
     MgScal *sc = nullptr;
     int nb0 = 0;
     int first_small = 0;      // first level that runs inside one workgroup
+    size_t img_bytes = 0;     // of its LDS image
     bool fourth = false;      // smoother coefficients of the fourth kind
     char *img = nullptr;      // LDS image of those levels
     MgBDesc hdesc;
@@ -1690,7 +1691,7 @@ static size_t mg_layout(MgJob *j, bool assign)
            o_q = take(n0 * 8), o_part = take(nb0 * 8), o_part2 = take(nb0 * 8), o_sc = take(sizeof(MgScal)),
            o_desc = take(sizeof(MgBDesc));
     const MgLevel &c = j->lv[j->nlev - 1];
-    size_t o_inv = take(c.n * c.n * 8), o_img = take(MG_LDS_MAX);
+    size_t o_inv = take(c.n * c.n * 8), o_img = take(j->img_bytes);
     std::vector<size_t> o(MG_MAX_LEVELS * 10);
     for (int l = 0; l < j->nlev; ++l) {
         const MgLevel &L = j->lv[l];
@@ -1739,19 +1740,6 @@ static size_t mg_layout(MgJob *j, bool assign)
     return off;
 }
 
-int64_t mg_job_bytes(const MgLevelIn *in, int nlev)
-{
-    MgJob j;
-    j.nlev = nlev;
-    for (int l = 0; l < nlev; ++l) {
-        j.lv[l].in = in[l];
-        j.lv[l].n = in[l].A->n;
-        j.lv[l].nnz = in[l].A->nnz;
-        j.lv[l].nc = in[l].sp->mesh->ncells;
-    }
-    return (int64_t)mg_layout(&j, false);
-}
-
 // the packed form of the levels from first_small on
 static bool mg_job_pack_layout(const MgJob *j, MgPack &P)
 {
@@ -1762,6 +1750,37 @@ static bool mg_job_pack_layout(const MgJob *j, MgPack &P)
                                              L.in.fe == GRMP_FE_H1P2 ? TR_P2 : TR_P1};
     }
     return mg_pack_layout(P, sh, j->nlev - j->first_small);
+}
+
+// the first level that may run inside one workgroup: a request with at most
+// block_rows rows runs whole in it, otherwise its levels with at most
+// coarse_rows rows do
+static int mg_first_small(const int64_t *n, int nlev, int block_rows, int coarse_rows)
+{
+    if (n[0] <= block_rows) return 0;
+    int f = nlev - 1;
+    while (f > 1 && n[f - 1] <= std::max(coarse_rows, MG_DENSE_MAX)) --f;
+    return f;
+}
+
+// Bytes of a job's buffer at most, for levels of n rows and up to nnz
+// nonzeros: which of them make up the LDS image depends on their nonzeros, so
+// it is counted with all that may.
+int64_t mg_job_bytes(int nlev, const int64_t *n, const int64_t *nnz, const int64_t *nc, const int *N, int block_rows,
+                     int coarse_rows)
+{
+    MgJob j;
+    j.nlev = nlev;
+    for (int l = 0; l < nlev; ++l) {
+        j.lv[l].n = n[l];
+        j.lv[l].nnz = nnz[l];
+        j.lv[l].nc = nc[l];
+        j.lv[l].in.N = N[l];
+    }
+    for (int l = mg_first_small(n, nlev, block_rows, coarse_rows); l < nlev; ++l)
+        j.img_bytes += 11 * n[l] + 6 * nnz[l] + sizeof(MgCheb) + 32;  // mg_pack_layout's arrays and their padding
+    j.img_bytes = std::min<size_t>(j.img_bytes, MG_LDS_MAX);
+    return (int64_t)mg_layout(&j, false);
 }
 
 static void fill_desc(MgJob *j)
@@ -1858,6 +1877,21 @@ int mg_job_create(grmp_ctx *ctx, hipStream_t st, const MgLevelIn *in, int nlev, 
         j->lv[l].nnz = in[l].A->nnz;
         j->lv[l].nc = in[l].sp->mesh->ncells;
     }
+    {
+        int64_t rows[MG_MAX_LEVELS];
+        for (int l = 0; l < nlev; ++l) rows[l] = j->lv[l].n;
+        j->first_small = mg_first_small(rows, nlev, block_rows, coarse_rows);
+    }
+    // a coarse end that does not fit LDS gives its finest levels to grid
+    // kernels: six launches of about 4.5 us against the 104 us that elasticity's
+    // 1,250 ... 32 rows took in device memory
+    MgPack P;
+    bool fits = mg_job_pack_layout(j, P);
+    while (!fits && j->first_small > 0 && j->first_small < nlev - 1) {
+        ++j->first_small;
+        fits = mg_job_pack_layout(j, P);
+    }
+    j->img_bytes = fits ? P.image : 0;
     j->bytes = mg_layout(j, false);
     hipError_t e = ctx_malloc(ctx, (void **)&j->buf, j->bytes, st);
     if (e != hipSuccess) {
@@ -1865,18 +1899,6 @@ int mg_job_create(grmp_ctx *ctx, hipStream_t st, const MgLevelIn *in, int nlev, 
         return grmp_fail(ctx, e == hipErrorOutOfMemory ? GRMP_ERR_OOM : GRMP_ERR_HIP, "multigrid: device buffer");
     }
     mg_layout(j, true);
-    // a request with at most block_rows rows runs whole in one workgroup;
-    // otherwise its levels with at most coarse_rows rows do
-    coarse_rows = std::max(coarse_rows, MG_DENSE_MAX);
-    j->first_small = nlev - 1;
-    if (j->lv[0].n <= block_rows) j->first_small = 0;
-    else
-        while (j->first_small > 1 && j->lv[j->first_small - 1].n <= coarse_rows) --j->first_small;
-    // a coarse end that does not fit LDS gives its finest levels to grid
-    // kernels: six launches of about 4.5 us against the 104 us that elasticity's
-    // 1,250 ... 32 rows took in device memory
-    MgPack P;
-    while (j->first_small > 0 && j->first_small < nlev - 1 && !mg_job_pack_layout(j, P)) ++j->first_small;
     fill_desc(j);
     if (mg_allow_lds(ctx, (const void *)k_mg_vcycle_block) || mg_allow_lds(ctx, (const void *)k_mg_pcg_block) ||
         mg_allow_lds(ctx, (const void *)k_mgb_vcycle_block) || mg_allow_lds(ctx, (const void *)k_mgb_pcg_block)) {

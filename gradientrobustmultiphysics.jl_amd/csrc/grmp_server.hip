@@ -70,6 +70,42 @@ extern "C" int64_t grmp_request_footprint(const grmp_request *r)
     return (int64_t)b;
 }
 
+// Levels of a multigrid request, (fe, N): its own, P1 on the same square when it
+// is P2, then P1 on ceil(N/2), ceil(N/4), ... down to N <= 4
+static std::vector<std::pair<int, int>> mg_request_levels(const grmp_request &r)
+{
+    const int fe0 = r.kind == GRMP_REQ_ELASTICITY ? GRMP_FE_H1P1 : r.fe;
+    std::vector<std::pair<int, int>> lev{{fe0, r.N}};
+    if (fe0 == GRMP_FE_H1P2) lev.push_back({GRMP_FE_H1P1, r.N});
+    for (int N = r.N; N > 4;) {
+        N = (N + 1) / 2;
+        lev.push_back({GRMP_FE_H1P1, N});
+    }
+    return lev;
+}
+
+// What a request reserves of the memory budget in mode 3: twice the footprint,
+// which covers the hierarchies of some thousand rows and more, and what the
+// hierarchy's buffer can take where that is more (fixed tables and the LDS
+// image of the small levels: a 16 x 16 P1 request takes 103 KB, twice its
+// footprint is 92).
+extern "C" int64_t mg_request_reserve(const grmp_request *r, int block_rows, int coarse_rows)
+{
+    std::vector<int64_t> n, nnz, nc;
+    std::vector<int> N;
+    for (const auto &lv : mg_request_levels(*r)) {
+        grmp_request q = *r;
+        q.fe = lv.first;
+        q.N = lv.second;
+        n.push_back(grmp_request_ndofs(&q));
+        nnz.push_back(req_nnz_bound(q));
+        nc.push_back(req_ncells(q));
+        N.push_back(q.N);
+    }
+    return std::max(2 * grmp_request_footprint(r), mg_job_bytes((int)n.size(), n.data(), nnz.data(), nc.data(), N.data(),
+                                                                block_rows, coarse_rows));
+}
+
 struct Template {
     int kind = 0, fe = 0, N = 0;
     grmp_mesh *mesh = nullptr;
@@ -557,25 +593,17 @@ static int mg_template(grmp_server *S, grmp_ctx *c, const grmp_request &r, Templ
     return GRMP_OK;
 }
 
-// Levels: the request's shape, P1 on the same square when it is P2, then P1
-// on ceil(N/2), ceil(N/4), ... down to N <= 4.  mg_build makes the shapes,
-// the job, its coefficient and right-hand side; the level assembly and the
-// first V-cycle follow (mg_prepare: for this job alone; the setup threads:
-// for a group of jobs with one assembly launch).
+// mg_build makes the shapes of the levels, the job, its coefficient and
+// right-hand side; the level assembly and the first V-cycle follow (mg_prepare:
+// for this job alone; the setup threads: for a group of jobs with one assembly
+// launch).
 static int mg_build(grmp_server *S, Job *j, grmp_ctx *c, bool prof)
 {
     hipStream_t st = c->stream;
     j->res.t_admit = now(S);
     const grmp_request &r = j->req;
     const int ncomp = r.kind == GRMP_REQ_ELASTICITY ? 2 : 1;
-    const int fe0 = r.kind == GRMP_REQ_ELASTICITY ? GRMP_FE_H1P1 : r.fe;
-    std::vector<std::pair<int, int>> shape;  // (fe, N)
-    shape.push_back({fe0, r.N});
-    if (fe0 == GRMP_FE_H1P2) shape.push_back({GRMP_FE_H1P1, r.N});
-    for (int N = r.N; N > 4;) {
-        N = (N + 1) / 2;
-        shape.push_back({GRMP_FE_H1P1, N});
-    }
+    const std::vector<std::pair<int, int>> shape = mg_request_levels(r);
     std::vector<MgLevelIn> in(shape.size());
     for (size_t l = 0; l < shape.size(); ++l) {
         grmp_request rl = r;
@@ -1150,8 +1178,9 @@ extern "C" int grmp_server_submit(grmp_server *S, const grmp_request *req, int64
     j->req = *req;
     memset(&j->res, 0, sizeof(j->res));
     // multigrid jobs hold the hierarchy's values and vectors besides the fine level's
-    j->footprint = grmp_request_footprint(req) * (S->cfg.mode == 3 ? 2 : 1);
-    if (S->cfg.mode != 2 && j->footprint > S->cfg.memory_budget) {
+    const int64_t least = grmp_request_footprint(req) * (S->cfg.mode == 3 ? 2 : 1);
+    j->footprint = S->cfg.mode == 3 ? mg_request_reserve(req, S->cfg.mg_block_rows, S->cfg.mg_coarse_rows) : least;
+    if (S->cfg.mode != 2 && least > S->cfg.memory_budget) {
         delete j;
         return grmp_fail(S->user, GRMP_ERR_ADMISSION, "grmp_server_submit: footprint %lld B exceeds the budget %lld B",
                          (long long)grmp_request_footprint(req), (long long)S->cfg.memory_budget);

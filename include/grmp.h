@@ -566,7 +566,10 @@ double grmp_server_clock(const grmp_server *s);
 /* engine counters since creation (profile = 1 for the SpMV timings) */
 int grmp_server_stats(grmp_server *s, grmp_kernel_stats *out);
 int grmp_server_destroy(grmp_server *s);
-/* footprint in bytes the server would reserve for a request */
+/* bytes of the budget that mode 1 reserves for a request; mode 3 reserves twice
+ * as much, or what its hierarchy's buffer can take where that is more (requests
+ * of up to some 2,000 rows: at most 160 KB more).  A request is refused when
+ * the budget is below the one or two footprints; admitted alone it always runs. */
 int64_t grmp_request_footprint(const grmp_request *req);
 int64_t grmp_request_ndofs(const grmp_request *req);
 

@@ -71,3 +71,57 @@ def test_closed_server_gives_its_memory_back(grmp):
         assert _usage(grmp, ctx)[1] > held0
     used1, held1 = _usage(grmp, ctx)
     assert used1 == used0 and held1 <= held0, (used0, held0, used1, held1)
+
+
+def _levels(grmp, kind, fe, N):
+    """(matrix, space, mesh) of a multigrid request's levels"""
+    shape = [(fe, N)] + ([(1, N)] if fe == 2 else [])
+    while N > 4:
+        N = (N + 1) // 2
+        shape.append((1, N))
+    out = []
+    for f, n in shape:
+        grid = grmp.grid_unitsquare(n)
+        fes = grmp.FESpace(grmp.H1P2(1) if f == 2 else grmp.H1P1(kind), grid)
+        op = grmp.LaplaceOperator(1.0) if kind == 1 else grmp.HookStiffnessOperator2D(1.0, 1.0)
+        A = grmp.FEMatrix([fes])
+        A.add_form(*op.form(fes, 0, 0, fes.ctx))
+        A.set_fixed(fes.boundary_dofs(), 1e60)
+        A.build_pattern()
+        out.append((A, fes, grid))
+    return out
+
+
+# one workgroup's LDS image with and without all levels (1,250 rows of
+# elasticity do not fit), the largest that run whole in one workgroup (P1 44, P2
+# 22, elasticity 31), one level
+@pytest.mark.parametrize("kind,fe,N", [(1, 1, 2), (1, 1, 4), (1, 1, 16), (1, 1, 35), (1, 1, 44), (1, 1, 64), (1, 1, 200),
+                                       (1, 2, 1), (1, 2, 9), (1, 2, 22), (1, 2, 40), (2, 1, 3), (2, 1, 16), (2, 1, 24),
+                                       (2, 1, 31), (2, 1, 64)])
+def test_multigrid_buffer_is_within_its_account(grmp, kind, fe, N):
+    """What a hierarchy allocates is at most what the server reserves for such a
+    request, and at most mg_job_bytes of its actual nonzeros.  (With the LDS
+    image at its largest size for all, P1 16x16 took 240 KB of 92 reserved.)"""
+    print(f"[case] multigrid buffer {kind} {fe} {N}", flush=True)
+    gc.collect()
+    lv = _levels(grmp, kind, fe, N)
+    ctx = lv[0][1].ctx
+    kappa0 = grmp.DeviceVector(ctx, lv[0][2].ncells)
+    kappa0.fill(1.0)
+    used0 = _usage(grmp, ctx)[0]
+    M = grmp.MultigridSolver(lv, kappa0)
+    taken = _usage(grmp, ctx)[0] - used0
+    del M
+
+    L = grmp.lib()
+    L.mg_request_reserve.restype = L.mg_job_bytes.restype = ctypes.c_int64
+    req = grmp.server.request(kind, fe, N, 1)
+    reserve = L.mg_request_reserve(ctypes.byref(req), 2048, 2048)
+    k = len(lv)
+    arr = lambda t, v: (t * k)(*v)
+    info = [a.info() for a, _, _ in lv]
+    bound = L.mg_job_bytes(k, arr(ctypes.c_int64, [i[0] for i in info]), arr(ctypes.c_int64, [i[1] for i in info]),
+                           arr(ctypes.c_int64, [g.ncells for _, _, g in lv]), arr(ctypes.c_int, [g.N for _, _, g in lv]),
+                           2048, 2048)
+    assert 0 < taken <= bound <= reserve, (taken, bound, reserve)
+    assert reserve >= 2 * grmp.server.footprint(kind, fe, N)
