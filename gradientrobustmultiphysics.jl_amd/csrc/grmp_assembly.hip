@@ -1670,6 +1670,7 @@ extern "C" int grmp_matrix_build_pattern(grmp_matrix *A)
     GRMP_TRY(dalloc(ctx, &A->diagpos, A->n));
     // rows of up to 32 columns (every P1 and P2 pattern of a regular mesh) leave 20 waves' sets in a CU's LDS,
     // longer ones 10; the last pass takes the slot map's 255
+    GRMP_TRY(ctx_pin(ctx));
     int *flags = reinterpret_cast<int *>(ctx->pin);
     int64_t *total = reinterpret_cast<int64_t *>(ctx->pin + 64);
     for (int big = 0;; ++big) {
@@ -1735,6 +1736,7 @@ extern "C" int grmp_matrix_assemble(grmp_matrix *A, int values)
             for (auto &r : A->forms)
                 if (r.f.row_block == rb) fill_devform(A, r, hf[k++]);
     }
+    GRMP_TRY(ctx_asm_events(ctx));
     hipEvent_t *ev = ctx->asm_ev;
     GRMP_HIP(ctx, hipEventRecord(ev[0], ctx->stream));
     for (int rb = 0; rb < A->nblocks; ++rb) {

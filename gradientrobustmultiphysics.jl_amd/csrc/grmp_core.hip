@@ -202,6 +202,19 @@ hipError_t ctx_malloc_fixed(grmp_ctx *ctx, void **p, size_t bytes)
     return alloc_or_release([&] { return hipMalloc(p, bytes); }, [&] { pool_trim(ctx, ctx->stream); });
 }
 
+int ctx_pin(grmp_ctx *ctx)
+{
+    if (!ctx->pin) GRMP_HIP(ctx, hipHostMalloc((void **)&ctx->pin, GRMP_PIN_BYTES, hipHostMallocDefault));
+    return GRMP_OK;
+}
+
+int ctx_asm_events(grmp_ctx *ctx)
+{
+    for (hipEvent_t &e : ctx->asm_ev)
+        if (!e) GRMP_HIP(ctx, hipEventCreate(&e));
+    return GRMP_OK;
+}
+
 extern "C" int grmp_ctx_create(int device, grmp_ctx **out)
 {
     if (!out) return GRMP_ERR_ARG;
@@ -216,9 +229,7 @@ extern "C" int grmp_ctx_create(int device, grmp_ctx **out)
         return GRMP_ERR_HIP;
     }
     c->pool = pool_acquire(device);
-    if (ctx_malloc_fixed(c, (void **)&c->dflag, 64) != hipSuccess ||
-        hipHostMalloc((void **)&c->pin, GRMP_PIN_BYTES, hipHostMallocDefault) != hipSuccess ||
-        hipEventCreate(&c->asm_ev[0]) != hipSuccess || hipEventCreate(&c->asm_ev[1]) != hipSuccess) {
+    if (ctx_malloc_fixed(c, (void **)&c->dflag, 64) != hipSuccess) {
         grmp_ctx_destroy(c);
         return GRMP_ERR_OOM;
     }

@@ -51,9 +51,13 @@ struct grmp_ctx {
     // held for each (a server has ten), and blocks freed by one were of no use
     // to the others.
     hipMemPool_t pool = nullptr;
-    // page-locked scratch of the calls that read device scalars back; under mu
+    // Page-locked scratch of the calls that read device scalars back, and the
+    // events that time grmp_matrix_assemble; under mu.  Made by the first call
+    // that needs them (ctx_pin, ctx_asm_events): most of a server's ten
+    // contexts never do (making them all: 0.64 ms to open a server and 1.4 to
+    // close it, against 0.36 and 0.29).
     char *pin = nullptr;
-    hipEvent_t asm_ev[2] = {nullptr, nullptr};  // timing of grmp_matrix_assemble
+    hipEvent_t asm_ev[2] = {nullptr, nullptr};
     // Device tables of the forms of destroyed matrices, for the next ones; under
     // mu, reused in the order of the stream, and as many as there were matrices
     // at once.  Freed with each matrix they leave nothing of a hierarchy's
@@ -93,6 +97,8 @@ int grmp_fail(grmp_ctx *ctx, int code, const char *fmt, ...);
 // they fail for lack of memory
 hipError_t ctx_malloc(grmp_ctx *ctx, void **p, size_t bytes, hipStream_t st);
 hipError_t ctx_malloc_fixed(grmp_ctx *ctx, void **p, size_t bytes);
+int ctx_pin(grmp_ctx *ctx);
+int ctx_asm_events(grmp_ctx *ctx);
 template <class T>
 int dalloc(grmp_ctx *ctx, T **p, size_t count)
 {

@@ -469,6 +469,7 @@ int minres_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solve_
         if ((rc = dalloc(ctx, &H.dS, 1))) break;
         if ((rc = dalloc(ctx, &H.part, MR_GRID_ROWS))) break;
         if ((rc = dalloc(ctx, &dsg, n))) break;
+        if ((rc = ctx_pin(ctx))) break;
         H.hS = reinterpret_cast<MrScal *>(ctx->pin);
         if (ir) {
             if ((rc = dalloc(ctx, &dsg32, n))) break;

@@ -473,6 +473,7 @@ int plain_cg_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solv
     GRMP_TRY(dalloc(ctx, &B.q, n));
     GRMP_TRY(dalloc(ctx, &B.part, 2 * PGRID_ROWS + 2));
     GRMP_TRY(dalloc(ctx, &B.dsc, 2));
+    GRMP_TRY(ctx_pin(ctx));
     B.hsc = reinterpret_cast<PlainScal *>(ctx->pin);
     double *r = B.r, *z = B.z, *p = B.p, *q = B.q, *part = B.part;
     PlainScal *dsc = B.dsc, *hsc = B.hsc;
@@ -787,6 +788,7 @@ int bicgstab_solve(grmp_matrix *A, const double *bd, double *xd, const grmp_solv
     } B{ctx};
     GRMP_TRY(dalloc(ctx, &B.w, 8 * (size_t)n + 2 * PGRID_ROWS + 2));
     GRMP_TRY(dalloc(ctx, &B.S, 1));
+    GRMP_TRY(ctx_pin(ctx));
     B.hp = reinterpret_cast<double *>(ctx->pin);
     double *r = B.w, *rh = r + n, *p = rh + n, *v = p + n, *s = v + n, *t = s + n, *ph = t + n, *sh = ph + n;
     double *part = sh + n, *fold = part + 2 * PGRID_ROWS;
