@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from test_gpu_mg import _reference
+from test_gpu_stokes import _stokes
 
 pytestmark = pytest.mark.gpu
 
@@ -228,15 +229,21 @@ def test_tet_pattern_and_load_sizes(grmp, O, n):
 # whole 256-row blocks and one row past them, levels in and out of LDS
 @pytest.mark.parametrize("count", [1, 16, 17])
 def test_group_setup_equals_alone(grmp, count):
-    """The same bits as each request set up and solved by itself"""
+    """The same bits as each request set up and solved by itself.  The one setup
+    thread is at work on a large request while the others come, so it takes them
+    in groups of 16: all were there before the first was begun."""
     print(f"[case] setup of {count} requests", flush=True)
     shapes = [(1, 1, 15), (1, 2, 33), (2, 1, 3), (1, 1, 2), (2, 1, 63), (1, 1, 16), (1, 2, 2), (1, 1, 127)]
     reqs = [(*shapes[k % len(shapes)], 60 + k) for k in range(count)]
     out = []
     for kw in ({"mg_slots": 1, "mg_batch": 0}, {"mg_batch": 32, "mg_threads": 1}):
         with grmp.Server("mg", mg_block_rows=1000, mg_coarse_rows=1000, **kw) as S:
+            S.submit(1, 2, 500, 59, keep_solution=False)
             ts = [S.submit(*r, rtol=1e-11) for r in reqs]
-            out.append([(S.wait(t).iterations, S.solution(t).copy()) for t in ts])
+            res = [S.wait(t) for t in ts]
+            out.append([(r.iterations, S.solution(t).copy()) for r, t in zip(res, ts)])
+            if kw["mg_batch"]:
+                assert max(r.t_submit for r in res) < min(r.t_admit for r in res)
     for r, (ia, xa), (ib, xb) in zip(reqs, *out):
         assert ia == ib and np.array_equal(xa, xb), r
 
@@ -258,3 +265,131 @@ def test_batch_restarts_equal_alone(grmp, rtol):
     for got in out[1:]:
         for r, a, b in zip(reqs, out[0], got):
             assert a[:3] == b[:3] and np.array_equal(a[3], b[3]), (r, a[:3], b[:3])
+
+
+def _bicgstab(grmp, A, b, maxit, pc=None, rtol=1e-13):
+    """(status, iterations, relres, x) of BiCGStab stopped after maxit steps"""
+    import ctypes
+    o, info = grmp._abi.SolveOpts(), grmp._abi.SolveInfo()
+    L = grmp.lib()
+    L.grmp_solve_opts_default(ctypes.byref(o))
+    o.method, o.precision, o.rtol, o.maxit = grmp._abi.SOLVE_BICGSTAB, grmp._abi.PRECISION_FP64, rtol, maxit
+    x = grmp.DeviceVector(A.ctx, A.n)
+    if pc:
+        rc = L.grmp_solve_bicgstab_amg(A.h, b.h, x.h, ctypes.byref(o), pc.h, ctypes.byref(info))
+    else:
+        rc = L.grmp_solve(A.h, b.h, x.h, ctypes.byref(o), ctypes.byref(info))
+    assert rc == info.status
+    return info.status, info.iterations, info.relres, x.download()
+
+
+def _newton_matrix(grmp, n=9):
+    """A P2 Newton matrix (nonsymmetric) with its boundary fixed, a right-hand
+    side, and both on the host"""
+    fes = grmp.FESpace(grmp.H1P2(1), grmp.grid_unitsquare(n))
+    nlf = grmp.NonlinearForm(grmp.Gradient, [grmp.Identity, grmp.Gradient], [0, 0],
+                             grmp.NonlinearDiffusion(1.0, 0.0, 1.0), [2, 3], bonus_quadorder=2)
+    X = grmp.FEVector([fes])
+    X.set_entries(np.random.default_rng(3).standard_normal(fes.ndofs))
+    A = grmp.FEMatrix([fes])
+    A.add_form(*nlf.form(fes, 0, 0, fes.ctx, current=X))
+    A.set_fixed(fes.boundary_dofs())
+    A.assemble(grmp._abi.VALUES_FP64)
+    bh = np.random.default_rng(4).standard_normal(fes.ndofs)
+    b = grmp.DeviceVector(fes.ctx, fes.ndofs)
+    b.upload(bh)
+    free = np.ones(fes.ndofs, bool)
+    free[fes.boundary_dofs()] = False
+    return A, b, A.to_scipy().tocsr(), bh, free
+
+
+def _bicgstab_host(K, b, free, steps):
+    """x and |r| / |r_0| after steps of right-Jacobi BiCGStab on the free rows"""
+    d = K.diagonal()
+    x = np.where(free, 0.0, b / d)
+    mul = lambda v: np.where(free, K @ v, 0.0)
+    dinv = np.where(free, 1.0 / d, 0.0)
+    r = np.where(free, b - K @ x, 0.0)
+    rh, p, rho, r0 = r.copy(), r.copy(), r @ r, np.linalg.norm(r)
+    for _ in range(steps):
+        ph = dinv * p
+        v = mul(ph)
+        alpha = rho / (rh @ v)
+        s = r - alpha * v
+        sh = dinv * s
+        t = mul(sh)
+        omega = (s @ t) / (t @ t)
+        x = x + alpha * ph + omega * sh
+        r = s - omega * t
+        rho, old = rh @ r, rho
+        p = r + (rho / old) * (alpha / omega) * (p - omega * v)
+    return x, np.linalg.norm(r) / r0
+
+
+# BiCGStab's steps are enqueued two at a time: caps inside a pair and at its end
+@pytest.mark.parametrize("maxit", [1, 2, 3, 5])
+def test_bicgstab_iteration_cap(grmp, maxit):
+    """Exactly maxit steps, x and the residual those of the recurrence on the
+    host: 1e-12 (on the host, five steps in 64 and in 80 bits differ by 4e-16).
+    With a V-cycle the residual is that of the x returned: nothing enqueued
+    behind the last step touches it."""
+    print(f"[case] BiCGStab stopped after {maxit} steps", flush=True)
+    A, b, K, bh, free = _newton_matrix(grmp)
+    xh, relh = _bicgstab_host(K, bh, free, maxit)
+    st, it, rel, x = _bicgstab(grmp, A, b, maxit)
+    assert st == grmp._abi.ERR_NOCONV and it == maxit
+    assert np.linalg.norm(x - xh) <= 1e-12 * np.linalg.norm(xh) and abs(rel - relh) <= 1e-12, (rel, relh)
+    x0 = np.where(free, 0.0, bh / K.diagonal())
+    r0 = np.linalg.norm((bh - K @ x0)[free])
+    for pc in (None, grmp.AlgebraicMultigridSolver(A)):
+        st, it, rel, x = _bicgstab(grmp, A, b, maxit, pc)
+        true = np.linalg.norm((bh - K @ x)[free]) / r0
+        assert st == grmp._abi.ERR_NOCONV and it == maxit and abs(rel - true) <= 1e-12, (pc, rel, true)
+
+
+def test_bicgstab_ends(grmp):
+    """A right-hand side with a NaN ends at once; one free row converges in the
+    first half of a step (s = 0)."""
+    print("[case] BiCGStab ends", flush=True)
+    A, b, K, bh, free = _newton_matrix(grmp, 5)
+    bh[np.flatnonzero(free)[3]] = np.nan
+    b.upload(bh)
+    for pc in (None, grmp.AlgebraicMultigridSolver(A)):
+        st, it, rel, x = _bicgstab(grmp, A, b, 50, pc)
+        assert st == grmp._abi.ERR_NONFINITE and it == 0, (pc, st, it)
+    fes = grmp.FESpace(grmp.H1P1(1), grmp.grid_unitsquare(2))
+    A = grmp.FEMatrix([fes])
+    A.add_form(*grmp.LaplaceOperator(1.0).form(fes, 0, 0, fes.ctx))
+    A.set_fixed(fes.boundary_dofs())
+    A.assemble(grmp._abi.VALUES_FP64)
+    b = grmp.DeviceVector(fes.ctx, fes.ndofs)
+    b.upload(np.where(np.arange(fes.ndofs) == 4, 3.0, 0.0))
+    st, it, rel, x = _bicgstab(grmp, A, b, 50)
+    assert st == 0 and it == 1 and rel == 0.0 and np.array_equal(x, np.where(np.arange(9) == 4, 0.75, 0.0))
+
+
+# the whole hierarchy in one workgroup (P1 16^2) and grid levels over it (64^2)
+@pytest.mark.parametrize("N", [16, 64])
+def test_hierarchy_for_cg_and_minres_in_turn(grmp, N):
+    """CG takes the smoother's coefficients of the fourth kind, MINRES of the
+    first: each use gives the same bits before and after the other."""
+    print(f"[case] one hierarchy under CG, MINRES and CG, {N}x{N}", flush=True)
+    grid, V, Q, pde, sol = _stokes(grmp, N)
+    A, b, fixed = grmp.assemble(pde, sol)
+    M = grmp.stokes_velocity_mg(pde, V)
+    cfg = grmp.SolverConfig(rtol=1e-9)
+    f = grmp.FEVector([M.levels[0][1]])
+    f.set_entries(np.random.default_rng(N).standard_normal(f.n))
+
+    def cg():
+        x = grmp.FEVector([M.levels[0][1]])
+        info = M.solve(f, x, 1e-10)
+        return info.iterations, x.entries()
+
+    def minres():
+        info = grmp.solve_system(A, b, sol, cfg, grmp._abi.SOLVE_MINRES, velocity_mg=M)
+        return info.iterations, sol.entries().copy()
+
+    first, second = (cg(), minres()), (cg(), minres())
+    for (ia, xa), (ib, xb) in zip(first, second):
+        assert ia == ib and np.array_equal(xa, xb), (ia, ib)
