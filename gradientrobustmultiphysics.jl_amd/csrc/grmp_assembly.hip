@@ -888,7 +888,11 @@ __device__ __forceinline__ void pattern_put_forms(const FormPack &P, int64_t g, 
     }
 }
 
-#define PATTERN_COLS_CAP 6144  // 24 KB: 256 rows of 24 columns
+// 24 KB, 256 rows of 24 columns.  Smaller, blocks of a Stokes system's rows no
+// longer fit; larger gives nothing: 4096 / 6144 / 8192 take
+// 127 / 78 / 80 us on Stokes 512^2, 141 / 139 / 146 on P2 1023^2, 614 / 619 / 611 on
+// the 128^3 tetrahedra.
+#define PATTERN_COLS_CAP 6144
 __global__ __launch_bounds__(256) void k_pattern_cols(FormPack P, int64_t g0, int64_t g1, int64_t rblock,
                                                       const uint8_t *__restrict__ fixed,
                                                       const int32_t *__restrict__ rowptr,

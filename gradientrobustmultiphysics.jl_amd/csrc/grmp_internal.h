@@ -45,9 +45,14 @@ struct grmp_ctx {
     // blocks for the next call; the default pool gives every free block back at
     // each synchronization, and mapping them anew took longer than many
     // kernels: with the pool (and fewer synchronizations) the 128^3 tets' solve
-    // went from 69.4 to 55.3 ms.  The rest goes back at synchronizations, every
-    // free block when a context is destroyed or an allocation finds no memory,
-    // the pool with the last context.  With a pool for each context the bound
+    // went from 69.4 to 55.3 ms.  The rest goes back at synchronizations.  The
+    // runtime gives all free blocks back besides, whatever the bound, at a free
+    // that finds more memory free in the pool than in use (twelve blocks of 64
+    // MiB freed one after the other: at the eighth and the eleventh), 1.8 ms for
+    // 450 MiB: a program that holds little else than the solve itself spends 14
+    // of the tets' 65 ms and 9 of P2 1023^2's 37 on that.  Every free block also
+    // goes back when a context is destroyed or an allocation finds no memory, the
+    // pool with the last context.  With a pool for each context the bound
     // held for each (a server has ten), and blocks freed by one were of no use
     // to the others.
     hipMemPool_t pool = nullptr;

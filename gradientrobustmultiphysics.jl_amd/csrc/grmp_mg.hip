@@ -17,10 +17,11 @@
 // coarse triangulation (nested or not) and its exact transpose, both written
 // as gathers so that every sum has a fixed order; fixed dofs receive no
 // correction and carry no residual.  Smoothing is Chebyshev of degree 2 on
-// D^-1 A over [lmax/8, lmax] with lmax the Gershgorin bound of D^-1 A; the
-// coarsest level is solved exactly with its dense inverse.  Pre- and
-// post-smoothing are the same polynomial, so the V-cycle is symmetric and CG
-// applies.  All scalars live on the device; the host only polls a status
+// D^-1 A with lmax the Gershgorin bound of D^-1 A: of the first kind over
+// [lmax/8, lmax], or of the fourth kind on hierarchies of one P1 component
+// under CG (MgCheb).  The coarsest level is solved exactly with its dense
+// inverse.  Pre- and post-smoothing are the same polynomial, so the V-cycle is
+// symmetric and CG applies.  All scalars live on the device; the host only polls a status
 // copy.
 #include <algorithm>
 #include <cmath>
@@ -825,9 +826,9 @@ __device__ double blk_sum(double v)
 
 // The fixed-order sum of nb partials by one workgroup of MG_BT threads, the
 // same for a request alone and in a batch.  One workgroup, so bound by the
-// latency of its loads: eight are in flight per thread, which takes the 16,385
-// partials of 4.2M rows in two rounds (256 threads with one load at a time:
-// 17 us, and three of them an iteration).
+// latency of its loads: eight are in flight per thread, which takes the 16,401
+// partials of 4.2M rows in three rounds, 5.0 us (256 threads with one load at a
+// time: 17 us, and three of them an iteration).  Four loads: 5.3 us, sixteen 5.0.
 #define MG_RED_U 8
 __device__ double red_sum(const double *__restrict__ part, int nb)
 {
@@ -2545,7 +2546,8 @@ int mg_jobs_setup_batched(MgJob *const *jobs, int n, hipStream_t st, double *con
         return GRMP_OK;
     };
     const int rc = run();
-    if (rc) (void)hipStreamSynchronize(st);  // the upload reads h
+    // the upload reads h: on success assemble_batch, behind it, has waited for the stream
+    if (rc) (void)hipStreamSynchronize(st);
     (void)hipFreeAsync(d, st);
     return rc;
 }
@@ -2932,8 +2934,9 @@ extern "C" int grmp_mg_solve(grmp_ctx *ctx, int nlev, const grmp_matrix *const *
 //                 single when it has none.
 //                 No absolute threshold: on coarse 3D levels with 20-30
 //                 neighbours per row every normalized coupling is small.
-//   coarse level  the Galerkin product P^T A P of the piecewise-constant P:
-//                 every entry keyed (agg i, agg j), stably sorted, runs summed.
+//   coarse level  the Galerkin product P^T A P of the piecewise-constant P, a
+//                 thread a coarse row (rows of more than 255 columns: every
+//                 entry keyed (agg i, agg j), stably sorted, runs summed).
 //   cycle         V(1,1) with the Chebyshev smoothing of the geometric levels
 //                 (FP32-stored values, FP64 vectors), the coarse correction
 //                 scaled by AMG_SCALE (plain aggregation under-corrects smooth
@@ -2998,9 +3001,7 @@ static int amg_alloc(grmp_amg *m, T **p, size_t count)
 // 128^3 tetrahedra a choice on the symmetric fine level takes 184 us (one lane:
 // 382), on a coarse one 50 (109), the diagonal 15 (24); the solve 53.8 -> 51.1
 // ms.  Eight lanes measured the same.
-#ifndef AMG_LANES
 #define AMG_LANES 4
-#endif
 // diagonal of each row (0 if it has none)
 __global__ void k_amg_diag(const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
                            const double *__restrict__ val, int64_t n, double *__restrict__ diag)
@@ -3257,13 +3258,13 @@ __global__ void k_amg_restrict(const int32_t *__restrict__ mptr, const int32_t *
 // each a member's row (a level's free rows are all members; the fixed ones'
 // residual is not read), the sums in row order as above.  The rows are read
 // uncoalesced, out of L2 on the levels it is taken for, where two launches are
-// bound by their latency: a solve on 211^2 P2 15.9 -> 15.6 ms, the 256^2 Newton
-// loop 78.4 -> 77.4.  Limits of 2^15 / 2^17 / 2^19 rows and none: the 128^3 tets
-// 53.8 / 54.3 / 55.3 / 59.4 ms.
+// bound by their latency.  A CG iteration with no level / levels up to 2^15 / up to
+// 2^17 rows fused (best of eight solves, which differ by 0.5 %): P1 100^2 80.9 /
+// 78.6 / 78.7 us, P1 512^2 160.0 / 157.0 / 155.1, P2 211^2 141.6 / 139.5 / 138.5,
+// tets 50^3 209.4 / 206.2 / 207.1, 75^3 294.5 / 290.7 / 293.5.  On the 128^3 tets'
+// solve limits of 2^15 / 2^17 / 2^19 rows and none took 53.8 / 54.3 / 55.3 / 59.4 ms.
 #define AMG_RR_LANES 4
-#ifndef AMG_RR_ROWS
 #define AMG_RR_ROWS (1 << 15)
-#endif
 __global__ __launch_bounds__(256) void k_amg_resid_restrict(MgRows a, const int32_t *__restrict__ mptr,
                                                             const int32_t *__restrict__ midx,
                                                             const uint8_t *__restrict__ fixed_c,

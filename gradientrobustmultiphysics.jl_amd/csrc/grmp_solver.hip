@@ -283,7 +283,15 @@ __global__ __launch_bounds__(PB) void k_plain_beta(const double *__restrict__ pa
 // the fold kernels, and the direction update p = z + beta p happens where the
 // product gathers it: the same iterates, 7.08 -> 4.21 ms for the whole solve of
 // those rows.  Folding costs every workgroup a read of all partials, so it ends
-// at PLAIN_FUSE_GRID workgroups.
+// at PLAIN_FUSE_GRID workgroups.  An iteration of two and of five launches, us:
+//   workgroups       16     64    128    256    510   1024   2048   4096
+//   P1   two        9.8   10.0    9.9   10.8   13.4   19.5   30.7   60.2
+//        five      15.9   16.2   16.2   16.3   17.3   22.4   30.8   46.0
+//   P2   two                11.8          12.4   15.2   20.4   33.6   65.4
+//        five               16.3          16.9   18.9   25.1   32.2   49.7
+//   tets two                              15.2          25.9   48.3
+//        five                             19.4          27.6   41.4
+// They cross between 1024 and 2048 workgroups; the limit is below that.
 #define PLAIN_FUSE_GRID 512
 __device__ __forceinline__ void plain_fold_all(const double *__restrict__ part, int np, double &a, double &b)
 {
@@ -902,16 +910,16 @@ int zero_fixed_launch(const grmp_matrix *A, double *b, hipStream_t st)
 
 // ============================================================ the engine
 //
-// Step = 7 launches over the tile table:
+// Step = 6 launches over the tile table:
 //   spmv  (ITER)            q = A32 p, tile partials of p.q
-//   red A                   alpha = rz / p.q
+//         (RESID)           r64 = b - A64 x, tile partials r64.r64   (FP64)
+//   red A                   alpha = rz / p.q; the phase after RESID
 //   axpy  (ITER)            dx += alpha p, r -= alpha q, tile partials (r.z, r.r)
 //   red B                   convergence estimate, reliable-update trigger, beta
 //   elem  (ITER)            p = D r + beta p
 //         (UPDATE)          x += dx / s (FP64), and p = D r + beta p
 //         (INIT/REINIT)     r = s r64, dx = 0, p = D r | p *= s/s_old
-//   resid (RESID)           r64 = b - A64 x, tile partials r64.r64   (FP64)
-//   red C                   phase changes of elem / resid
+//   red C                   phase changes of elem
 // Tile kernels write one pair of partials per tile; the reduce kernels sum a
 // problem's partials in a fixed order (one block per problem).  Kernel
 // boundaries order the memory, so no fence or atomic is needed on the data
