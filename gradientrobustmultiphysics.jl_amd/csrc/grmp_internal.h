@@ -41,7 +41,7 @@ struct grmp_ctx {
     size_t scratch_bytes = 0;
     int *dflag = nullptr;  // device error/overflow flag
     // Stream-ordered allocations come from this pool, one for all contexts of a
-    // device.  It keeps up to 1/32 of the device's memory (9 GB) of freed
+    // device.  It keeps up to 1/16 of the device's memory (19 GB) of freed
     // blocks for the next call; the default pool gives every free block back at
     // each synchronization, and mapping them anew took longer than many
     // kernels: with the pool (and fewer synchronizations) the 128^3 tets' solve

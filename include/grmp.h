@@ -156,7 +156,7 @@ typedef struct grmp_solve_info {
 
 /* ------------------------------------------------------------- context
  * The contexts of a device share one pool of device memory.  Between calls it
- * keeps up to 1/32 of the device's memory in freed blocks (9 GB of 288), which
+ * keeps up to 1/16 of the device's memory in freed blocks (19 GB of 309), which
  * other allocators of the process cannot use: they go back when a context is
  * destroyed, the pool with the last one.  An allocation of this library that
  * finds no memory gives them back and tries once more. */
