@@ -334,6 +334,7 @@ int mg_pair_prepare(grmp_mg *m);
 int mg_precond_apply_pair(grmp_mg *m, const double *v0, double *z0, const double *v1, double *z1, hipStream_t st);
 int64_t mg_level0_rows(const grmp_mg *m);
 int mg_job_iterate(MgJob *j, int iters);
+double mg_job_margin(const MgJob *j);  // CG goes on to this part of rtol
 int mg_job_verify(MgJob *j);         // after done == 2: check the true residual
 int mg_job_restart(MgJob *j);        // after done == 3: the restart a batch's check asked for
 bool mg_job_block(const MgJob *j);   // whole iterations in one workgroup (checks in place)

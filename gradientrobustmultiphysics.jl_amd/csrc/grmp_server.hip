@@ -655,7 +655,7 @@ static int mg_start(grmp_server *S, Job *j, int slot)
 static int mg_chunk(const grmp_server *S, const Job *j, const MgStatus &h)
 {
     if (S->cfg.graph) return kMgChunk;
-    const double rtol = j->req.rtol > 0 ? j->req.rtol : 1e-10;
+    const double rtol = (j->req.rtol > 0 ? j->req.rtol : 1e-10) * mg_job_margin(j->mg);
     if (j->mg_it <= 0 || h.it <= j->mg_it || !(h.relres > 0.0) || !(h.relres < j->mg_rel)) return kMgChunk;
     const double rate = pow(h.relres / j->mg_rel, 1.0 / (h.it - j->mg_it));
     const double need = ceil(log(rtol / h.relres) / log(rate));

@@ -393,3 +393,27 @@ def test_hierarchy_for_cg_and_minres_in_turn(grmp, N):
     first, second = (cg(), minres()), (cg(), minres())
     for (ia, xa), (ib, xb) in zip(first, second):
         assert ia == ib and np.array_equal(xa, xb), (ia, ib)
+
+
+@pytest.mark.parametrize("N", [30, 200])
+def test_fourth_kind_goes_on_below_rtol(grmp, N):
+    """P1 hierarchies under CG stop at 0.4 rtol (the error at a given residual is
+    larger with their smoother); at the cap rtol itself is enough."""
+    print(f"[case] margin below rtol, P1 {N}x{N}", flush=True)
+    fes = grmp.FESpace(grmp.H1P1(1), grmp.grid_unitsquare(N))
+    pde = grmp.PoissonProblem(1.0)
+    pde.add_rhsdata(0, grmp.LinearForm(grmp.Identity, grmp.DataFunction([1.0])))
+    pde.add_boundarydata(0)
+    sol = grmp.FEVector([fes])
+    A, b, fixed = grmp.assemble(pde, sol)
+    M = grmp.MultigridSolver(*grmp.mg_hierarchy(pde, fes, A))
+    i0 = M.solve(b, sol, 1e-8)
+    assert i0.status == 0 and i0.relres <= 0.4e-8
+    rtol = 1.5 * i0.relres  # met by the residual of i0, its margin is not
+    i1 = M.solve(b, sol, rtol)
+    assert i1.status == 0 and i1.iterations == i0.iterations + 1 and i1.relres <= 0.4 * rtol
+    i2 = M.solve(b, sol, rtol, maxit=i0.iterations)
+    assert i2.status == 0 and i2.iterations == i0.iterations and i2.relres <= rtol
+    with pytest.raises(grmp.GrmpError) as e:
+        M.solve(b, sol, rtol, maxit=i0.iterations - 1)
+    assert e.value.code == grmp._abi.ERR_NOCONV
