@@ -196,16 +196,24 @@ static void pool_trim(grmp_ctx *ctx, hipStream_t st)
     if (pool || hipDeviceGetDefaultMemPool(&pool, ctx->device) == hipSuccess) (void)hipMemPoolTrimTo(pool, 0);
 }
 
+// The code is returned; left as the thread's last error, too, it would fail the
+// next launch's check.
+static hipError_t alloc_result(hipError_t e)
+{
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
+
 hipError_t ctx_malloc(grmp_ctx *ctx, void **p, size_t bytes, hipStream_t st)
 {
-    return alloc_or_release(
+    return alloc_result(alloc_or_release(
         [&] { return ctx->pool ? hipMallocFromPoolAsync(p, bytes, ctx->pool, st) : hipMallocAsync(p, bytes, st); },
-        [&] { pool_trim(ctx, st); });
+        [&] { pool_trim(ctx, st); }));
 }
 
 hipError_t ctx_malloc_fixed(grmp_ctx *ctx, void **p, size_t bytes)
 {
-    return alloc_or_release([&] { return hipMalloc(p, bytes); }, [&] { pool_trim(ctx, ctx->stream); });
+    return alloc_result(alloc_or_release([&] { return hipMalloc(p, bytes); }, [&] { pool_trim(ctx, ctx->stream); }));
 }
 
 int ctx_pin(grmp_ctx *ctx)

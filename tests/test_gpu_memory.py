@@ -125,3 +125,26 @@ def test_multigrid_buffer_is_within_its_account(grmp, kind, fe, N):
                            2048, 2048)
     assert 0 < taken <= bound <= reserve, (taken, bound, reserve)
     assert reserve >= 2 * grmp.server.footprint(kind, fe, N)
+
+
+def test_out_of_memory_gives_free_blocks_back(grmp):
+    """A vector larger than the device fails with the library's code after the
+    free blocks were given back for it, and the context works on."""
+    print("[case] a vector larger than the device", flush=True)
+    size = 256 << 20
+    gc.collect()
+    ctx = grmp._abi.Context(0)
+    v = grmp.DeviceVector(ctx, size // 8)
+    del v
+    gc.collect()
+    assert _usage(grmp, ctx)[1] >= size
+    with pytest.raises(grmp.GrmpError) as e:
+        grmp.DeviceVector(ctx, 1 << 40)
+    assert e.value.code == grmp._abi.ERR_OOM
+    used, held = _usage(grmp, ctx)
+    assert held - used < size
+    w = grmp.DeviceVector(ctx, 1000)
+    w.fill(2.0)
+    assert (w.download() == 2.0).all()
+    del w
+    ctx.close()
